@@ -1550,6 +1550,21 @@ __global__ __launch_bounds__(256) void k_gather_plain(
   out[m] = make_float2(ar, ai);
 }
 
+// Scatter of one coil.  The L2 serves float atomics per 64-byte line request
+// (about 21 G requests/s), and lanes of one instruction on one line share its
+// request: with a thread per sample every tap cost two requests of its own.
+// Here SP_LANES lanes hold one sample, two per x tap (real, imaginary), so a
+// row of taps -- up to 64 contiguous bytes for 8 taps -- is one instruction
+// and one or two requests.  96^3, 393216 radial samples, W = 5, A then A^H:
+// 5.60 ms in the scatter before, 1.3 now (the pair 5.90 -> 1.62 ms).
+// Each lane evaluates one z, one y and one x weight; rows get theirs from the
+// sample's lanes.  Per tap the value is ((wz wy) wx) v, as in a loop over the
+// taps; only the order of the atomics differs.  A workgroup takes samples
+// until none is left (SP_BLOCKS workgroups at most), so that the kernel
+// tables are loaded into LDS once for many samples.
+#define SP_LANES 16
+#define SP_BLOCKS 2048
+static_assert(SP_LANES == 2 * MRN_MAXT, "two lanes per x tap");
 __global__ __launch_bounds__(256) void k_scatter_plain(
     float2 *__restrict__ grid, const float2 *__restrict__ data, const float *__restrict__ kx,
     const float *__restrict__ ky, const float *__restrict__ kz, const float *__restrict__ kw,
@@ -1557,37 +1572,65 @@ __global__ __launch_bounds__(256) void k_scatter_plain(
   extern __shared__ float tab_s[];
   load_tables(tab_s, tables, g.ntab);
   __syncthreads();
-  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= M) return;
-  const float w = kw[m];
-  if (w == 0.0f) return;
-  const float2 d = data[m];
-  float vr = d.x * w, vi = d.y * w;
-  if (vr == 0.f && vi == 0.f) return;
-  const float k[3] = {kx[m], ky[m], kz[m]};
-  float dk[3];
-  int s[3], e[3];
+  const int j = threadIdx.x & (SP_LANES - 1);  // lane of the sample
+  const int tap = j >> 1, part = j & 1;        // x tap, real or imaginary
+  const int64_t step = (int64_t)gridDim.x * (256 / SP_LANES);
+  for (int64_t m0 = (int64_t)blockIdx.x * (256 / SP_LANES); m0 < M; m0 += step) {
+    const int64_t m = m0 + threadIdx.x / SP_LANES;
+    // every lane stays for the shuffles; a sample without taps has no rows
+    bool live = m < M;
+    const float w = live ? kw[m] : 0.0f;
+    const float2 d = live ? data[m] : make_float2(0.f, 0.f);
+    float vr = d.x * w, vi = d.y * w;
+    live = live && w != 0.0f && !(vr == 0.f && vi == 0.f);
+    float k[3] = {0.f, 0.f, 0.f};
+    if (live) {
+      k[0] = kx[m];
+      k[1] = ky[m];
+      k[2] = kz[m];
+    }
+    float dk[3];
+    int s[3], e[3];
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
-    dk[a] = grid_coord(g, a, k[a]);
-    if (!axis_range(g, a, dk[a], s[a], e[a])) return;
-  }
-  float kr = 0.f;
+    for (int a = 0; a < 3; a++) {
+      dk[a] = grid_coord(g, a, k[a]);
+      live = axis_range(g, a, dk[a], s[a], e[a]) && live;
+    }
+    float wa[3] = {0.f, 0.f, 0.f};  // this lane's weights: tap `tap` of x, tap j of y and z
+    float v = 0.f;
+    if (live) {
+      float kr = 0.f;
 #pragma unroll
-  for (int a = 0; a < 3; a++)
-    if (g.fft_in[a]) kr += k[a] * k[a];
-  const float tp = (float)exp(-(double)kr / (2.0 * (double)g.k_rad * (double)g.k_rad));
-  vr *= tp;
-  vi *= tp;
-  for (int lz = s[2]; lz <= e[2]; lz++) {
-    const float wz = tap_weight(g, 2, tab_s + g.toff[2], dk[2], lz);
-    for (int ly = s[1]; ly <= e[1]; ly++) {
-      const float wzy = wz * tap_weight(g, 1, tab_s + g.toff[1], dk[1], ly);
-      float2 *row = grid + ((int64_t)lz * g.S[1] + ly) * g.S[0];
-      for (int lx = s[0]; lx <= e[0]; lx++) {
-        const float ww = wzy * tap_weight(g, 0, tab_s + g.toff[0], dk[0], lx);
-        atomicAdd(&row[lx].x, ww * vr);
-        atomicAdd(&row[lx].y, ww * vi);
+      for (int a = 0; a < 3; a++)
+        if (g.fft_in[a]) kr += k[a] * k[a];
+      const float tp = (float)exp(-(double)kr / (2.0 * (double)g.k_rad * (double)g.k_rad));
+      vr *= tp;
+      vi *= tp;
+      v = part ? vi : vr;
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        const int l = s[a] + (a == 0 ? tap : j);
+        if (l <= e[a]) wa[a] = tap_weight(g, a, tab_s + g.toff[a], dk[a], l);
+      }
+    }
+    const int ny = live ? e[1] - s[1] + 1 : 0, nz = live ? e[2] - s[2] + 1 : 0;
+    const bool in = live && s[0] + tap <= e[0];
+    // rows of the wavefront's samples: up to MRN_MAXT taps per axis,
+    // every lane in step (the shuffles need the sample's 16 lanes)
+    int nzw = nz, nyw = ny;
+#pragma unroll
+    for (int o = 32; o >= SP_LANES; o >>= 1) {
+      nzw = max(nzw, __shfl_xor(nzw, o));
+      nyw = max(nyw, __shfl_xor(nyw, o));
+    }
+    for (int z = 0; z < nzw; z++) {
+      const float wz = __shfl(wa[2], z, SP_LANES);
+      for (int y = 0; y < nyw; y++) {
+        const float wzy = wz * __shfl(wa[1], y, SP_LANES);
+        if (in && z < nz && y < ny) {
+          float2 *row = grid + ((int64_t)(s[2] + z) * g.S[1] + (s[1] + y)) * g.S[0] + s[0];
+          atomicAdd(reinterpret_cast<float *>(row) + j, (wzy * wa[0]) * v);
+        }
       }
     }
   }
@@ -1874,7 +1917,8 @@ int launch_scatter_plain(mrn_op *op, float2 *grid, const float2 *data, int64_t M
   Geom g = op->g;
   g.CC = 1;
   g.lgCC = 0;
-  hipLaunchKernelGGL(k_scatter_plain, dim3(nblk(M, 256)), dim3(256), sizeof(float) * g.ntab, st,
+  const unsigned nb = nblk(M, 256 / SP_LANES);
+  hipLaunchKernelGGL(k_scatter_plain, dim3(nb < SP_BLOCKS ? nb : SP_BLOCKS), dim3(256), sizeof(float) * g.ntab, st,
                      grid, data, kx, ky, kz, kw, M, g, op->tables_d);
   MRN_HIP(op, hipGetLastError());
   return MRN_OK;
