@@ -264,8 +264,8 @@ int mrn_get_tuning(const mrn_op *op, mrn_tuning *out);
 
 /* Average device time (ms, HIP events on `stream`) of each batched stage of
  * one frame over `reps` runs: [0] set_image+z FFT, [1] y FFT, [2] x FFT,
- * [3] gather (with the k-space weighting of E'E), [4] zeroing of the tiles
- * that several scatter work items share, [5] tile scatter, [6] x IFFT,
+ * [3] gather (with the k-space weighting of E'E), [4] nothing (0; kept for
+ * the layout), [5] scatter (tiles, split tiles' sums, window edges), [6] x IFFT,
  * [7] y IFFT, [8] z IFFT+accumulate.  Each stage is one kernel per coil block
  * or one kernel over all blocks.  Diagnostic; no counterpart in the reference
  * (its -time_grid prints, gridFFT.cpp:727-747, time the same stages on the
@@ -281,9 +281,9 @@ typedef struct mrn_frame_stats {
   int64_t valid;           /* samples with kw != 0 inside the grid */
   int64_t tile_visits;     /* sample visits over the scatter's 4^3 tiles */
   int64_t scatter_atomics; /* float atomics of one scatter over all coils, upper bound
-                              (split tiles' flushes and window-edge samples; zero sums skip theirs) */
+                              (window-edge samples; the tiles are written with plain stores) */
   int32_t scatter_items;   /* scatter work items */
-  int32_t split_items;     /* work items of tiles split over several items (flushed with atomics) */
+  int32_t split_items;     /* work items of tiles split over several items (summed in order) */
   int32_t split_tiles;     /* tiles split over several work items */
   int32_t wide;            /* samples with one tap more than usual on some axis */
   int32_t gather_items;    /* tile-staged gather work items */

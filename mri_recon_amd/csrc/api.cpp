@@ -188,6 +188,9 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
     MRN_HIP(op, hipMalloc(&op->kwork_all, sizeof(float2) * (tot > 0 ? tot : 1)));
     op->kwork_all_cap = tot;
   }
+  int64_t ptot = 0;
+  for (int f = 0; f < F; f++) ptot += (int64_t)op->frames[f].nslots * op->nch * 64 * g.CC;
+  MRN_HIP(op, grow(op->part_all, op->part_all_cap, ptot));
   if (!op->fdev) MRN_HIP(op, hipMalloc(&op->fdev, sizeof(FrameDev) * F));
   const int64_t nrow = (int64_t)g.S[1] * g.S[2];
   if (fft_x_pruned(op)) {
@@ -203,7 +206,7 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
                                  hipMemcpyDeviceToDevice, st));
   }
   std::vector<FrameDev> h(F);
-  int64_t off = 0;
+  int64_t off = 0, poff = 0;
   op->fmax_nsub = op->fmax_nheavy = op->fmax_nwide = op->fmax_xsplit = 0;
   op->fmax_Mv = 0;
   for (int f = 0; f < F; f++) {
@@ -217,6 +220,8 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
     d.heavy = fr.heavy;
     d.wide = fr.wide;
     d.xsplit = fr.xsplit;
+    d.part = op->part_all + poff;
+    poff += (int64_t)fr.nslots * op->nch * 64 * g.CC;
     d.kwork = op->kwork_all + off;
     d.kdata = fr.kdata;
     d.Mv = fr.Mv;
@@ -964,9 +969,8 @@ int mrn_stage_times(mrn_op *op, int f, const void *Xv, int reps, float ms[MRN_NS
     }
     MRN_TRY(launch_gather(op, op->grid, op->kwork, fr, nullptr, true, st));
     MRN_HIP(op, hipEventRecord(ev[e++], st));
-    MRN_TRY(launch_scatter_zero(op, op->grid, fr, st));
-    MRN_HIP(op, hipEventRecord(ev[e++], st));
-    MRN_TRY(launch_scatter_tiles(op, op->grid, op->kwork, fr, st));
+    MRN_HIP(op, hipEventRecord(ev[e++], st));  // the stage between held the split tiles' zeroing
+    MRN_TRY(launch_scatter(op, op->grid, op->kwork, fr, st));
     MRN_HIP(op, hipEventRecord(ev[e++], st));
     for (int q = 0; q < 3; q++) {
       MRN_TRY(adj_stage(op, q, op->vX0, true, &fr, st));
@@ -1003,11 +1007,10 @@ int mrn_get_frame_stats(mrn_op *op, int f, mrn_frame_stats *out) {
       if (w.w) out->split_items++;
     }
   }
-  // a split tile's items each add 64 cells x 2 CC reals; a wide sample adds at
-  // most NT^3 taps x 2 CC reals; per coil block
+  // a wide sample adds at most NT^3 taps x 2 CC reals; per coil block
   const int64_t per_cell = 2 * (int64_t)op->g.CC;
   const int64_t nt3 = (int64_t)op->t.NT * op->t.NT * op->t.NT;
-  out->scatter_atomics = (out->split_items * 64 * per_cell + (int64_t)fr.nwide * nt3 * per_cell) * op->nch;
+  out->scatter_atomics = (int64_t)fr.nwide * nt3 * per_cell * op->nch;
   return MRN_OK;
 }
 

@@ -14,8 +14,8 @@
 // of the bins that can reach the tile (wave-uniform loads) and every lane adds
 // its own tap.  No atomics on this path (LDS float atomics run at about 3 cycles
 // per lane on gfx950); a tile is written once with plain stores.  Tiles whose
-// sample list exceeds one work item are split; only those are pre-zeroed and
-// flushed with global atomics.
+// sample list exceeds one work item are split; their items' sums go to slots
+// of their own, added up in order afterwards.
 #include <hipcub/hipcub.hpp>
 
 #include <climits>
@@ -125,8 +125,9 @@ __host__ __device__ __forceinline__ void tile_bins(const Tiles &t, int a, int ti
 
 // xrng (null: every tile): a tile without samples gets no work item when no
 // row's k-space support reaches its cells -- the inverse x pass never reads them
+// slots: the tile's partial-sum slots, one per work item of a split tile.
 __global__ void k_tile_nsub(const int32_t *__restrict__ bin_start, Tiles t, int32_t *nsub,
-                            int32_t *visits, const int2 *__restrict__ xrng, int S1, int S2) {
+                            int32_t *visits, int32_t *slots, const int2 *__restrict__ xrng, int S1, int S2) {
   int tile = blockIdx.x * blockDim.x + threadIdx.x;
   if (tile >= t.ntiles) return;
   const int tx = tile % t.nt[0], ty = (tile / t.nt[0]) % t.nt[1], tz = tile / (t.nt[0] * t.nt[1]);
@@ -147,17 +148,27 @@ __global__ void k_tile_nsub(const int32_t *__restrict__ bin_start, Tiles t, int3
       const int2 rr = xrng[(int64_t)z * S1 + y];
       needed = rr.x <= tx * t.T + t.T - 1 && rr.y >= tx * t.T;
     }
-  nsub[tile] = v > t.maxv ? (v + t.maxv - 1) / t.maxv : (needed ? 1 : 0);
+  const int n = v > t.maxv ? (int)(((int64_t)v + t.maxv - 1) / t.maxv) : (needed ? 1 : 0);
+  nsub[tile] = n;
+  slots[tile] = n > 1 ? n : 0;
 }
 
 __global__ void k_fill_subs(const int32_t *__restrict__ nsub, const int32_t *__restrict__ off,
-                            const int32_t *__restrict__ visits, Tiles t, int4 *subs,
-                            int32_t *heavy_flag) {
+                            const int32_t *__restrict__ visits, const int32_t *__restrict__ slot0, Tiles t,
+                            int4 *subs, int32_t *heavy_flag) {
   int tile = blockIdx.x * blockDim.x + threadIdx.x;
   if (tile >= t.ntiles) return;
   const int n = nsub[tile], o = off[tile], v = visits[tile];
-  for (int s = 0; s < n; s++) subs[o + s] = make_int4(tile, s * t.maxv, min((s + 1) * t.maxv, v), n > 1);
+  for (int s = 0; s < n; s++)
+    subs[o + s] = make_int4(tile, s * t.maxv, s + 1 < n ? (s + 1) * t.maxv : v, n > 1 ? slot0[tile] + s + 1 : 0);
   heavy_flag[tile] = n > 1;
+}
+
+// the split tiles {tile, first slot, slots}
+__global__ void k_heavy_tiles(const int32_t *__restrict__ flag, const int32_t *__restrict__ off,
+                              const int32_t *__restrict__ nsub, const int32_t *__restrict__ slot0, int n, int4 *out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n && flag[i]) out[off[i]] = make_int4(i, slot0[i], nsub[i], 0);
 }
 
 // Visit counts widened for the offsets' scan (entry ntiles: 0).
@@ -273,12 +284,6 @@ __global__ void k_gtile_fill(const int32_t *__restrict__ nsub, const int32_t *__
   if (tile >= t.ntiles) return;
   const int n = nsub[tile], o = off[tile], v = count[tile];
   for (int q = 0; q < n; q++) gsubs[o + q] = make_int4(tile, q * per, min((q + 1) * per, v), 0);
-}
-
-__global__ void k_compact(const int32_t *__restrict__ flag, const int32_t *__restrict__ off, int n,
-                          int32_t *out) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && flag[i]) out[off[i]] = i;
 }
 
 // ------------------------------------------------------------ gather
@@ -1058,25 +1063,55 @@ static size_t gather_mm_lds(int nt) {
 }
 
 // ------------------------------------------------------------ scatter
-__global__ void k_zero_tiles(float2 *grid, const int32_t *__restrict__ tiles, Geom g, Tiles t,
-                             int64_t chunk_grid, const FrameDev *__restrict__ fdt) {
-  if (fdt) {  // every frame at once: frame blockIdx.z
-    const FrameDev &fd = fdt[blockIdx.z];
+// Sum of the split tiles' partial sums: work item i of a split tile leaves
+// its 64 cells x CC coils in slot first + i, and here one thread per cell and
+// coil adds the tile's slots in order and stores the cell (or adds to it).
+// The result does not depend on the order in which the work items ran.
+#define ST_UNROLL 8
+__global__ __launch_bounds__(256) void k_sum_tiles(float2 *grid, const float2 *__restrict__ part,
+                                                   const int4 *__restrict__ tiles, Geom g, Tiles t, int nch,
+                                                   int64_t chunk_grid, int accum, const FrameDev *__restrict__ fdt) {
+  if (fdt) {  // every frame at once: frame blockIdx.z / nch
+    const FrameDev &fd = fdt[blockIdx.z / nch];
     if ((int)blockIdx.x >= fd.nheavy) return;
     grid += fd.grid_off;
     tiles = fd.heavy;
+    part = fd.part;
   }
-  const int tile = tiles[blockIdx.x];
-  const int ch = blockIdx.y;
-  const int tx0 = (tile % t.nt[0]) * t.T, ty0 = ((tile / t.nt[0]) % t.nt[1]) * t.T,
-            tz0 = (tile / (t.nt[0] * t.nt[1])) * t.T;
-  const int ncell = t.T * t.T * t.T * g.CC;
-  for (int idx = threadIdx.x; idx < ncell; idx += blockDim.x) {
-    const int cell = idx >> g.lgCC, c = idx & (g.CC - 1);
-    const int x = tx0 + cell % t.T, y = ty0 + (cell / t.T) % t.T, z = tz0 + cell / (t.T * t.T);
-    if (x < g.S[0] && y < g.S[1] && z < g.S[2])
-      grid[ch * chunk_grid + (((int64_t)z * g.S[1] + y) * g.S[0] + x) * g.CC + c] = make_float2(0.f, 0.f);
+  const int4 w = tiles[blockIdx.x];
+  const int ch = blockIdx.z % nch;
+  const int idx = blockIdx.y * blockDim.x + threadIdx.x;
+  const int per = 64 << g.lgCC;
+  if (idx >= per) return;
+  const int cell = idx >> g.lgCC, c = idx & (g.CC - 1);
+  const int x = (w.x % t.nt[0]) * 4 + (cell & 3), y = ((w.x / t.nt[0]) % t.nt[1]) * 4 + ((cell >> 2) & 3),
+            z = (w.x / (t.nt[0] * t.nt[1])) * 4 + (cell >> 4);
+  if (x >= g.S[0] || y >= g.S[1] || z >= g.S[2]) return;
+  const float2 *p = part + ((int64_t)w.y * nch + ch) * per + idx;
+  const int64_t step = (int64_t)nch * per;
+  float2 a = make_float2(0.f, 0.f);
+  int i = 0;
+  for (; i + ST_UNROLL <= w.z; i += ST_UNROLL, p += ST_UNROLL * step) {
+    float2 v[ST_UNROLL];
+#pragma unroll
+    for (int q = 0; q < ST_UNROLL; q++) v[q] = p[q * step];
+#pragma unroll
+    for (int q = 0; q < ST_UNROLL; q++) {
+      a.x += v[q].x;
+      a.y += v[q].y;
+    }
   }
+  for (; i < w.z; i++, p += step) {
+    a.x += p->x;
+    a.y += p->y;
+  }
+  float2 *dst = grid + ch * chunk_grid + ((((int64_t)z * g.S[1] + y) * g.S[0] + x) << g.lgCC) + c;
+  if (accum) {
+    const float2 o = *dst;
+    a.x += o.x;
+    a.y += o.y;
+  }
+  *dst = a;
 }
 
 // Grid-driven scatter on the matrix cores (8- and 16-coil blocks).  A
@@ -1099,8 +1134,8 @@ __global__ void k_zero_tiles(float2 *grid, const int32_t *__restrict__ tiles, Ge
 // one bin row, so most groups skip a plane or two.  Locating and weighting a
 // sample takes two lanes, not a whole quad per tile offset, and not 64 lanes
 // per cell.  Sums are FP32; only the order of the additions differs from a
-// per-sample loop.  Each tile is written once with plain stores (atomics
-// for a tile split over several work items).
+// per-sample loop.  Each tile is written once with plain stores; a tile split
+// over several work items goes to its items' slots, which k_sum_tiles adds.
 // PAIR (8-coil blocks): a work item takes coil blocks 2 y and 2 y + 1 as its
 // two 16-real blocks, so step A's weights serve both (the second is skipped
 // when nch is odd and y is the last pair).
@@ -1110,7 +1145,7 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
     float2 *__restrict__ grid, const float2 *__restrict__ kin, const float4 *__restrict__ coords,
     const int64_t *__restrict__ vofs, const int32_t *__restrict__ vlist, const int4 *__restrict__ subs, int nsub,
     Geom g, Tiles t, const float *__restrict__ tables, int64_t chunk_grid, int64_t chunk_k, int accum,
-    const FrameDev *__restrict__ fdt, const int32_t *__restrict__ xs, int nch) {
+    const FrameDev *__restrict__ fdt, const int32_t *__restrict__ xs, int nch, float2 *__restrict__ part) {
   static_assert(CCT == 8 || CCT == 16, "matrix-core scatter needs 8 or 16 coils per cell");
   static_assert(!PAIR || CCT == 8, "coil blocks are paired only at 8 coils");
   constexpr int NB = PAIR ? 2 : CCT / 8;  // 16-real blocks of a cell's coil values (or the pair's blocks)
@@ -1134,6 +1169,7 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
     nsub = fd.nsub;
     chunk_k = fd.Mv * g.CC;
     xs = fd.xsplit;
+    part = fd.part;
   }
   const int sidx = scatter_item(blockIdx.x, gridDim.x, wave, t.xrun, xs);
   if (sidx < 0 || sidx >= nsub) return;
@@ -1269,16 +1305,17 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
     for (int r = 0; r < 4; r++) {
       const int cx = t0[0] + r, cy = t0[1] + kq, cz = t0[2] + p;
       if (cx >= g.S[0] || cy >= g.S[1] || cz >= g.S[2]) continue;
-      float *dst = reinterpret_cast<float *>(grid + ch * chunk_grid +
-                                             (((int64_t)cz * g.S[1] + cy) * g.S[0] + cx) * CCT) + ci;
+      // a split tile's item writes its slot, [nch][64 cells][CCT]
+      const int64_t cell = sp.w ? (((int64_t)(sp.w - 1) * nch + ch) * 64 + 16 * p + 4 * kq + r) * CCT
+                                : ch * chunk_grid + (((int64_t)cz * g.S[1] + cy) * g.S[0] + cx) * CCT;
+      const int64_t next = sp.w ? 64 * CCT : chunk_grid;  // PAIR: the second block's cell
+      float *dst = reinterpret_cast<float *>((sp.w ? part : grid) + cell) + ci;
 #pragma unroll
       for (int nb = 0; nb < NB; nb++) {
         if (nb > 0 && !have1) continue;
         const float v = acc[p][nb][r];
-        float *d = PAIR ? dst + nb * 2 * chunk_grid : dst + 16 * nb;
-        if (sp.w) {
-          if (v != 0.f) atomicAdd(d, v);
-        } else if (accum) {  // the tile's only work item: a plain read-modify-write
+        float *d = PAIR ? dst + nb * 2 * next : dst + 16 * nb;
+        if (accum && !sp.w) {  // the tile's only work item: a plain read-modify-write
           *d += v;
         } else {
           *d = v;
@@ -1309,7 +1346,7 @@ __global__ __launch_bounds__(256, 6) void k_scatter_gd(
     float2 *__restrict__ grid, const float2 *__restrict__ kin, const float4 *__restrict__ coords,
     const int64_t *__restrict__ vofs, const int32_t *__restrict__ vlist, const int4 *__restrict__ subs, int nsub,
     Geom g, Tiles t, const float *__restrict__ tables, int64_t chunk_grid, int64_t chunk_k, int accum,
-    const FrameDev *__restrict__ fdt, const int32_t *__restrict__ xs) {
+    const FrameDev *__restrict__ fdt, const int32_t *__restrict__ xs, int nch, float2 *__restrict__ part) {
   __shared__ float s_w[4][SG_BATCH * 12];    // [sample][axis][offset] weights
   __shared__ float2 s_d[4][SG_BATCH * CCT];  // [sample][coil] data
   extern __shared__ float tab_s[];           // kernel tables (g.ntab floats)
@@ -1328,6 +1365,7 @@ __global__ __launch_bounds__(256, 6) void k_scatter_gd(
     nsub = fd.nsub;
     chunk_k = fd.Mv * g.CC;
     xs = fd.xsplit;
+    part = fd.part;
   }
   const int sidx = scatter_item(blockIdx.x, gridDim.x, wave, t.xrun, xs);
   if (sidx < 0 || sidx >= nsub) return;
@@ -1404,14 +1442,9 @@ __global__ __launch_bounds__(256, 6) void k_scatter_gd(
   }
   const int cx = t0[0] + lx, cy = t0[1] + ly, cz = t0[2] + lz;
   if (cx >= g.S[0] || cy >= g.S[1] || cz >= g.S[2]) return;
-  float2 *dst = grid + ch * chunk_grid + (((int64_t)cz * g.S[1] + cy) * g.S[0] + cx) * CCT;
-  if (sp.w) {
-#pragma unroll
-    for (int c = 0; c < CCT; c++) {
-      if (ar[c] != 0.f) atomicAdd(&dst[c].x, ar[c]);
-      if (ai[c] != 0.f) atomicAdd(&dst[c].y, ai[c]);
-    }
-  } else if (accum) {
+  float2 *dst = sp.w ? part + (((int64_t)(sp.w - 1) * nch + ch) * 64 + lane) * CCT  // a split tile's slot
+                     : grid + ch * chunk_grid + (((int64_t)cz * g.S[1] + cy) * g.S[0] + cx) * CCT;
+  if (accum && !sp.w) {
 #pragma unroll
     for (int c = 0; c < CCT; c++) {
       const float2 o = dst[c];
@@ -1797,23 +1830,22 @@ int launch_gather_frames(mrn_op *op, int fsub, hipStream_t st) {
   return launch_gather_direct(op, op->grid, nullptr, op->frames[0], nullptr, 1, nullptr, 0, st, op->fdev, fsub);
 }
 
-// Zero the tiles that several work items flush with atomics (part of the scatter).
-int launch_scatter_zero(mrn_op *op, float2 *grid, const mrn::FrameData &fr, hipStream_t st,
-                        const FrameDev *fdt) {
+// The split tiles from their work items' partial sums (after the tile scatter).
+int launch_scatter_sum(mrn_op *op, float2 *grid, const mrn::FrameData &fr, hipStream_t st, bool accum,
+                       const FrameDev *fdt) {
   const Geom &g = op->g;
   const int nh = fdt ? op->fmax_nheavy : fr.nheavy;
   if (nh > 0) {
     const int64_t cg = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC;
-    hipLaunchKernelGGL(k_zero_tiles, dim3(nh, op->nch, fdt ? op->F : 1), dim3(256), 0, st, grid, fr.heavy, g,
-                       op->t, cg, fdt);
+    hipLaunchKernelGGL(k_sum_tiles, dim3(nh, nblk(64 * g.CC, 256), op->nch * (fdt ? op->F : 1)), dim3(256), 0, st, grid,
+                       op->part, fr.heavy, g, op->t, op->nch, cg, accum ? 1 : 0, fdt);
     MRN_HIP(op, hipGetLastError());
   }
   return MRN_OK;
 }
 
-// The tile scatter proper; launch_scatter_zero must precede it unless
-// accum (add into the grid's contents: tiles split over several work items
-// add with atomics, the others read, add and store).
+// The tile scatter proper: every tile but the split ones is written (accum:
+// read, added to and stored); launch_scatter_sum and launch_scatter_wide follow.
 int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn::FrameData &fr,
                          hipStream_t st, bool accum, const FrameDev *fdt) {
   const int af = accum ? 1 : 0;
@@ -1821,7 +1853,7 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
   const Tiles &t = op->t;
   // fdt: every frame at once (grid dimension z = frame; the frames' largest
   // work lists size the grid, each frame's kernel reads its own)
-  const int nsub = fdt ? op->fmax_nsub : fr.nsub, nwide = fdt ? op->fmax_nwide : fr.nwide;
+  const int nsub = fdt ? op->fmax_nsub : fr.nsub;
   const int64_t Mv = fdt ? op->fmax_Mv : fr.Mv;
   int64_t cg = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC, ck = fr.Mv * g.CC;
   // per-XCD ranges (xcd_run < 0): MRN_XCDS workgroup columns, each as long
@@ -1844,7 +1876,7 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
     if (pair) gm.y = (unsigned)((op->nch + 1) / 2);
 #define MRN_MM(n, km, pr)                                                                                \
   hipLaunchKernelGGL((k_scatter_mm<n, km, pr>), gm, dim3(256), sh, st, grid, kin, fr.coords, fr.vofs,   \
-                     fr.vlist, fr.subs, fr.nsub, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit, op->nch)
+                     fr.vlist, fr.subs, fr.nsub, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit, op->nch, op->part)
     if (g.CC == 16 && !exact) MRN_MM(16, 0, false);
     else if (g.CC == 16) MRN_MM(16, 1, false);
     else if (pair && !exact) MRN_MM(8, 0, true);
@@ -1857,7 +1889,7 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
 #define MRN_S(n)                                                                                 \
   case n:                                                                                        \
     hipLaunchKernelGGL((k_scatter_gd<n>), g3, dim3(256), sh, st, grid, kin, fr.coords, fr.vofs,  \
-                       fr.vlist, fr.subs, fr.nsub, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit);   \
+                       fr.vlist, fr.subs, fr.nsub, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit, op->nch, op->part); \
     break;
     MRN_S(1) MRN_S(2) MRN_S(4) MRN_S(8) MRN_S(16)
 #undef MRN_S
@@ -1866,9 +1898,18 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
     }
   }
   MRN_HIP(op, hipGetLastError());
-  if (nwide > 0) {  // after the tiles' plain stores
+  return MRN_OK;
+}
+
+// The window-edge taps (k_scatter_wide), after the tiles' plain stores.
+int launch_scatter_wide(mrn_op *op, float2 *grid, const float2 *kin, const mrn::FrameData &fr, hipStream_t st,
+                        const FrameDev *fdt) {
+  const Geom &g = op->g;
+  const int nwide = fdt ? op->fmax_nwide : fr.nwide;
+  if (nwide > 0) {
+    const int64_t cg = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC, ck = fr.Mv * g.CC;
     hipLaunchKernelGGL(k_scatter_wide, dim3(nblk((int64_t)nwide * g.CC, 256), op->nch, fdt ? op->F : 1), dim3(256), 0,
-                       st, grid, kin, fr.coords, fr.wide, fr.nwide, g, t.NTb, op->tables_d, cg, ck, fdt);
+                       st, grid, kin, fr.coords, fr.wide, fr.nwide, g, op->t.NTb, op->tables_d, cg, ck, fdt);
     MRN_HIP(op, hipGetLastError());
   }
   return MRN_OK;
@@ -1876,14 +1917,17 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
 
 int launch_scatter(mrn_op *op, float2 *grid, const float2 *kin, const mrn::FrameData &fr,
                    hipStream_t st, bool accum) {
-  if (!accum) MRN_TRY(launch_scatter_zero(op, grid, fr, st));
-  return launch_scatter_tiles(op, grid, kin, fr, st, accum);
+  MRN_TRY(launch_scatter_tiles(op, grid, kin, fr, st, accum));
+  MRN_TRY(launch_scatter_sum(op, grid, fr, st, accum));
+  return launch_scatter_wide(op, grid, kin, fr, st);
 }
 
 // Scatter of every frame at once, from their kwork arrays into their grids.
 int launch_scatter_frames(mrn_op *op, hipStream_t st) {
-  MRN_TRY(launch_scatter_zero(op, op->grid, op->frames[0], st, op->fdev));
-  return launch_scatter_tiles(op, op->grid, nullptr, op->frames[0], st, false, op->fdev);
+  const mrn::FrameData &fr = op->frames[0];
+  MRN_TRY(launch_scatter_tiles(op, op->grid, nullptr, fr, st, false, op->fdev));
+  MRN_TRY(launch_scatter_sum(op, op->grid, fr, st, false, op->fdev));
+  return launch_scatter_wide(op, op->grid, nullptr, fr, st, op->fdev);
 }
 
 int launch_weight(mrn_op *op, float2 *kout, const float2 *kin, const mrn::FrameData &fr,
@@ -2023,6 +2067,24 @@ __global__ void k_xcd_split(const int64_t *__restrict__ pre, int n, int32_t *xs)
   xs[x] = lo;
 }
 
+// Visits per scatter work item when the caller gave none.  A work item is one
+// wavefront's serial walk (2.4 us per batch of 32 visits), so a dense tile's
+// item must not outlast the rest of the launch; the chip holds about 4096
+// scatter wavefronts.  Hence the frame's visits over 4096, in whole batches:
+// at least 64 (below it the split tiles' atomics cost more than the shorter
+// walks save) and at most 1024 (more gains nothing at 41 M visits).
+// Scatter at 64 / 256 / 1024 / 4096 visits per item: 32^3 x 8 coils, 8192
+// samples 23 / 33 / 74 / 86 us; 128^3 x 8, 262144 samples 180 / 169 / 179 /
+// 338; 100 x 84 x 92 x 8, 303101 samples 211 / 165 / 186 / 346; 160^3 x 24,
+// 768000 samples 1268 / 1028 / 1007 / 1119; 256^3 x 16, 5.12 M samples
+// 4280 / 2217 / 2036 / 2066.
+#define MIN_PART (8ll << 20)  // partial sums always allowed: 8 M values, 64 MB
+static int visits_per_item(const Tiles &t, int64_t Mv) {
+  const double per = (t.NTb + t.T - 1) / (double)t.T;  // tiles a sample reaches, per axis
+  const int64_t v = (int64_t)((double)Mv * per * per * per / 4096.0) / SM_BATCH * SM_BATCH;
+  return (int)std::min<int64_t>(std::max<int64_t>(v, 64), MRN_AUTO_MAXV);
+}
+
 // Sort one frame's samples into tiles and build the scatter work list.  The
 // frame's arrays and the bind's scratch only grow (FrameCaps, BindScratch), so
 // binding a trajectory no larger than the last one allocates nothing; the
@@ -2031,7 +2093,7 @@ __global__ void k_xcd_split(const int64_t *__restrict__ pre, int n, int32_t *xs)
 int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const float *ky,
                const float *kz, const float *kw, hipStream_t st) {
   const Geom &g = op->g;
-  const Tiles &t = op->t;
+  Tiles t = op->t;
   const int nt = t.ntiles, nbin = t.nbins;
   BindScratch &b = op->bind;
   FrameCaps &cp = fr.cap;
@@ -2051,6 +2113,7 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
   fr.nsparse = 0;
   fr.nsub = 0;
   fr.nheavy = 0;
+  fr.nslots = 0;
   fr.M = M;
   MRN_BH(grow(b.keys, b.c_keys, M));
   MRN_BH(grow(b.keys2, b.c_keys2, M));
@@ -2138,6 +2201,7 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
       cp.yrng = 0;
     }
   }
+  if (op->auto_maxv) t.maxv = visits_per_item(t, fr.Mv);
   int32_t *nsub = nullptr, *visits = nullptr, *off = nullptr, *hflag = nullptr, *hoff = nullptr;
   MRN_BH(grow(b.nsub, b.c_nsub, (int64_t)nt + 1));
   MRN_BH(grow(b.visits, b.c_visits, (int64_t)nt + 1));
@@ -2151,9 +2215,43 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
   hoff = b.hoff;
   MRN_BH(hipMemsetAsync(nsub, 0, sizeof(int32_t) * (nt + 1), st));
   MRN_BH(hipMemsetAsync(hflag, 0, sizeof(int32_t) * (nt + 1), st));
-  hipLaunchKernelGGL(k_tile_nsub, dim3(nblk(nt, 256)), dim3(256), 0, st, fr.bin_start, t, nsub, visits,
-                     fft_x_pruned(op) ? fr.xrng : nullptr, g.S[1], g.S[2]);
-  MRN_BH(hipGetLastError());
+  MRN_BH(grow(b.slots, b.c_slots, (int64_t)nt + 1));
+  MRN_BH(grow(b.slot0, b.c_slot0, (int64_t)nt + 1));
+  MRN_BH(hipMemsetAsync(b.slots, 0, sizeof(int32_t) * (nt + 1), st));
+  // work items, with room for the split tiles' partial sums: where that takes
+  // more than a quarter of the grids (or is not to be had) the items are made longer, in the
+  // end one per tile
+  for (;;) {
+    hipLaunchKernelGGL(k_tile_nsub, dim3(nblk(nt, 256)), dim3(256), 0, st, fr.bin_start, t, nsub, visits, b.slots,
+                       fft_x_pruned(op) ? fr.xrng : nullptr, g.S[1], g.S[2]);
+    MRN_BH(hipGetLastError());
+    MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.tmp, tb, b.slots, b.slot0, nt + 1, st));
+    int32_t ns = 0;
+    MRN_BH(hipMemcpyAsync(&ns, b.slot0 + nt, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    MRN_BH(hipStreamSynchronize(st));
+    const int64_t elems = (int64_t)ns * op->nch * 64 * g.CC, cells = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC * op->nch;
+    hipError_t e = hipErrorOutOfMemory;
+    if ((size_t)elems <= op->part_cap) {
+      e = hipSuccess;
+    } else if (elems <= std::max<int64_t>(cells / 4, MIN_PART)) {
+      // the other frames' slots must keep fitting: the old buffer goes only
+      // once the larger one is there
+      float2 *p = nullptr;
+      e = hipMalloc((void **)&p, sizeof(float2) * elems);
+      if (e == hipSuccess) {
+        hipFree(op->part);
+        op->part = p;
+        op->part_cap = (size_t)elems;
+      }
+    }
+    if (e == hipSuccess) {
+      fr.nslots = ns;
+      break;
+    }
+    if (e != hipErrorOutOfMemory || ns == 0) MRN_BH(e);
+    (void)hipGetLastError();
+    t.maxv = t.maxv > (1 << 29) ? INT32_MAX : t.maxv * 2;
+  }
   // visit list (offsets in 64 bits: about 8 visits per sample); it is
   // filled once the work items exist
   int64_t nvisits = 0;
@@ -2177,7 +2275,7 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
   MRN_BH(hipStreamSynchronize(st));
   MRN_BH(grow(fr.subs, cp.subs, nsub_total));
   fr.nsub = nsub_total;
-  hipLaunchKernelGGL(k_fill_subs, dim3(nblk(nt, 256)), dim3(256), 0, st, nsub, off, visits, t,
+  hipLaunchKernelGGL(k_fill_subs, dim3(nblk(nt, 256)), dim3(256), 0, st, nsub, off, visits, b.slot0, t,
                      fr.subs, hflag);
   MRN_BH(hipGetLastError());
   if (nvisits > 0 && nsub_total > 0) {  // the visit list, one wavefront per work item
@@ -2212,7 +2310,7 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
   MRN_BH(grow(fr.heavy, cp.heavy, nh));
   fr.nheavy = nh;
   if (nh > 0) {
-    hipLaunchKernelGGL(k_compact, dim3(nblk(nt, 256)), dim3(256), 0, st, hflag, hoff, nt, fr.heavy);
+    hipLaunchKernelGGL(k_heavy_tiles, dim3(nblk(nt, 256)), dim3(256), 0, st, hflag, hoff, nsub, b.slot0, nt, fr.heavy);
     MRN_BH(hipGetLastError());
   }
   // gather work list (home samples per tile), reusing the scratch arrays

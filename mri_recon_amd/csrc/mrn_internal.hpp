@@ -21,6 +21,7 @@
 #define FFT_LINES 16         // 1-D lines per FFT workgroup
 #define FFT_THREADS 256
 #define FFT_PAD 1            // LDS line padding (float2) against bank conflicts
+#define MRN_AUTO_MAXV 1024   // visits per scatter work item where each frame chooses: the largest
 #define MRN_TRACE_CAP 65536  // solver trace ring (iterations)
 #define MRN_MAX_SPINS 64     // wavelet cycle spins per L1 step
 
@@ -70,9 +71,10 @@ struct FrameDev {
   const int4 *subs;
   const int64_t *vofs;
   const int32_t *vlist;
-  const int32_t *heavy;
+  const int4 *heavy;
   const int32_t *wide;
   const int32_t *xsplit;   // [MRN_XCDS + 1] per-XCD ranges of the scatter work list
+  float2 *part;            // this frame's split tiles' partial sums
   float2 *kwork;           // this frame's [nch][Mv][CC] k-space work array
   const float2 *kdata;     // measured k-space, same layout
   int64_t Mv;
@@ -106,16 +108,16 @@ struct FrameCaps {
 struct BindScratch {
   uint32_t *keys = nullptr, *keys2 = nullptr;
   int32_t *vals = nullptr, *counts = nullptr, *nsub = nullptr, *visits = nullptr, *off = nullptr,
-          *hflag = nullptr, *hoff = nullptr, *wflag = nullptr, *woff = nullptr;
+          *hflag = nullptr, *hoff = nullptr, *wflag = nullptr, *woff = nullptr, *slots = nullptr, *slot0 = nullptr;
   int2 *brow = nullptr;
   int64_t *vw = nullptr, *icost = nullptr, *ipre = nullptr;
   uint8_t *tmp = nullptr, *wtmp = nullptr, *vtmp = nullptr;
   size_t c_keys = 0, c_keys2 = 0, c_vals = 0, c_counts = 0, c_nsub = 0, c_visits = 0, c_off = 0, c_hflag = 0,
          c_hoff = 0, c_wflag = 0, c_woff = 0, c_brow = 0, c_vw = 0, c_icost = 0, c_ipre = 0, c_tmp = 0, c_wtmp = 0,
-         c_vtmp = 0;
+         c_vtmp = 0, c_slots = 0, c_slot0 = 0;
   void release() {
     void *ps[] = {keys, keys2, vals, counts, nsub, visits, off, hflag, hoff, wflag, woff, brow, vw, icost, ipre,
-                  tmp, wtmp, vtmp};
+                  tmp, wtmp, vtmp, slots, slot0};
     for (void *q : ps) hipFree(q);
     *this = BindScratch{};
   }
@@ -130,11 +132,12 @@ struct FrameData {
   int32_t *perm = nullptr;     // [Mv] tile order -> caller index
   int32_t *inv = nullptr;      // [M] caller index -> tile order, -1 if skipped
   int32_t *bin_start = nullptr;// [nbins + 1] first sample of each bin
-  int4 *subs = nullptr;        // [nsub] {tile, first visit, end visit, heavy}
+  int4 *subs = nullptr;        // [nsub] {tile, first visit, end visit, 0 or its partial-sum slot + 1}
   int32_t *xsplit = nullptr;   // [MRN_XCDS + 1] work-list ranges of equal cost, one per XCD
   int xsplit_max = 0;          // longest of those ranges (work items)
-  int32_t *heavy = nullptr;    // [nheavy] tiles split over several work items
+  int4 *heavy = nullptr;       // [nheavy] tiles split over several work items {tile, first slot, slots}
   int nsub = 0, nheavy = 0;
+  int nslots = 0;              // partial-sum slots of those tiles, [nch][64 cells][CC] each
   int64_t *vofs = nullptr;     // [ntiles + 1] first entry of each tile's visits in vlist
   int32_t *vlist = nullptr;    // [vofs[ntiles]] samples of each tile's bin rows, in visit order
   int4 *gsubs = nullptr;       // [ngsub] gather work items {tile, first, end, 0} (home samples)
@@ -175,6 +178,10 @@ struct mrn_op {
   bool fuse = false;
   mrn::FrameDev *fdev = nullptr;  // [F] on the device
   int fdev_version = -1;
+  float2 *part = nullptr;      // split tiles' partial sums of the frame at hand (grow-only, every frame's fit)
+  size_t part_cap = 0;
+  float2 *part_all = nullptr;  // ... of every frame, frame after frame (fused launches)
+  size_t part_all_cap = 0;
   float2 *kwork_all = nullptr; // frames' k-space work arrays, frame after frame
   int64_t kwork_all_cap = 0;   // elements
   int2 *xrng_all = nullptr;    // [F][Sz][Sy] x support rows (k_row_xrange) of every frame
@@ -218,6 +225,7 @@ struct mrn_op {
   void *scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;
   // L1 wavelet proximal step of FISTA (fraction 0 = none)
+  bool auto_maxv = false;      // scatter work items sized per frame (visits_per_item), t.maxv the upper bound
   int gather_tiles = 0;        // dense tiles: 1 = LDS-staged gather, 2 = box matrix-core gather
   bool scatter_valu = false;   // VALU scatter accumulate (else matrix cores for 16-coil blocks)
   bool fft_stockham = false;   // LDS Stockham FFT passes (else four-step where the size allows)
@@ -521,14 +529,16 @@ int taps_main(const Geom &g);
 int launch_gather(mrn_op *op, const float2 *grid, float2 *out, const FrameData &fr, const float2 *sub,
                   bool weighted, hipStream_t st);
 int launch_weight(mrn_op *op, float2 *kout, const float2 *kin, const FrameData &fr, hipStream_t st);
-// the scatter: overwrite the tiles it reaches (zeroing the split tiles first),
-// or with accum add into the grid's contents
+// the scatter: overwrite the tiles it reaches, or with accum add into the
+// grid's contents; its three launches (tiles, split tiles' sums, window edges)
 int launch_scatter(mrn_op *op, float2 *grid, const float2 *kin, const FrameData &fr, hipStream_t st,
                    bool accum = false);
-int launch_scatter_zero(mrn_op *op, float2 *grid, const FrameData &fr, hipStream_t st,
-                        const FrameDev *fdt = nullptr);
 int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const FrameData &fr, hipStream_t st,
                          bool accum = false, const FrameDev *fdt = nullptr);
+int launch_scatter_sum(mrn_op *op, float2 *grid, const FrameData &fr, hipStream_t st, bool accum = false,
+                       const FrameDev *fdt = nullptr);
+int launch_scatter_wide(mrn_op *op, float2 *grid, const float2 *kin, const FrameData &fr, hipStream_t st,
+                        const FrameDev *fdt = nullptr);
 // every frame at once (op->fdev set up): gather from / scatter into the
 // frames' grids, k-space in their kwork arrays
 int launch_gather_frames(mrn_op *op, int fsub, hipStream_t st);

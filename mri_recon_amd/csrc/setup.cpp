@@ -305,7 +305,8 @@ int mrn_op_create(const mrn_params *pin, mrn_op **out) {
   }
   op->t.nbins = op->t.nb[0] * op->t.nb[1] * op->t.nb[2];
   op->t.ntiles = op->t.nt[0] * op->t.nt[1] * op->t.nt[2];
-  op->t.maxv = p.max_visits > 0 ? p.max_visits : 4096;
+  op->t.maxv = p.max_visits > 0 ? p.max_visits : MRN_AUTO_MAXV;
+  op->auto_maxv = p.max_visits <= 0;  // each frame's own, from its sample count
   op->t.xrun = p.xcd_run > 0 ? p.xcd_run : (p.xcd_run < 0 ? -1 : 1);
   op->t.xrun_gather = p.xcd_run_gather > 0 ? p.xcd_run_gather : 64;
   op->gather_tiles = p.gather_tiles == 2 ? 2 : p.gather_tiles != 0 ? 1 : 0;
@@ -428,6 +429,8 @@ int mrn_op_destroy(mrn_op *op) {
   op->bind.release();
   hipFree(op->fdev);
   hipFree(op->kwork_all);
+  hipFree(op->part);
+  hipFree(op->part_all);
   hipFree(op->xrng_all);
   hipFree(op->yrng_all);
   hipFree(op->tables_d);

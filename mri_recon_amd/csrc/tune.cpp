@@ -40,12 +40,12 @@ int adj_grid_pub(mrn_op *op, float2 *X, bool overwrite, const FrameData *fr, hip
 
 namespace {
 
-struct Knobs {
+struct Knobs {  // maxv 0: each frame's own (visits_per_item)
   int B, maxv, xrun_gather, gather_coils, xcd_run_fft, fft_stockham, scatter_valu;
 };
 
 Knobs current(const mrn_op *op) {
-  return Knobs{op->t.B, op->t.maxv, op->t.xrun_gather, op->gather_coils, op->xcd_run_fft,
+  return Knobs{op->t.B, op->auto_maxv ? 0 : op->t.maxv, op->t.xrun_gather, op->gather_coils, op->xcd_run_fft,
                op->fft_stockham ? 1 : 0, op->scatter_valu ? 1 : 0};
 }
 
@@ -57,7 +57,8 @@ void set_bins(mrn_op *op, int B) {
 
 void apply(mrn_op *op, const Knobs &k) {
   set_bins(op, k.B);
-  op->t.maxv = k.maxv;
+  op->t.maxv = k.maxv > 0 ? k.maxv : MRN_AUTO_MAXV;
+  op->auto_maxv = k.maxv <= 0;
   op->t.xrun_gather = k.xrun_gather;
   op->gather_coils = k.gather_coils;
   op->xcd_run_fft = k.xcd_run_fft;
@@ -228,7 +229,7 @@ bool from_map(const std::map<std::string, long long> &m, Knobs &k, float &ms) {
   k.scatter_valu = (int)m.at("scatter_valu");
   ms = (float)m.at("normal_us") / 1000.0f;
   // accept only values the op accepts
-  return (k.B == 1 || k.B == 2) && k.maxv > 0 && k.xrun_gather > 0 && k.xcd_run_fft > 0 &&
+  return (k.B == 1 || k.B == 2) && k.maxv >= 0 && k.xrun_gather > 0 && k.xcd_run_fft > 0 &&
          (k.gather_coils == 1 || k.gather_coils == 2 || k.gather_coils == 4 || k.gather_coils == 8);
 }
 
@@ -288,7 +289,7 @@ int autotune_impl(mrn_op *op, int f, const char *cache_path, hipStream_t st) {
   // 1. scatter
   float best_ms = 1e30f;
   for (int B : {1, 2})
-    for (int maxv : {1024, 4096, 16384})
+    for (int maxv : {0, 1024, 4096, 16384})
       for (int valu = 0; valu <= ((op->g.CC == 16 || op->g.CC == 8) ? 1 : 0); valu++) {
         Knobs k = best;
         k.B = B;

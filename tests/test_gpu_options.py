@@ -331,3 +331,28 @@ def test_kspace_support_pruning_bin_edge_2_and_autotune():
     after = op.normal(to_dev(X)).cpu().numpy()
     assert rel(after, before) <= 1e-5
     assert rel(op.backward(to_dev(X)).cpu().numpy(), A32) <= 1e-5
+
+
+@pytest.mark.parametrize("C", [2, 8, 16])
+@pytest.mark.parametrize("spokes", [3, 1100, 17000])
+def test_work_items_sized_from_the_sample_count(C, spokes):
+    """A^H with the default work items (64 visits at 96 samples, 64 to 1024
+    in whole batches between, 1024 at 544000) against one item per tile: the
+    same sums in another order, so FP32 rounding of a cell's partial sums.
+    The split tiles' parts are added in order: the same bits on every call."""
+    N = 24
+    traj = [t.cuda() for t in synth.radial_traj(spokes, 32, N)]
+    smaps = synth.coil_maps(C, N, seed=3).cuda()
+    d = synth.cn_image((C, traj[0].numel()), seed=4).cuda()
+    out = []
+    for mv in (0, 1 << 30):
+        op = GridFFT(N, ncoils=C, max_visits=mv)
+        op.set_traj(*traj)
+        op.set_smaps(smaps)
+        split = op.frame_stats()["split_tiles"]
+        assert (split > 0) if (mv == 0 and spokes > 3) else split == 0
+        out.append(op.forward(d, accumulate=False).cpu().numpy())
+        if op.frame_stats()["wide"] == 0:
+            assert np.array_equal(out[-1], op.forward(d, accumulate=False).cpu().numpy())
+        op.close()
+    assert rel(out[0], out[1]) <= 1e-6
