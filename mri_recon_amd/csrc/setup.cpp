@@ -136,8 +136,32 @@ static void make_window(mrn_op *op, int a) {
   op->win_h[a] = std::move(w);
 }
 
+// Coils per grid cell where the caller gave none.  8- and 16-coil blocks take
+// the four-step FFT passes, the k-space support and the matrix-core scatter;
+// blocks of 1, 2 and 4 take none of them, so that even mostly empty 8-coil
+// blocks are faster: the coils are padded to whole blocks (zero maps), of 16
+// when that pads no more than blocks of 8 would.  3 coils go as 4.  Pair of A
+// and A^H at 160^3, 800000 samples, the largest block that divides C / 8 / 16:
+// 3 coils 2.20 ms (4: 1.65) / 1.82 / 3.17; 5: 3.52 / 1.85 / 3.20; 6: 2.86 /
+// 1.87 / 3.20; 12: 4.55 / 3.40 / 3.23; 18: 7.94 / 5.19 / 6.30; 20: 7.49 /
+// 5.23 / 6.30; 28: 10.4 / 6.78 / 6.35.  1, 2 and 4 coils stay as they are:
+// 0.82, 1.05 and 1.69 ms against 1.83 ms in a block of 8.
 static int pick_cc(int C, int req) {
   if (req > 0) return req;
+  if (C <= 2) return C;
+  if (C <= 4) return 4;
+  return ((C + 7) / 8) % 2 ? 8 : 16;
+}
+
+static void set_blocks(mrn_op *op, int cc) {
+  op->g.CC = cc;
+  op->g.lgCC = 0;
+  while ((1 << op->g.lgCC) < cc) op->g.lgCC++;
+  op->nch = (op->C + cc - 1) / cc;
+}
+
+// The largest block that divides C: no padding, for grids that do not fit with it.
+static int exact_cc(int C) {
   int cc = 16;
   while (cc > 1 && (C % cc) != 0) cc >>= 1;
   return cc;
@@ -274,10 +298,7 @@ int mrn_op_create(const mrn_params *pin, mrn_op **out) {
   }
   g.ntab = (int)packed.size();
   const bool batched = p.form == MRN_FORM_BATCHED;
-  g.CC = batched ? pick_cc(op->C, p.coil_chunk) : 1;
-  g.lgCC = 0;
-  while ((1 << g.lgCC) < g.CC) g.lgCC++;
-  op->nch = (op->C + g.CC - 1) / g.CC;
+  set_blocks(op, batched ? pick_cc(op->C, p.coil_chunk) : 1);
   op->nvox = (int64_t)g.N[0] * g.N[1] * g.N[2];
   // sample bins (B = 1: one cell per bin, so a tile's bin neighbourhood is
   // exact) and scatter tiles (T = 4 cells: one wavefront)
@@ -371,23 +392,33 @@ int mrn_op_create(const mrn_params *pin, mrn_op **out) {
   }
   const int64_t ncell = (int64_t)g.S[0] * g.S[1] * g.S[2];
   if (batched) {
-    // frames fused into one launch per stage keep F grids side by side:
-    // forced (fuse_frames > 0), off (0), or when they take at most half the
-    // free device memory (-1)
-    op->fuse = false;
-    if (op->F > 1 && p.fuse_frames != 0) {
-      const double bytes = (double)sizeof(float2) * ncell * g.CC * op->nch * op->F;
-      size_t fm = 0, tm = 0;
-      op->fuse = p.fuse_frames > 0 || (hipMemGetInfo(&fm, &tm) == hipSuccess && bytes <= 0.5 * (double)fm);
+    for (;;) {
+      // frames fused into one launch per stage keep F grids side by side:
+      // forced (fuse_frames > 0), off (0), or when they take at most half the
+      // free device memory (-1)
+      op->fuse = false;
+      if (op->F > 1 && p.fuse_frames != 0) {
+        const double bytes = (double)sizeof(float2) * ncell * g.CC * op->nch * op->F;
+        size_t fm = 0, tm = 0;
+        op->fuse = p.fuse_frames > 0 || (hipMemGetInfo(&fm, &tm) == hipSuccess && bytes <= 0.5 * (double)fm);
+      }
+      const int64_t ngrid = ncell * g.CC * op->nch * (op->fuse ? op->F : 1);
+      if (amalloc((void **)&op->grid, sizeof(float2) * ngrid) == hipSuccess &&
+          amalloc((void **)&op->smaps, sizeof(float2) * op->nvox * g.CC * op->nch) == hipSuccess) {
+        // zeroed once: the forward x pass leaves the cells outside a frame's
+        // k-space support as they are, and readers of whole tile regions weight
+        // them by zero, so they must hold finite values
+        if (hipMemset(op->grid, 0, sizeof(float2) * ngrid) != hipSuccess) return cleanup_fail(MRN_EHIP);
+        break;
+      }
+      // no room for padded coil blocks: those that divide the coil count
+      (void)hipGetLastError();
+      hipFree(op->grid);
+      op->grid = nullptr;
+      const int cc = p.coil_chunk > 0 ? g.CC : exact_cc(op->C);
+      if (cc == g.CC) return cleanup_fail(MRN_ENOMEM);
+      set_blocks(op, cc);
     }
-    const int64_t ngrid = ncell * g.CC * op->nch * (op->fuse ? op->F : 1);
-    if (amalloc((void **)&op->grid, sizeof(float2) * ngrid) != hipSuccess) return cleanup_fail(MRN_ENOMEM);
-    // zeroed once: the forward x pass leaves the cells outside a frame's
-    // k-space support as they are, and readers of whole tile regions weight
-    // them by zero, so they must hold finite values
-    if (hipMemset(op->grid, 0, sizeof(float2) * ngrid) != hipSuccess) return cleanup_fail(MRN_EHIP);
-    if (amalloc((void **)&op->smaps, sizeof(float2) * op->nvox * g.CC * op->nch) != hipSuccess)
-      return cleanup_fail(MRN_ENOMEM);
   } else {
     if (amalloc((void **)&op->smaps, sizeof(float2) * op->nvox * op->C) != hipSuccess)
       return cleanup_fail(MRN_ENOMEM);

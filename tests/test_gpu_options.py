@@ -356,3 +356,16 @@ def test_work_items_sized_from_the_sample_count(C, spokes):
             assert np.array_equal(out[-1], op.forward(d, accumulate=False).cpu().numpy())
         op.close()
     assert rel(out[0], out[1]) <= 1e-6
+
+
+@pytest.mark.parametrize("C,block", [(1, 1), (2, 2), (3, 4), (4, 4), (5, 8), (8, 8), (9, 16), (16, 16), (17, 8),
+                                     (25, 16), (33, 8)])
+def test_padded_coil_blocks(C, block):
+    """The default coil block at the edges of its ranges: the grid in blocks
+    of that size, A and A^H of every coil against the oracle, and E'E against
+    A^H W A (the padding coils add nothing)."""
+    N = 16
+    op = GridFFT(N, ncoils=C)
+    assert op.grid_raw().shape[-1] == block and op.grid().shape[0] == C
+    op.close()
+    check({}, N, C, 60 + C, forms=("batched",))
