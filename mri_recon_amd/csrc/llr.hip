@@ -3,7 +3,9 @@
 // recon_lib calls them after each gradient step (recon_lib.cpp:2117-2126).
 //
 // Block b of a pass is the Np x N matrix A (N = frames along `dim`, Np = the
-// other frames x block voxels).  One wavefront (or half of one) per block:
+// other frames x block voxels).  Up to 8 frames go 8 or 16 blocks to a
+// wavefront with the matrices in registers (k_llr_reg); more take a wavefront,
+// or half of one, per block:
 //   1-2. G = A^H A in FP64, A's rows streamed through LDS one chunk of LPB
 //      rows at a time (periodic wrap, the pass's shift), so a block holds
 //      N x (LPB + 1) values of A in LDS instead of all Np rows;
@@ -26,6 +28,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+
+#include <type_traits>
 
 #include "mrn_internal.hpp"
 
@@ -324,6 +328,230 @@ __global__ __launch_bounds__(64) void k_llr_block(float2 *__restrict__ X, LlrGeo
 #undef GM
 #undef VM
 
+// ---- up to 8 frames: the Gram matrix in registers
+// NL lanes per block (4 or 8; frames beyond N are zero columns), 64 / NL
+// blocks per wavefront, neighbouring blocks along x.  Lane j of a block's
+// group holds column j of G = A^H A and of V; register i of G is row i ^ j, so
+// that the diagonal is register 0 and every index below is a constant.  The
+// rounds of a Jacobi sweep pair lane j with lane j ^ m, m = 1 .. NL - 1 (every
+// pair once), and all exchanges are lane xors: DPP moves or LDS swizzles, no
+// LDS traffic and no barriers.
+// The form above spent its time in LDS round trips and barriers with N / 2 of
+// 32 lanes on a rotation.  256^3 x 8 frames, 4^3 blocks: 4.42 ms per pass
+// before, 2.0 now (the call 21.1 -> 9.1 ms).  What remains is the rotations' FP64 arithmetic and the
+// image traffic.  16 lanes for 9 to 16 frames (256 registers, one wavefront per
+// SIMD, and 10 frames rotating 120 pairs for their 45) was slower than the form
+// above, 160^3 x 10 frames with 8^3 blocks 109.2 against 103.8 ms per two
+// FISTA iterations, so those keep it.
+template <int M>
+__device__ __forceinline__ int lane_xor(int v) {
+  static_assert(M >= 1 && M < 32, "within 32 lanes");
+  if constexpr (M == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);        // quad_perm 1,0,3,2
+  else if constexpr (M == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);   // quad_perm 2,3,0,1
+  else if constexpr (M == 3) return __builtin_amdgcn_mov_dpp(v, 0x1B, 0xF, 0xF, true);   // quad_perm 3,2,1,0
+  else if constexpr (M == 7) return __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true);  // row_half_mirror
+  else if constexpr (M == 15) return __builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, true); // row_mirror
+  else return __builtin_amdgcn_ds_swizzle(v, (M << 10) | 0x1F);
+}
+template <int M>
+__device__ __forceinline__ float lane_xor(float v) {
+  return __int_as_float(lane_xor<M>(__float_as_int(v)));
+}
+template <int M>
+__device__ __forceinline__ double lane_xor(double v) {
+  return __hiloint2double(lane_xor<M>(__double2hiint(v)), lane_xor<M>(__double2loint(v)));
+}
+
+// f(std::integral_constant<int, I>) for I in [B, E)
+template <int B, int E, class F>
+__device__ __forceinline__ void unroll(F &&f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    unroll<B + 1, E>(f);
+  }
+}
+
+template <bool THRESH, int NL>
+__global__ __launch_bounds__(64) void k_llr_reg(float2 *__restrict__ X, LlrGeom g, int pass,
+                                                const int *__restrict__ counter, long long call,
+                                                const double *__restrict__ tau_dev, double *__restrict__ smax_out) {
+  constexpr int BPW = 64 / NL;
+  constexpr int LDV = NL + 1;  // a row of V in LDS, padded against bank conflicts
+  __shared__ double2 s_v[THRESH ? BPW : 1][THRESH ? NL * LDV : 1];
+  __shared__ double s_f[THRESH ? BPW : 1][THRESH ? NL : 1];
+  const int lane = threadIdx.x, grp = lane / NL, j = lane % NL;
+  const int N = g.N;
+  const long long bq = (long long)blockIdx.x * BPW + grp;
+  const bool live = bq < g.nblk;  // a padding group repeats the last block and writes nothing
+  const long long b = live ? bq : g.nblk - 1;
+  const int bi = (int)(b % g.nb[0]), bj = (int)((b / g.nb[0]) % g.nb[1]),
+            bk = (int)(b / ((long long)g.nb[0] * g.nb[1]));
+  int sh[3] = {0, 0, 0};
+  if (THRESH && g.block_iter > 1) {
+    const long long c = counter ? (long long)(*counter - 1) : call;
+    for (int q = 0; q < 3; q++)
+      sh[q] = (int)(splitmix(g.seed, 3ull * (unsigned long long)(c * g.block_iter + pass) + q) %
+                    (unsigned long long)g.bs[q]) -
+              g.bs[q] / 2;
+  }
+  const int o0 = bi * g.bs[0] + sh[0], o1 = bj * g.bs[1] + sh[1], o2 = bk * g.bs[2] + sh[2];
+  auto wrap = [&](int v, int n) -> int { return v < 0 ? v + n : v >= n ? v - n : v; };  // v in (-n, 2 n)
+  const int nother = g.dim == 0 ? g.Ne : g.Nt;
+  // this lane's column: frame j of the low-rank dimension
+  const bool col = j < N;
+  // f(voxel address of this lane's frame) for the block's rows, LLR_STEP at a
+  // time (every lane of a wavefront walks the same number)
+  constexpr int STEP = 4;
+  auto rows = [&](auto &&f) {
+    for (int o = 0; o < nother; o++) {
+      const long long fr = g.dim == 0 ? ((long long)(col ? j : 0) * g.Ne + o) : ((long long)o * g.Ne + (col ? j : 0));
+      float2 *F = X + fr * g.nvox;
+      for (int kk = 0; kk < g.bs[2]; kk++) {
+        const int pz = wrap(o2 + kk, g.Nv[2]);
+        for (int jj = 0; jj < g.bs[1]; jj++) {
+          float2 *row = F + ((long long)pz * g.Nv[1] + wrap(o1 + jj, g.Nv[1])) * g.Nv[0];
+          for (int ii = 0; ii < g.bs[0]; ii += STEP) {
+            float2 *at[STEP];
+            float2 v[STEP];
+#pragma unroll
+            for (int q = 0; q < STEP; q++) {
+              const bool in = ii + q < g.bs[0];
+              at[q] = row + wrap(o0 + (in ? ii + q : ii), g.Nv[0]);
+              v[q] = in && col ? *at[q] : make_float2(0.f, 0.f);
+            }
+#pragma unroll
+            for (int q = 0; q < STEP; q++)
+              if (ii + q < g.bs[0]) f(at[q], v[q]);  // (uniform)
+          }
+        }
+      }
+    }
+  };
+  // 1. Gram matrix: G[i ^ j][j] += conj(x_{i ^ j}) x_j
+  double gr[NL], gi[NL];
+#pragma unroll
+  for (int i = 0; i < NL; i++) gr[i] = gi[i] = 0.0;
+  rows([&](float2 *, float2 v) {
+    const double xr = v.x, xi = v.y;
+    gr[0] += xr * xr + xi * xi;
+    unroll<1, NL>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      const double ar = lane_xor<i>(v.x), ai = lane_xor<i>(v.y);
+      gr[i] += ar * xr + ai * xi;
+      gi[i] += ar * xi - ai * xr;
+    });
+  });
+  // 2. Jacobi sweeps
+  double vr[THRESH ? NL : 1], vi[THRESH ? NL : 1];
+  if constexpr (THRESH) {
+#pragma unroll
+    for (int r = 0; r < NL; r++) {
+      vr[r] = r == j ? 1.0 : 0.0;
+      vi[r] = 0.0;
+    }
+  }
+  for (int sweep = 0; sweep < LLR_SWEEPS; sweep++) {
+    double off = 0.0, dia = gr[0] * gr[0];
+#pragma unroll
+    for (int i = 1; i < NL; i++) off += gr[i] * gr[i] + gi[i] * gi[i];
+    for (int q = 1; q < NL; q <<= 1) {
+      off += __shfl_xor(off, q);
+      dia += __shfl_xor(dia, q);
+    }
+    const bool done = off <= 1e-24 * dia || dia == 0.0;
+    if (__all(done)) break;  // a converged block stops rotating until its wavefront is done
+    unroll<1, NL>([&](auto MM) {
+      constexpr int m = decltype(MM)::value;
+      const bool lower = j < (j ^ m);  // this lane is column p of the pair (p, q)
+      // the rotation that zeroes G[p][q], from lane p's values in both lanes:
+      // t = 2 |G_pq| / (|d| + sqrt(d^2 + 4 |G_pq|^2)) with the sign of d = G_qq - G_pp,
+      // w = t G_pq / |G_pq|, c = 1 / sqrt(1 + t^2), s e = c w.  Entries are
+      // sums of squared floats: their squares neither overflow nor vanish.
+      const double hr0 = lane_xor<m>(gr[m]), hi0 = lane_xor<m>(gi[m]), dg = lane_xor<m>(gr[0]);
+      const double hr = lower ? gr[m] : hr0, hi = lower ? gi[m] : hi0;  // G[q][p]
+      const double d = lower ? dg - gr[0] : gr[0] - dg;
+      const double h2 = hr * hr + hi * hi;
+      double c = 1.0, cr = 0.0, ci = 0.0;  // this column: own' = c own + (cr + i ci) other
+      if (h2 > 0.0 && !done) {
+        const double t = (d >= 0.0 ? 2.0 : -2.0) / (fabs(d) + sqrt(d * d + 4.0 * h2));
+        const double wr = t * hr, wi = -t * hi;  // w = t G[p][q]
+        c = 1.0 / sqrt(1.0 + (wr * wr + wi * wi));
+        cr = lower ? -c * wr : c * wr;  // p: -conj(s e), q: s e
+        ci = c * wi;
+      }
+      // columns, then rows i ^ j and i ^ j ^ m (registers i and i ^ m) with
+      // the rotation of the lanes that hold those columns
+      unroll<0, NL>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        if constexpr (i < (i ^ m)) {
+          constexpr int k = i ^ m;
+          const double ar = lane_xor<m>(gr[k]), ai = lane_xor<m>(gi[k]), br = lane_xor<m>(gr[i]), bi_ = lane_xor<m>(gi[i]);
+          const double xr = c * gr[i] + (cr * ar - ci * ai), xi = c * gi[i] + (cr * ai + ci * ar);
+          const double yr = c * gr[k] + (cr * br - ci * bi_), yi = c * gi[k] + (cr * bi_ + ci * br);
+          double rc = c, rr = cr, ri = ci;  // lane i ^ j's rotation; lane i ^ j ^ m has c, -conj
+          if constexpr (i != 0) {
+            rc = lane_xor<i>(c);
+            rr = lane_xor<i>(cr);
+            ri = lane_xor<i>(ci);
+          }
+          gr[i] = rc * xr + (rr * yr + ri * yi);  // conj(r) y
+          gi[i] = rc * xi + (rr * yi - ri * yr);
+          gr[k] = rc * yr - (rr * xr - ri * xi);  // -r x
+          gi[k] = rc * yi - (rr * xi + ri * xr);
+        }
+      });
+      if (!done) gr[m] = gi[m] = 0.0;  // the pair's own entries
+      if constexpr (THRESH) {
+#pragma unroll
+        for (int r = 0; r < NL; r++) {
+          const double ar = lane_xor<m>(vr[r]), ai = lane_xor<m>(vi[r]);
+          const double xr = c * vr[r] + (cr * ar - ci * ai);
+          vi[r] = c * vi[r] + (cr * ai + ci * ar);
+          vr[r] = xr;
+        }
+      }
+    });
+  }
+  // 3. results: the eigenvalue of column j is gr[0]
+  const double sv = sqrt(fmax(gr[0], 0.0));
+  if constexpr (!THRESH) {
+    double m = sv;
+    for (int q = 1; q < NL; q <<= 1) m = fmax(m, __shfl_xor(m, q));
+    if (j == 0 && live) smax_out[b] = m;
+  } else {
+    const double tau = *tau_dev;
+    s_f[grp][j] = sv > 0.0 ? fmax(sv - tau, 0.0) / sv : 0.0;
+#pragma unroll
+    for (int r = 0; r < NL; r++) s_v[grp][r * LDV + j] = make_double2(vr[r], vi[r]);
+    __syncthreads();
+    // P = V diag(f) V^H, column j in gr, gi with the rows in their xor order
+#pragma unroll
+    for (int i = 0; i < NL; i++) gr[i] = gi[i] = 0.0;
+    for (int k = 0; k < NL; k++) {
+      const double2 w = s_v[grp][j * LDV + k];
+      const double ur = s_f[grp][k] * w.x, ui = -s_f[grp][k] * w.y;  // f_k conj(V[j][k])
+#pragma unroll
+      for (int i = 0; i < NL; i++) {
+        const double2 v = s_v[grp][(i ^ j) * LDV + k];
+        gr[i] += v.x * ur - v.y * ui;
+        gi[i] += v.x * ui + v.y * ur;
+      }
+    }
+    // A P back to the image (blocks of a pass share no voxel)
+    rows([&](float2 *at, float2 v) {
+      const double xr = v.x, xi = v.y;
+      double yr = xr * gr[0] - xi * gi[0], yi = xr * gi[0] + xi * gr[0];
+      unroll<1, NL>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        const double ar = lane_xor<i>(v.x), ai = lane_xor<i>(v.y);
+        yr += ar * gr[i] - ai * gi[i];
+        yi += ar * gi[i] + ai * gr[i];
+      });
+      if (live && col) *at = make_float2((float)yr, (float)yi);
+    });
+  }
+}
+
 // ---- exact median of the nonzero block maxima: radix select over the bit
 // patterns of the (non-negative) doubles, 8 bits per pass, two ranks at once.
 struct SelState {
@@ -472,7 +700,18 @@ static hipError_t llr_launch(const LlrGeom &g, float2 *X, float alpha, float amp
   const size_t lds = llr_lds(g);
   const unsigned nwg = (unsigned)((nblk + (64 / g.lpb) - 1) / (64 / g.lpb));
   auto blocks = [&](bool thresh, int pass) {
-    if (g.lpb == 32) {
+    if (g.N <= 8) {  // 4 or 8 lanes per block, in registers
+      const int nl = g.N <= 4 ? 4 : 8;
+      const unsigned nw = (unsigned)((nblk + 64 / nl - 1) / (64 / nl));
+#define LLR_REG(T, n)                                                                                          \
+  hipLaunchKernelGGL((k_llr_reg<T, n>), dim3(nw), dim3(64), 0, st, X, g, pass, counter, call,                 \
+                     T ? (const double *)tau : nullptr, T ? nullptr : sblocks)
+      if (thresh && nl == 4) LLR_REG(true, 4);
+      else if (thresh) LLR_REG(true, 8);
+      else if (nl == 4) LLR_REG(false, 4);
+      else LLR_REG(false, 8);
+#undef LLR_REG
+    } else if (g.lpb == 32) {
       if (thresh)
         hipLaunchKernelGGL((k_llr_block<true, 32>), dim3(nwg), dim3(64), lds, st, X, g, pass, counter, call, tau,
                            (double *)nullptr);
