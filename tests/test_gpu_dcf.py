@@ -111,3 +111,25 @@ def test_dcf_full_size_duplicate_property():
     M = kx.numel()
     assert torch.count_nonzero(a).item() > 0.99 * M
     assert rel(b[:M].cpu().numpy(), a.cpu().numpy() / 2) < 1e-4
+
+
+@pytest.mark.parametrize("N,spokes,npts,dwin,os_", [(7, 3, 5, 2.1, 2.1), ((9, 21, 33), 40, 30, 1.0, 1.3),
+                                                   (24, 400, 60, 2.5, 2.1), (31, 50, 40, 2.9, 1.7),
+                                                   (20, 9000, 24, 2.0, 2.1)])
+def test_dcf_tiles_match_oracle(N, spokes, npts, dwin, os_):
+    """The one-width form at its edges: a grid of a few tiles with partly
+    filled last ones, narrow and wide kernels (3 to 6 taps), tiles whose visits
+    fill several work items (9000 spokes through the centre), samples off the
+    grid and at infinity; the same weights on every call."""
+    n = N if isinstance(N, tuple) else (N, N, N)
+    kx, ky, kz = radial(spokes, npts, min(n))
+    kx, ky, kz = [np.r_[k, e].astype(np.float32) for k, e in
+                  ((kx, [300.0, 0.0, 0.0, 1e30]), (ky, [0.0, -300.0, 0.0, 0.0]), (kz, [0.0, 0.0, n[0] / 2.0, 0.0]))]
+    d = [dev(k) for k in (kx, ky, kz)]
+    got = dcf_calc(*d, N=n, iters=4, dwin=dwin, overgrid=os_).cpu().numpy()
+    again = dcf_calc(*d, N=n, iters=4, dwin=dwin, overgrid=os_).cpu().numpy()
+    assert np.array_equal(got, again, equal_nan=True)
+    p = orc.dcf_params(n, iters=4, dwin=dwin, overgrid=os_)
+    ref, _ = orc.dcf_calc(p, kx[:-1], ky[:-1], kz[:-1], "f32")
+    assert not got[-1] > 0  # the sample at infinity has no taps
+    assert rel(got[:-1], ref) <= 3e-5
