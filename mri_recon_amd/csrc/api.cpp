@@ -822,7 +822,7 @@ int mrn_fista(mrn_op *op, void *Xv, int iters, double step, int use_graph, doubl
   const float stf = (float)step;
   const bool l1 = op->l1_fraction > 0.0f;
   const bool cauchy = op->step_type == MRN_STEP_CAUCHY;
-  if (l1) MRN_TRY(ensure_l1_state(op));  // before any capture
+  if (l1) MRN_TRY(l1_fista_prepare(op));  // before any capture
   MRN_TRY(llr_fista_prepare(op));
   MRN_TRY(fused_prepare(op, st));
   if (cauchy) MRN_TRY(op_set_step(op, stf, 0.0f, st));  // the step until the first Cauchy update

@@ -243,6 +243,8 @@ struct mrn_op {
   void *dthr = nullptr;        // threshold search state
   int *dsh = nullptr;          // cycle-spin shifts [MRN_MAX_SPINS][3]
   double *dthr_log = nullptr;  // threshold per FISTA iteration
+  float2 *wave_T = nullptr;    // second image of the wavelet step (grow-only; null: no memory for it)
+  size_t wave_T_cap = 0;
   // locally low-rank step of FISTA over the frames (off unless alpha_time > 0)
   bool llr_on = false;
   mrn_llr_params llr{};
@@ -558,5 +560,6 @@ int l1_wavelet_host(mrn_op *op, float2 *X, int frames, float fraction, const int
                     const int32_t *shifts, double *thr, hipStream_t st);
 int l1_fista_step(mrn_op *op, float2 *X, hipStream_t st);
 int ensure_l1_state(mrn_op *op);
+int l1_fista_prepare(mrn_op *op);
 
 }  // namespace mrn

@@ -488,6 +488,7 @@ int mrn_op_destroy(mrn_op *op) {
   hipFree(op->dthr);
   hipFree(op->dsh);
   hipFree(op->dthr_log);
+  hipFree(op->wave_T);
   hipFree(op->llr_sblocks);
   hipFree(op->llr_sel);
   hipFree(op->llr_scal);

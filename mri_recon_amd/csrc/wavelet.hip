@@ -138,6 +138,203 @@ __global__ __launch_bounds__(256) void k_wave_lines(float2 *X, int N0, int N1, i
   });
 }
 
+// ------------------------------------------------------- first level, 3 axes
+// The first level of a 3-D transform, all three axes in one pass from one
+// image to another: 7/8 of a transform's traffic is in this level, which as
+// three line passes reads and writes the image three times.  A workgroup
+// loads the region that its outputs reach into LDS and transforms it along x,
+// y, z (synthesis: z, y, x) in place, each thread holding its outputs in
+// registers across the barrier; the products and their order are those of
+// k_wave_lines, so the results are the same bits.  The synthesis applies the
+// soft threshold to the seven detail octants as it loads them (the low-pass
+// octant holds the deeper levels' image by then).
+// 256 x 256 x 192, 4 levels, 4 spins: the step 3.10 -> 2.05 ms (analysis of the
+// first level 63 us, synthesis with the threshold 154 us).
+#define W3_THREADS 512
+#define W3_PX 16  // analysis: output positions of a workgroup (a low- and a high-pass value each per axis)
+#define W3_PY 8
+#define W3_PZ 4
+
+__device__ __forceinline__ float cabs_rn(float2 v) {
+  return (float)sqrt((double)v.x * v.x + (double)v.y * v.y);
+}
+__device__ __forceinline__ float2 soft(float2 v, float thr) {
+  const float cc = cabs_rn(v);
+  if (cc <= thr) return make_float2(0.f, 0.f);
+  const float f = 1.0f - thr / cc;
+  return make_float2(v.x * f, v.y * f);
+}
+
+// out[(line, pos)] = the filter pair at `pos` over in[base + (2 pos + 3 - fp) st], fp = 0..3
+__device__ __forceinline__ void wave_pair(const float2 *in, int at, int st, const D4 &f, float2 &lo, float2 &hi) {
+  lo = hi = make_float2(0.f, 0.f);
+#pragma unroll
+  for (int fp = 0; fp < 4; fp++) {
+    const float2 v = in[at + (3 - fp) * st];
+    lo.x += f.lpf[fp] * v.x;
+    lo.y += f.lpf[fp] * v.y;
+    hi.x += f.hpf[fp] * v.x;
+    hi.y += f.hpf[fp] * v.y;
+  }
+}
+
+__global__ __launch_bounds__(W3_THREADS) void k_wave3_fwd(float2 *__restrict__ T, const float2 *__restrict__ X, int N0,
+                                                          int N1, int N2, int nz, const int *__restrict__ sh, D4 f) {
+  constexpr int RX = 2 * W3_PX + 2, RY = 2 * W3_PY + 2, RZ = 2 * W3_PZ + 2;
+  __shared__ float2 A[RX * RY * RZ];
+  const int fr = blockIdx.z / nz;
+  const int p0[3] = {(int)blockIdx.x * W3_PX, (int)blockIdx.y * W3_PY, (int)(blockIdx.z - fr * nz) * W3_PZ};
+  const int64_t n = (int64_t)N0 * N1 * N2;
+  const float2 *Xf = X + fr * n;
+  float2 *Tf = T + fr * n;
+  // cell (x, y, z) of the region: image point 2 p0 + shift - 3 + (x, y, z)
+  const int ox = 2 * p0[0] + sh[0] - 3, oy = 2 * p0[1] + sh[1] - 3, oz = 2 * p0[2] + sh[2] - 3;
+  for (int q = threadIdx.x; q < RX * RY * RZ; q += W3_THREADS) {
+    const int x = q % RX, yz = q / RX, y = yz % RY, z = yz / RY;
+    A[q] = Xf[((int64_t)wmod(oz + z, N2) * N1 + wmod(oy + y, N1)) * N0 + wmod(ox + x, N0)];
+  }
+  __syncthreads();
+  {  // x: RY * RZ lines of W3_PX positions
+    constexpr int TOT = RY * RZ * W3_PX, PER = (TOT + W3_THREADS - 1) / W3_THREADS;
+    float2 lo[PER], hi[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int q = threadIdx.x + k * W3_THREADS, p = q % W3_PX, ln = q / W3_PX;
+      if (q < TOT) wave_pair(A, ln * RX + 2 * p, 1, f, lo[k], hi[k]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int q = threadIdx.x + k * W3_THREADS, p = q % W3_PX, ln = q / W3_PX;
+      if (q < TOT) {
+        A[ln * RX + p] = lo[k];
+        A[ln * RX + W3_PX + p] = hi[k];
+      }
+    }
+    __syncthreads();
+  }
+  {  // y: 2 W3_PX x RZ lines of W3_PY positions, x fastest
+    constexpr int NX = 2 * W3_PX, TOT = NX * RZ * W3_PY, PER = (TOT + W3_THREADS - 1) / W3_THREADS;
+    float2 lo[PER], hi[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int q = threadIdx.x + k * W3_THREADS, x = q % NX, p = (q / NX) % W3_PY, z = q / (NX * W3_PY);
+      if (q < TOT) wave_pair(A, (z * RY + 2 * p) * RX + x, RX, f, lo[k], hi[k]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int q = threadIdx.x + k * W3_THREADS, x = q % NX, p = (q / NX) % W3_PY, z = q / (NX * W3_PY);
+      if (q < TOT) {
+        A[(z * RY + p) * RX + x] = lo[k];
+        A[(z * RY + W3_PY + p) * RX + x] = hi[k];
+      }
+    }
+    __syncthreads();
+  }
+  // z, straight to the image
+  constexpr int NX = 2 * W3_PX, NY = 2 * W3_PY, TOT = NX * NY * W3_PZ;
+  const int h0 = N0 >> 1, h1 = N1 >> 1, h2 = N2 >> 1;
+  for (int q = threadIdx.x; q < TOT; q += W3_THREADS) {
+    const int x = q % NX, y = (q / NX) % NY, p = q / (NX * NY);
+    const int px = p0[0] + x % W3_PX, py = p0[1] + y % W3_PY, pz = p0[2] + p;
+    if (px >= h0 || py >= h1 || pz >= h2) continue;
+    float2 lo, hi;
+    wave_pair(A, (2 * p * RY + y) * RX + x, RY * RX, f, lo, hi);
+    float2 *dst = Tf + (int64_t)(py + (y < W3_PY ? 0 : h1)) * N0 + px + (x < W3_PX ? 0 : h0);
+    dst[(int64_t)pz * N1 * N0] = lo;
+    dst[(int64_t)(pz + h2) * N1 * N0] = hi;
+  }
+}
+
+// Synthesis: a workgroup makes W3_IX x W3_IY x W3_IZ points.  Point p takes the
+// positions t / 2 of the even t = p - fp + 3 - shift; the region holds the
+// workgroup's n / 2 + 2 positions per axis, low-pass then high-pass values.
+#define W3_IX 32
+#define W3_IY 16
+#define W3_IZ 8
+template <int H>  // distance of the high-pass value
+__device__ __forceinline__ float2 wave_point(const float2 *in, int p, int shift, int b0, int st, const D4 &f) {
+  float2 o = make_float2(0.f, 0.f);
+#pragma unroll
+  for (int fp = 0; fp < 4; fp++) {
+    const int t = p - fp + 3 - shift;
+    if (t & 1) continue;
+    const int at = ((t >> 1) - b0) * st;
+    const float2 a = in[at], d = in[at + H];
+    o.x += a.x * f.slpf[fp];
+    o.y += a.y * f.slpf[fp];
+    o.x += d.x * f.shpf[fp];
+    o.y += d.y * f.shpf[fp];
+  }
+  return o;
+}
+
+__global__ __launch_bounds__(W3_THREADS) void k_wave3_inv(float2 *__restrict__ X, const float2 *__restrict__ T, int N0,
+                                                          int N1, int N2, int nz, const int *__restrict__ sh, D4 f,
+                                                          const float *__restrict__ thr_p) {
+  constexpr int CX = W3_IX / 2 + 2, CY = W3_IY / 2 + 2, CZ = W3_IZ / 2 + 2;  // positions
+  constexpr int RX = 2 * CX, RY = 2 * CY, RZ = 2 * CZ;
+  extern __shared__ float2 A[];  // [RZ][RY][RX]
+  const int fr = blockIdx.z / nz;
+  const int p0[3] = {(int)blockIdx.x * W3_IX, (int)blockIdx.y * W3_IY, (int)(blockIdx.z - fr * nz) * W3_IZ};
+  const int64_t n = (int64_t)N0 * N1 * N2;
+  const float2 *Tf = T + fr * n;
+  float2 *Xf = X + fr * n;
+  const int h0 = N0 >> 1, h1 = N1 >> 1, h2 = N2 >> 1;
+  const int s0 = sh[0], s1 = sh[1], s2 = sh[2];
+  const int b0 = (p0[0] - s0 + 1) >> 1, b1 = (p0[1] - s1 + 1) >> 1, b2 = (p0[2] - s2 + 1) >> 1;  // first positions
+  const float thr = *thr_p;
+  for (int q = threadIdx.x; q < RX * RY * RZ; q += W3_THREADS) {
+    const int x = q % RX, yz = q / RX, y = yz % RY, z = yz / RY;
+    const bool hx = x >= CX, hy = y >= CY, hz = z >= CZ;
+    const int px = wmod(b0 + (hx ? x - CX : x), h0) + (hx ? h0 : 0), py = wmod(b1 + (hy ? y - CY : y), h1) + (hy ? h1 : 0),
+              pz = wmod(b2 + (hz ? z - CZ : z), h2) + (hz ? h2 : 0);
+    const float2 v = Tf[((int64_t)pz * N1 + py) * N0 + px];
+    A[q] = hx || hy || hz ? soft(v, thr) : v;
+  }
+  __syncthreads();
+  {  // z
+    constexpr int TOT = RX * RY * W3_IZ, PER = (TOT + W3_THREADS - 1) / W3_THREADS;
+    float2 o[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int q = threadIdx.x + k * W3_THREADS, xy = q % (RX * RY), p = q / (RX * RY);
+      if (q < TOT) o[k] = wave_point<CZ * RX * RY>(A + xy, p0[2] + p, s2, b2, RX * RY, f);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int q = threadIdx.x + k * W3_THREADS;
+      if (q < TOT) A[q] = o[k];  // [W3_IZ][RY][RX]
+    }
+    __syncthreads();
+  }
+  {  // y
+    constexpr int TOT = RX * W3_IY * W3_IZ, PER = (TOT + W3_THREADS - 1) / W3_THREADS;
+    float2 o[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int q = threadIdx.x + k * W3_THREADS, x = q % RX, p = (q / RX) % W3_IY, z = q / (RX * W3_IY);
+      if (q < TOT) o[k] = wave_point<CY * RX>(A + z * RY * RX + x, p0[1] + p, s1, b1, RX, f);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int q = threadIdx.x + k * W3_THREADS;
+      if (q < TOT) A[q] = o[k];  // [W3_IZ][W3_IY][RX]
+    }
+    __syncthreads();
+  }
+  // x, straight to the image
+  for (int q = threadIdx.x; q < W3_IX * W3_IY * W3_IZ; q += W3_THREADS) {
+    const int p = q % W3_IX, y = (q / W3_IX) % W3_IY, z = q / (W3_IX * W3_IY);
+    const int px = p0[0] + p, py = p0[1] + y, pz = p0[2] + z;
+    if (px >= N0 || py >= N1 || pz >= N2) continue;
+    Xf[((int64_t)pz * N1 + py) * N0 + px] = wave_point<CX>(A + (z * W3_IY + y) * RX, px, s0, b0, 1, f);
+  }
+}
+
 // ------------------------------------------------------------ threshold
 #define THR_DEPTH 4                         // bisection steps per counting pass
 #define THR_NODES ((1 << THR_DEPTH) - 1)    // candidate values per pass
@@ -168,10 +365,6 @@ __device__ __forceinline__ void thr_tree(const ThrState &s, float (&v)[THR_NODES
     hi[2 * k + 2] = hi[k];
     v[2 * k + 2] = 0.5f * (hi[2 * k + 2] + lo[2 * k + 2]);
   }
-}
-
-__device__ __forceinline__ float cabs_rn(float2 v) {
-  return (float)sqrt((double)v.x * v.x + (double)v.y * v.y);
 }
 
 __global__ void k_thr_reset(ThrState *s) {
@@ -295,17 +488,16 @@ __global__ void k_thr_final(ThrState *s, float scale, double *log, const int *co
   }
 }
 
-__global__ __launch_bounds__(256) void k_soft(float2 *X, int64_t n, const ThrState *__restrict__ s) {
+// soft threshold of the sub-block [0, s0) x [0, s1) x [0, s2) of each frame (blockIdx.y)
+__global__ __launch_bounds__(256) void k_soft(float2 *X, int N0, int N1, int s0, int s1, int s2, int64_t frame_stride,
+                                              const ThrState *__restrict__ s) {
   const float thr = s->thr;
+  float2 *Xf = X + (int64_t)blockIdx.y * frame_stride;
+  const int64_t n = (int64_t)s0 * s1 * s2;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const float2 v = X[i];
-    const float cc = cabs_rn(v);
-    if (cc <= thr) {
-      X[i] = make_float2(0.f, 0.f);
-    } else {
-      const float f = 1.0f - thr / cc;
-      X[i] = make_float2(v.x * f, v.y * f);
-    }
+    const int64_t yz = i / s0;
+    float2 *v = Xf + ((yz / s1) * N1 + yz % s1) * N0 + i % s0;
+    *v = soft(*v, thr);
   }
 }
 
@@ -339,6 +531,14 @@ int ensure_l1_state(mrn_op *op) {
   return MRN_OK;
 }
 
+// ... and what FISTA's step uses, before any capture
+static void ensure_wave_T(mrn_op *op, int frames);
+int l1_fista_prepare(mrn_op *op) {
+  MRN_TRY(ensure_l1_state(op));
+  ensure_wave_T(op, op->F);
+  return MRN_OK;
+}
+
 static int wave_axis(mrn_op *op, float2 *X, int frames, const int s[3], int axis, const int *sh, bool inv,
                      hipStream_t st) {
   static const D4 f = d4_filters();
@@ -360,16 +560,18 @@ static int wave_axis(mrn_op *op, float2 *X, int frames, const int s[3], int axis
   return MRN_OK;
 }
 
-// forward3D / backward3D of `frames` images, shifts sh[0..2] in device memory
-int wavelet3d(mrn_op *op, float2 *X, int frames, const int req[3], const int *sh, bool inv, hipStream_t st) {
+// forward3D / backward3D of `frames` images, shifts sh[0..2] in device memory;
+// levels l0 and deeper (l0 > 0: every axis has l0 levels, done elsewhere)
+int wavelet3d(mrn_op *op, float2 *X, int frames, const int req[3], const int *sh, bool inv, hipStream_t st,
+              int l0 = 0) {
   const int *N = op->g.N;
   int L[3];
   wavelet_levels(N, req, L);
   int maxl = 0;
   for (int a = 0; a < 3; a++) maxl = L[a] > maxl ? L[a] : maxl;
   if (!inv) {
-    int s[3] = {N[0], N[1], N[2]};
-    for (int l = 0; l < maxl; l++) {
+    int s[3] = {N[0] >> l0, N[1] >> l0, N[2] >> l0};
+    for (int l = l0; l < maxl; l++) {
       for (int a = 0; a < 3; a++)
         if (l < L[a]) MRN_TRY(wave_axis(op, X, frames, s, a, sh, false, st));
       for (int a = 0; a < 3; a++)
@@ -378,7 +580,7 @@ int wavelet3d(mrn_op *op, float2 *X, int frames, const int req[3], const int *sh
   } else {
     int s[3];
     for (int a = 0; a < 3; a++) s[a] = N[a] >> L[a];
-    for (int l = maxl - 1; l >= 0; l--) {
+    for (int l = maxl - 1; l >= l0; l--) {
       for (int a = 0; a < 3; a++)
         if (l < L[a]) s[a] = N[a] >> l;
       for (int a = 2; a >= 0; a--)
@@ -411,19 +613,62 @@ static int fraction_threshold(mrn_op *op, const float2 *X, int64_t n, float frac
   return MRN_OK;
 }
 
-// The L1 step over `frames` images; shifts of spin q at dsh[3q..3q+2].
+static unsigned wave_blocks(int n, int per) { return (unsigned)((n + per - 1) / per); }
+
+// first level of every axis: X -> T, and T (detail octants thresholded) -> X
+static int wave3_first(mrn_op *op, float2 *X, float2 *T, int frames, const int *sh, bool inv, hipStream_t st) {
+  static const D4 f = d4_filters();
+  const int *N = op->g.N;
+  if (!inv) {
+    const unsigned nz = wave_blocks(N[2] / 2, W3_PZ);
+    hipLaunchKernelGGL(k_wave3_fwd, dim3(wave_blocks(N[0] / 2, W3_PX), wave_blocks(N[1] / 2, W3_PY), nz * frames),
+                       dim3(W3_THREADS), 0, st, T, X, N[0], N[1], N[2], (int)nz, sh, f);
+  } else {
+    constexpr size_t lds = sizeof(float2) * (W3_IX + 4) * (W3_IY + 4) * (W3_IZ + 4);
+    static const hipError_t attr =
+        hipFuncSetAttribute((const void *)k_wave3_inv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    MRN_HIP(op, attr);
+    const unsigned nz = wave_blocks(N[2], W3_IZ);
+    hipLaunchKernelGGL(k_wave3_inv, dim3(wave_blocks(N[0], W3_IX), wave_blocks(N[1], W3_IY), nz * frames),
+                       dim3(W3_THREADS), lds, st, X, T, N[0], N[1], N[2], (int)nz, sh, f,
+                       &((const ThrState *)op->dthr)->thr);
+  }
+  MRN_HIP(op, hipGetLastError());
+  return MRN_OK;
+}
+
+// The L1 step over `frames` images; shifts of spin q at dsh[3q..3q+2].  With a
+// level on every axis and the second image (op->wave_T) the coefficients live
+// there; otherwise everything runs in place.
 int l1_wavelet_step(mrn_op *op, float2 *X, int frames, float fraction, const int levels[3], int spins,
                     const int *log_counter, hipStream_t st) {
   const int64_t n = (int64_t)frames * op->nvox;
+  const int *N = op->g.N;
+  int L[3];
+  wavelet_levels(N, levels, L);
+  const bool two = L[0] > 0 && L[1] > 0 && L[2] > 0 && op->wave_T && op->wave_T_cap >= (size_t)n &&
+                   wave_blocks(N[2], W3_IZ) * (int64_t)frames <= 65535;
+  float2 *T = two ? op->wave_T : X;
+  const int s = two ? 1 : 0;  // the level in T's (or X's) corner that is left to do in place
   for (int q = 0; q < spins; q++) {
     const int *sh = op->dsh + 3 * q;
-    MRN_TRY(wavelet3d(op, X, frames, levels, sh, false, st));
-    if (q == 0) MRN_TRY(fraction_threshold(op, X, n, fraction, 1.0f / (float)spins, log_counter, st));
-    hipLaunchKernelGGL(k_soft, dim3(grid_for(n)), dim3(256), 0, st, X, n, (const ThrState *)op->dthr);
+    if (two) MRN_TRY(wave3_first(op, X, T, frames, sh, false, st));
+    MRN_TRY(wavelet3d(op, T, frames, levels, sh, false, st, s));
+    if (q == 0) MRN_TRY(fraction_threshold(op, T, n, fraction, 1.0f / (float)spins, log_counter, st));
+    hipLaunchKernelGGL(k_soft, dim3(grid_for((n / frames) >> (3 * s)), frames), dim3(256), 0, st, T, N[0], N[1],
+                       N[0] >> s, N[1] >> s, N[2] >> s, op->nvox, (const ThrState *)op->dthr);
     MRN_HIP(op, hipGetLastError());
-    MRN_TRY(wavelet3d(op, X, frames, levels, sh, true, st));
+    MRN_TRY(wavelet3d(op, T, frames, levels, sh, true, st, s));
+    if (two) MRN_TRY(wave3_first(op, X, T, frames, sh, true, st));
   }
   return MRN_OK;
+}
+
+// The second image of l1_wavelet_step (grow-only; without the memory the step
+// runs in place).  Never called while capturing with a larger `frames`.
+static void ensure_wave_T(mrn_op *op, int frames) {
+  if (op->wave_T_cap >= (size_t)frames * op->nvox) return;
+  if (grow(op->wave_T, op->wave_T_cap, (int64_t)frames * op->nvox) != hipSuccess) (void)hipGetLastError();
 }
 
 // FISTA's step: shifts for the current iteration from the device counter
@@ -439,6 +684,7 @@ int l1_fista_step(mrn_op *op, float2 *X, hipStream_t st) {
 int l1_wavelet_host(mrn_op *op, float2 *X, int frames, float fraction, const int levels[3], int spins,
                     const int32_t *shifts, double *thr, hipStream_t st) {
   MRN_TRY(ensure_l1_state(op));
+  ensure_wave_T(op, frames);
   if (shifts) {
     MRN_HIP(op, hipMemcpyAsync(op->dsh, shifts, sizeof(int) * 3 * spins, hipMemcpyHostToDevice, st));
   } else {

@@ -108,3 +108,26 @@ def test_l1_fista_matches_oracle(graph):
     X0, _ = op.fista(iters, step, graph=graph)
     Xp, _ = o.fista(smaps, d, traj, iters, step)
     assert rel(X0[0].cpu().numpy(), Xp) < 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,levels", [((20, 34, 12), 4), ((4, 4, 6), 1), ((64, 32, 16), 1), ((84, 18, 10), 3),
+                                      ((15, 32, 16), 2), ((2, 8, 8), 3)])
+def test_l1_step_on_uneven_volumes(n, levels):
+    """The step at partly filled tiles of the three-axis first level, lines
+    shorter than the filter, one level only, and an odd axis (no level there:
+    in place), two frames, against the FP64 oracle; and one forward and inverse
+    transform of the same shifts in place, whose coefficients it thresholds."""
+    op = _op(F=2, N_=n)
+    x = crandn((2, n[2], n[1], n[0]), 17)
+    shifts = orc.spin_shifts(3, 6).reshape(2, 3)
+    X = to_dev(x)
+    thr = op.l1_wavelet(X, 0.5, (levels,) * 3, shifts=shifts.tolist())
+    ref, rthr = orc.l1_wavelet(x, 0.5, (levels,) * 3, shifts, precision="f64")
+    assert abs(thr - rthr) <= 1e-4 * rthr
+    assert rel(X.cpu().numpy(), ref) < 1e-4
+    W = to_dev(x)
+    op.wavelet(W, (levels,) * 3, [int(v) for v in shifts[0]])
+    c = W.cpu().numpy()
+    assert np.float32(op.l1_wavelet(to_dev(x), 0.5, (levels,) * 3, shifts=shifts[:1].tolist())) == \
+        np.float32(orc.fraction_threshold(c, 0.5, precision="f32"))
