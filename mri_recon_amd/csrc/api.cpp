@@ -207,7 +207,7 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
   }
   std::vector<FrameDev> h(F);
   int64_t off = 0, poff = 0;
-  op->fmax_nsub = op->fmax_nheavy = op->fmax_nwide = op->fmax_xsplit = 0;
+  op->fmax_ngrp = op->fmax_nheavy = op->fmax_nwide = op->fmax_xsplit = 0;
   op->fmax_Mv = 0;
   for (int f = 0; f < F; f++) {
     const FrameData &fr = op->frames[f];
@@ -215,6 +215,7 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
     d.coords = fr.coords;
     d.taper = fr.taper;
     d.subs = fr.subs;
+    d.gstart = fr.gstart;
     d.vofs = fr.vofs;
     d.vlist = fr.vlist;
     d.heavy = fr.heavy;
@@ -226,12 +227,12 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
     d.kdata = fr.kdata;
     d.Mv = fr.Mv;
     d.grid_off = (int64_t)f * op->nch * ncell(op) * g.CC;
-    d.nsub = fr.nsub;
+    d.ngrp = fr.ngrp;
     d.nheavy = fr.nheavy;
     d.nwide = fr.nwide;
     d.pad = 0;
     off += fr.Mv * g.CC * op->nch;
-    op->fmax_nsub = std::max(op->fmax_nsub, fr.nsub);
+    op->fmax_ngrp = std::max(op->fmax_ngrp, fr.ngrp);
     op->fmax_nheavy = std::max(op->fmax_nheavy, fr.nheavy);
     op->fmax_nwide = std::max(op->fmax_nwide, fr.nwide);
     op->fmax_xsplit = std::max(op->fmax_xsplit, fr.xsplit_max);

@@ -1136,6 +1136,15 @@ __global__ __launch_bounds__(256) void k_sum_tiles(float2 *grid, const float2 *_
 // per cell.  Sums are FP32; only the order of the additions differs from a
 // per-sample loop.  Each tile is written once with plain stores; a tile split
 // over several work items goes to its items' slots, which k_sum_tiles adds.
+// A wavefront takes a group of consecutive work items (gstart: equal cost,
+// group_cost) as one stream of batches: its visits are one run of the visit
+// list, so the loads of the next items' first batches fly while this item's
+// last ones are summed, and the kernel tables are loaded once per group.  One
+// item per wavefront waited for five dependent loads (item, offset, visits,
+// coordinates, values) for one or two batches of work in sparse k-space.
+// Scatter with one item per wavefront / with groups: 160^3 x 24 coils, 768000
+// samples 1007 / 845 us; 128^3 x 8, 262144 samples 165 / 144; 100 x 84 x 92 x 8
+// 163 / 148; 256^3 x 32, 5.12 M samples 3.86 / 3.69 ms.
 // PAIR (8-coil blocks): a work item takes coil blocks 2 y and 2 y + 1 as its
 // two 16-real blocks, so step A's weights serve both (the second is skipped
 // when nch is odd and y is the last pair).
@@ -1143,9 +1152,10 @@ __global__ __launch_bounds__(256) void k_sum_tiles(float2 *grid, const float2 *_
 template <int CCT, int KM, bool PAIR>
 __global__ __launch_bounds__(256, 4) void k_scatter_mm(
     float2 *__restrict__ grid, const float2 *__restrict__ kin, const float4 *__restrict__ coords,
-    const int64_t *__restrict__ vofs, const int32_t *__restrict__ vlist, const int4 *__restrict__ subs, int nsub,
-    Geom g, Tiles t, const float *__restrict__ tables, int64_t chunk_grid, int64_t chunk_k, int accum,
-    const FrameDev *__restrict__ fdt, const int32_t *__restrict__ xs, int nch, float2 *__restrict__ part) {
+    const int64_t *__restrict__ vofs, const int32_t *__restrict__ vlist, const int4 *__restrict__ subs,
+    const int32_t *__restrict__ gstart, int ngrp, Geom g, Tiles t, const float *__restrict__ tables,
+    int64_t chunk_grid, int64_t chunk_k, int accum, const FrameDev *__restrict__ fdt,
+    const int32_t *__restrict__ xs, int nch, float2 *__restrict__ part) {
   static_assert(CCT == 8 || CCT == 16, "matrix-core scatter needs 8 or 16 coils per cell");
   static_assert(!PAIR || CCT == 8, "coil blocks are paired only at 8 coils");
   constexpr int NB = PAIR ? 2 : CCT / 8;  // 16-real blocks of a cell's coil values (or the pair's blocks)
@@ -1166,28 +1176,56 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
     vofs = fd.vofs;
     vlist = fd.vlist;
     subs = fd.subs;
-    nsub = fd.nsub;
+    gstart = fd.gstart;
+    ngrp = fd.ngrp;
     chunk_k = fd.Mv * g.CC;
     xs = fd.xsplit;
     part = fd.part;
   }
-  const int sidx = scatter_item(blockIdx.x, gridDim.x, wave, t.xrun, xs);
-  if (sidx < 0 || sidx >= nsub) return;
-  const int4 sp = subs[sidx];
-  const int tile = sp.x;
-  const int tix = tile % t.nt[0], tiy = (tile / t.nt[0]) % t.nt[1], tiz = tile / (t.nt[0] * t.nt[1]);
-  const int t0[3] = {tix * 4, tiy * 4, tiz * 4};
+  const int unit = scatter_item(blockIdx.x, gridDim.x, wave, t.xrun, xs);
+  if (unit < 0 || unit >= ngrp) return;
+  const int ibeg = gstart[unit], iend = gstart[unit + 1];
+  if (ibeg >= iend) return;
   const int ch = PAIR ? 2 * (int)blockIdx.y : (int)blockIdx.y;
   const bool have1 = !PAIR || ch + 1 < nch;  // (uniform) the pair's second block exists
   const float *kch = reinterpret_cast<const float *>(kin + ch * chunk_k);
-  const int64_t v0 = vofs[tile];
-  const int32_t *vl = vlist + v0;
-  const int vbeg = max(sp.y, 0), vend = min(sp.z, (int)(vofs[tile + 1] - v0));
   const int sl = lane >> 1, h = lane & 1;    // step A: sample slot, offset pair
   const int ci = lane & 15, kq = lane >> 4;  // step B: cell / real, sample of the group
-  // internal index of visit v of this work item (the last one past the end:
-  // a valid index, so that every lane loads)
-  auto visit = [&](int v) -> int { return vl[min(v, vend - 1)]; };
+  // the stream of batches, each a scalar: its visits n (0 for a tile without
+  // samples), its item k of the group, and whether it is the item's last.  Lane k
+  // holds item k (at most 34 of them: an item costs at least 32 of a group's
+  // 1056), so that no load stands between two items.
+  enum : int { LAST = 1 << 8, VALID = 1 << 9 };
+  const int nit = iend - ibeg;
+  const int4 mine = subs[ibeg + min(lane, nit - 1)];
+  const int first = __builtin_amdgcn_readlane(mine.x, 0);
+  const int32_t *vl = vlist + (vofs[first] + __builtin_amdgcn_readlane(mine.y, 0));
+  int gk = 0, gq = 0, gp = 0;  // item; visits handed out of it, of the group
+  // the next batch, and the internal index of its visit of this lane (past the
+  // end: the last one, a valid index, so that every lane loads)
+  auto gen = [&](int &idx) -> int {
+    idx = 0;
+    if (gk >= nit) return 0;
+    const int len = __builtin_amdgcn_readlane(mine.z, gk) - __builtin_amdgcn_readlane(mine.y, gk);
+    const int n = min(SM_BATCH, len - gq);
+    if (n > 0) idx = vl[gp + min(sl, n - 1)];
+    gp += n;
+    gq += n;
+    int b = n | VALID | (gk << 16);
+    if (gq >= len) {
+      b |= LAST;
+      gk++;
+      gq = 0;
+    }
+    return b;
+  };
+  // origin of a batch's tile
+  auto origin = [&](int b, int (&o)[3]) {
+    const int tile = __builtin_amdgcn_readlane(mine.x, b >> 16);
+    o[0] = (tile % t.nt[0]) * 4;
+    o[1] = ((tile / t.nt[0]) % t.nt[1]) * 4;
+    o[2] = (tile / (t.nt[0] * t.nt[1])) * 4;
+  };
   // coil values of a batch in operand layout: group q, block nb holds real
   // 16 nb + ci of sample 4 q + kq (whose index lane 2 (4 q + kq) holds in
   // idx).  Past the end idx repeats the last visit, whose weights there are
@@ -1218,9 +1256,12 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
   // coordinates of this batch and the next; visit indices of the next two
   float4 kraw = make_float4(0.f, 0.f, 0.f, 0.f), kraw1 = kraw;
   int inext = 0, inext2 = 0;
-  auto batch = [&](int base, const float (&cur)[NG][NB], float (&nxt)[NG][NB]) {
+  int i0, t0[3];
+  int b0 = gen(i0), b1 = gen(inext), b2 = gen(inext2);
+  origin(b0, t0);
+  auto batch = [&](const float (&cur)[NG][NB], float (&nxt)[NG][NB]) {
     // ---- A: weights of the batch
-    const bool ok = base + sl < vend;
+    const bool ok = sl < (b0 & 0xFF);
     const float dk[3] = {kraw.x, kraw.y, kraw.z};
     int lo[3], hi[3];  // the sample's taps as tile offsets [lo, hi] per axis
     bool any = ok;
@@ -1253,11 +1294,11 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
     // ---- ahead: the next batch's coil values, the coordinates of the batch
     // after it (step A of the next batch starts with coordinates loaded one
     // batch earlier still), and the visit indices one batch further on
-    const int nbase = base + SM_BATCH;
-    if (nbase < vend) load_data(inext, nxt);
+    if (b1 & 0xFF) load_data(inext, nxt);
     float4 kraw2 = kraw1;
-    if (nbase + SM_BATCH < vend) kraw2 = *reinterpret_cast<const float4 *>(cb + (uint32_t)inext2 * 16u);
-    const int inext3 = visit(nbase + 2 * SM_BATCH + sl);
+    if (b2 & 0xFF) kraw2 = *reinterpret_cast<const float4 *>(cb + (uint32_t)inext2 * 16u);
+    int inext3;
+    const int b3 = gen(inext3);
     kraw = kraw1;
     kraw1 = kraw2;
     inext = inext2;
@@ -1281,47 +1322,63 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
       }
     }
     wave_sync();
+    if (b0 & LAST) {
+      const int slot = __builtin_amdgcn_readlane(mine.w, b0 >> 16);
+      // (opaque copies: the addresses below are not worth registers in the loop)
+      int cie = ci, kqe = kq;
+      asm volatile("" : "+v"(cie), "+v"(kqe));
+      // accumulator block (p, nb), register r of lane l: cell 16 p + 4 (l / 16) + r,
+      // real 16 nb + l % 16 of the cell's CCT coils (PAIR: real l % 16 of block
+      // ch + nb)
+#pragma unroll
+      for (int p = 0; p < 4; p++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int cx = t0[0] + r, cy = t0[1] + kqe, cz = t0[2] + p;
+          if (cx < g.S[0] && cy < g.S[1] && cz < g.S[2]) {
+            // a split tile's item writes its slot, [nch][64 cells][CCT]
+            const int64_t cell = slot ? (((int64_t)(slot - 1) * nch + ch) * 64 + 16 * p + 4 * kqe + r) * CCT
+                                      : ch * chunk_grid + (((int64_t)cz * g.S[1] + cy) * g.S[0] + cx) * CCT;
+            const int64_t next = slot ? 64 * CCT : chunk_grid;  // PAIR: the second block's cell
+            float *dst = reinterpret_cast<float *>((slot ? part : grid) + cell) + cie;
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) {
+              if (nb > 0 && !have1) continue;
+              const float v = acc[p][nb][r];
+              float *d = PAIR ? dst + nb * 2 * next : dst + 16 * nb;
+              if (accum && !slot) {  // the tile's only work item: a plain read-modify-write
+                *d += v;
+              } else {
+                *d = v;
+              }
+            }
+          }
+        }
+#pragma unroll
+      for (int p = 0; p < 4; p++)
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) acc[p][nb] = mrn_v4f{0.f, 0.f, 0.f, 0.f};
+      origin(b1, t0);
+    }
+    b0 = b1;
+    b1 = b2;
+    b2 = b3;
   };
   float dA[NG][NB], dB[NG][NB];
-  if (vbeg < vend) {
-    const int i0 = visit(vbeg + sl);
-    inext = visit(vbeg + SM_BATCH + sl);
-    inext2 = visit(vbeg + 2 * SM_BATCH + sl);
+#pragma unroll
+  for (int q = 0; q < NG; q++)
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) dA[q][nb] = dB[q][nb] = 0.f;
+  if (b0 & 0xFF) {
     kraw = *reinterpret_cast<const float4 *>(cb + (uint32_t)i0 * 16u);
-    kraw1 = *reinterpret_cast<const float4 *>(cb + (uint32_t)inext * 16u);
     load_data(i0, dA);
   }
-  for (int base = vbeg; base < vend; base += 2 * SM_BATCH) {
-    batch(base, dA, dB);
-    if (base + SM_BATCH >= vend) break;
-    batch(base + SM_BATCH, dB, dA);
+  if (b1 & 0xFF) kraw1 = *reinterpret_cast<const float4 *>(cb + (uint32_t)inext * 16u);
+  while (b0 & VALID) {
+    batch(dA, dB);
+    if (!(b0 & VALID)) break;
+    batch(dB, dA);
   }
-  // accumulator block (p, nb), register r of lane l: cell 16 p + 4 (l / 16) + r,
-  // real 16 nb + l % 16 of the cell's CCT coils (PAIR: real l % 16 of block
-  // ch + nb)
-#pragma unroll
-  for (int p = 0; p < 4; p++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int cx = t0[0] + r, cy = t0[1] + kq, cz = t0[2] + p;
-      if (cx >= g.S[0] || cy >= g.S[1] || cz >= g.S[2]) continue;
-      // a split tile's item writes its slot, [nch][64 cells][CCT]
-      const int64_t cell = sp.w ? (((int64_t)(sp.w - 1) * nch + ch) * 64 + 16 * p + 4 * kq + r) * CCT
-                                : ch * chunk_grid + (((int64_t)cz * g.S[1] + cy) * g.S[0] + cx) * CCT;
-      const int64_t next = sp.w ? 64 * CCT : chunk_grid;  // PAIR: the second block's cell
-      float *dst = reinterpret_cast<float *>((sp.w ? part : grid) + cell) + ci;
-#pragma unroll
-      for (int nb = 0; nb < NB; nb++) {
-        if (nb > 0 && !have1) continue;
-        const float v = acc[p][nb][r];
-        float *d = PAIR ? dst + nb * 2 * next : dst + 16 * nb;
-        if (accum && !sp.w) {  // the tile's only work item: a plain read-modify-write
-          *d += v;
-        } else {
-          *d = v;
-        }
-      }
-    }
 }
 
 // Grid-driven scatter on the vector ALUs (any coil block; the matrix-core
@@ -1344,9 +1401,10 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
 template <int CCT>
 __global__ __launch_bounds__(256, 6) void k_scatter_gd(
     float2 *__restrict__ grid, const float2 *__restrict__ kin, const float4 *__restrict__ coords,
-    const int64_t *__restrict__ vofs, const int32_t *__restrict__ vlist, const int4 *__restrict__ subs, int nsub,
-    Geom g, Tiles t, const float *__restrict__ tables, int64_t chunk_grid, int64_t chunk_k, int accum,
-    const FrameDev *__restrict__ fdt, const int32_t *__restrict__ xs, int nch, float2 *__restrict__ part) {
+    const int64_t *__restrict__ vofs, const int32_t *__restrict__ vlist, const int4 *__restrict__ subs,
+    const int32_t *__restrict__ gstart, int ngrp, Geom g, Tiles t, const float *__restrict__ tables,
+    int64_t chunk_grid, int64_t chunk_k, int accum, const FrameDev *__restrict__ fdt,
+    const int32_t *__restrict__ xs, int nch, float2 *__restrict__ part) {
   __shared__ float s_w[4][SG_BATCH * 12];    // [sample][axis][offset] weights
   __shared__ float2 s_d[4][SG_BATCH * CCT];  // [sample][coil] data
   extern __shared__ float tab_s[];           // kernel tables (g.ntab floats)
@@ -1362,97 +1420,100 @@ __global__ __launch_bounds__(256, 6) void k_scatter_gd(
     vofs = fd.vofs;
     vlist = fd.vlist;
     subs = fd.subs;
-    nsub = fd.nsub;
+    gstart = fd.gstart;
+    ngrp = fd.ngrp;
     chunk_k = fd.Mv * g.CC;
     xs = fd.xsplit;
     part = fd.part;
   }
-  const int sidx = scatter_item(blockIdx.x, gridDim.x, wave, t.xrun, xs);
-  if (sidx < 0 || sidx >= nsub) return;
-  const int4 sp = subs[sidx];
-  const int tile = sp.x;
-  const int tix = tile % t.nt[0], tiy = (tile / t.nt[0]) % t.nt[1], tiz = tile / (t.nt[0] * t.nt[1]);
-  const int t0[3] = {tix * 4, tiy * 4, tiz * 4};
-  const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
+  const int unit = scatter_item(blockIdx.x, gridDim.x, wave, t.xrun, xs);
+  if (unit < 0 || unit >= ngrp) return;
   const int ch = blockIdx.y;
   const float2 *kch = kin + ch * chunk_k;
-  const int64_t v0 = vofs[tile];
-  const int32_t *vl = vlist + v0;
-  const int vbeg = max(sp.y, 0), vend = min(sp.z, (int)(vofs[tile + 1] - v0));
-  float ar[CCT], ai[CCT];
+  const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
+  const int iend = gstart[unit + 1];
+  for (int item = gstart[unit]; item < iend; item++) {
+    const int4 sp = subs[item];
+    const int tile = sp.x;
+    const int tix = tile % t.nt[0], tiy = (tile / t.nt[0]) % t.nt[1], tiz = tile / (t.nt[0] * t.nt[1]);
+    const int t0[3] = {tix * 4, tiy * 4, tiz * 4};
+    const int32_t *vl = vlist + vofs[tile];
+    const int vbeg = sp.y, vend = sp.z;
+    float ar[CCT], ai[CCT];
 #pragma unroll
-  for (int c = 0; c < CCT; c++) ar[c] = ai[c] = 0.f;
-  const int sl = lane >> 2, q = lane & 3;
-  constexpr int CPL = CCT >= 4 ? CCT / 4 : 1;  // coil values a lane stages
-  for (int base = vbeg; base < vend; base += SG_BATCH) {
-    // ---- A: weights and data of the batch
-    const int v = base + sl;
-    const bool ok = v < vend;
-    const int64_t i = vl[min(v, vend - 1)];
-    float2 dv[CPL];
-    if (q * CPL < CCT) {
+    for (int c = 0; c < CCT; c++) ar[c] = ai[c] = 0.f;
+    const int sl = lane >> 2, q = lane & 3;
+    constexpr int CPL = CCT >= 4 ? CCT / 4 : 1;  // coil values a lane stages
+    for (int base = vbeg; base < vend; base += SG_BATCH) {
+      // ---- A: weights and data of the batch
+      const int v = base + sl;
+      const bool ok = v < vend;
+      const int64_t i = vl[min(v, vend - 1)];
+      float2 dv[CPL];
+      if (q * CPL < CCT) {
 #pragma unroll
-      for (int c = 0; c < CPL; c++) dv[c] = kch[i * CCT + q * CPL + c];
+        for (int c = 0; c < CPL; c++) dv[c] = kch[i * CCT + q * CPL + c];
+      }
+      const float4 k = ok ? coords[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float dk[3] = {k.x, k.y, k.z};
+      unsigned long long hit = ~0ull;
+      int sta[3], ena[3];
+      bool oka[3];
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        sta[a] = 0;
+        ena[a] = -1;
+        oka[a] = ok && axis_range(g, a, dk[a], sta[a], ena[a]);
+        // the first NTb taps (the tiles' bin reach); k_scatter_wide adds the rest
+        ena[a] = min(ena[a], sta[a] + t.NTb - 1);
+      }
+      const bool inall = oka[0] && oka[1] && oka[2];
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        const int l = t0[a] + q;
+        const bool in = inall && l >= sta[a] && l <= ena[a];
+        s_w[wave][sl * 12 + a * 4 + q] = in ? tap_weight(g, a, tab_s + g.toff[a], dk[a], l) : 0.0f;
+        unsigned long long m = __ballot(in);
+        m |= m >> 1;
+        m |= m >> 2;
+        hit &= m;  // bit 4s: sample s has a tap in the tile on every axis so far
+      }
+      hit &= 0x1111111111111111ull;
+      if (q * CPL < CCT && ok) {
+#pragma unroll
+        for (int c = 0; c < CPL; c++) s_d[wave][sl * CCT + q * CPL + c] = dv[c];
+      }
+      wave_sync();
+      // ---- B: accumulate the samples that reach the tile
+      while (hit) {
+        const int s = __builtin_ctzll(hit) >> 2;
+        hit &= hit - 1;
+        const float *wp = &s_w[wave][s * 12];
+        const float w = (wp[8 + lz] * wp[4 + ly]) * wp[lx];
+        const float2 *dp = &s_d[wave][s * CCT];
+#pragma unroll
+        for (int c = 0; c < CCT; c++) {
+          const float2 d = dp[c];
+          ar[c] += w * d.x;
+          ai[c] += w * d.y;
+        }
+      }
+      wave_sync();
     }
-    const float4 k = ok ? coords[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float dk[3] = {k.x, k.y, k.z};
-    unsigned long long hit = ~0ull;
-    int sta[3], ena[3];
-    bool oka[3];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      sta[a] = 0;
-      ena[a] = -1;
-      oka[a] = ok && axis_range(g, a, dk[a], sta[a], ena[a]);
-      // the first NTb taps (the tiles' bin reach); k_scatter_wide adds the rest
-      ena[a] = min(ena[a], sta[a] + t.NTb - 1);
-    }
-    const bool inall = oka[0] && oka[1] && oka[2];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      const int l = t0[a] + q;
-      const bool in = inall && l >= sta[a] && l <= ena[a];
-      s_w[wave][sl * 12 + a * 4 + q] = in ? tap_weight(g, a, tab_s + g.toff[a], dk[a], l) : 0.0f;
-      unsigned long long m = __ballot(in);
-      m |= m >> 1;
-      m |= m >> 2;
-      hit &= m;  // bit 4s: sample s has a tap in the tile on every axis so far
-    }
-    hit &= 0x1111111111111111ull;
-    if (q * CPL < CCT && ok) {
-#pragma unroll
-      for (int c = 0; c < CPL; c++) s_d[wave][sl * CCT + q * CPL + c] = dv[c];
-    }
-    wave_sync();
-    // ---- B: accumulate the samples that reach the tile
-    while (hit) {
-      const int s = __builtin_ctzll(hit) >> 2;
-      hit &= hit - 1;
-      const float *wp = &s_w[wave][s * 12];
-      const float w = (wp[8 + lz] * wp[4 + ly]) * wp[lx];
-      const float2 *dp = &s_d[wave][s * CCT];
+    const int cx = t0[0] + lx, cy = t0[1] + ly, cz = t0[2] + lz;
+    if (cx >= g.S[0] || cy >= g.S[1] || cz >= g.S[2]) continue;
+    float2 *dst = sp.w ? part + (((int64_t)(sp.w - 1) * nch + ch) * 64 + lane) * CCT  // a split tile's slot
+                       : grid + ch * chunk_grid + (((int64_t)cz * g.S[1] + cy) * g.S[0] + cx) * CCT;
+    if (accum && !sp.w) {
 #pragma unroll
       for (int c = 0; c < CCT; c++) {
-        const float2 d = dp[c];
-        ar[c] += w * d.x;
-        ai[c] += w * d.y;
+        const float2 o = dst[c];
+        dst[c] = make_float2(o.x + ar[c], o.y + ai[c]);
       }
-    }
-    wave_sync();
-  }
-  const int cx = t0[0] + lx, cy = t0[1] + ly, cz = t0[2] + lz;
-  if (cx >= g.S[0] || cy >= g.S[1] || cz >= g.S[2]) return;
-  float2 *dst = sp.w ? part + (((int64_t)(sp.w - 1) * nch + ch) * 64 + lane) * CCT  // a split tile's slot
-                     : grid + ch * chunk_grid + (((int64_t)cz * g.S[1] + cy) * g.S[0] + cx) * CCT;
-  if (accum && !sp.w) {
+    } else {
 #pragma unroll
-    for (int c = 0; c < CCT; c++) {
-      const float2 o = dst[c];
-      dst[c] = make_float2(o.x + ar[c], o.y + ai[c]);
+      for (int c = 0; c < CCT; c++) dst[c] = make_float2(ar[c], ai[c]);
     }
-  } else {
-#pragma unroll
-    for (int c = 0; c < CCT; c++) dst[c] = make_float2(ar[c], ai[c]);
   }
 }
 
@@ -1853,18 +1914,18 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
   const Tiles &t = op->t;
   // fdt: every frame at once (grid dimension z = frame; the frames' largest
   // work lists size the grid, each frame's kernel reads its own)
-  const int nsub = fdt ? op->fmax_nsub : fr.nsub;
+  const int ngrp = fdt ? op->fmax_ngrp : fr.ngrp;
   const int64_t Mv = fdt ? op->fmax_Mv : fr.Mv;
   int64_t cg = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC, ck = fr.Mv * g.CC;
   // per-XCD ranges (xcd_run < 0): MRN_XCDS workgroup columns, each as long
   // as the longest range needs
   const int xmax = fdt ? op->fmax_xsplit : fr.xsplit_max;
   const bool slabs = t.xrun < 0 && (fdt || fr.xsplit);
-  dim3 g3(slabs ? MRN_XCDS * ((xmax + 3) / 4) : (nsub + 3) / 4, op->nch, fdt ? op->F : 1);
+  dim3 g3(slabs ? MRN_XCDS * ((xmax + 3) / 4) : (ngrp + 3) / 4, op->nch, fdt ? op->F : 1);
   const size_t sh = sizeof(float) * g.ntab;  // kernel tables in LDS
   // no work item: a frame without valid samples whose x passes are limited to
   // its (empty) k-space support -- nothing reads the grid
-  if (nsub == 0) return MRN_OK;
+  if (ngrp == 0) return MRN_OK;
   const bool exact = g.kmode == MRN_KMODE_EXACT_KB;
   // the matrix-core form addresses a coil block's k-space and the coordinates
   // with 32-bit byte offsets
@@ -1876,7 +1937,7 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
     if (pair) gm.y = (unsigned)((op->nch + 1) / 2);
 #define MRN_MM(n, km, pr)                                                                                \
   hipLaunchKernelGGL((k_scatter_mm<n, km, pr>), gm, dim3(256), sh, st, grid, kin, fr.coords, fr.vofs,   \
-                     fr.vlist, fr.subs, fr.nsub, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit, op->nch, op->part)
+                     fr.vlist, fr.subs, fr.gstart, fr.ngrp, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit, op->nch, op->part)
     if (g.CC == 16 && !exact) MRN_MM(16, 0, false);
     else if (g.CC == 16) MRN_MM(16, 1, false);
     else if (pair && !exact) MRN_MM(8, 0, true);
@@ -1889,7 +1950,7 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
 #define MRN_S(n)                                                                                 \
   case n:                                                                                        \
     hipLaunchKernelGGL((k_scatter_gd<n>), g3, dim3(256), sh, st, grid, kin, fr.coords, fr.vofs,  \
-                       fr.vlist, fr.subs, fr.nsub, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit, op->nch, op->part); \
+                       fr.vlist, fr.subs, fr.gstart, fr.ngrp, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit, op->nch, op->part); \
     break;
     MRN_S(1) MRN_S(2) MRN_S(4) MRN_S(8) MRN_S(16)
 #undef MRN_S
@@ -2040,31 +2101,31 @@ __global__ void k_plane_yrange(int2 *xrng, int S1, int S2, int2 *yrng) {
 }
 
 // Cost of scatter work item i (entry n: 0, for the exclusive scan): its
-// visits plus a fixed part for the tile's zeroing and epilogue stores.
+// visits plus a fixed part for the tile's epilogue stores.
 __global__ void k_item_cost(const int4 *__restrict__ subs, int n, int64_t *cost) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) cost[i] = max(subs[i].z - subs[i].y, 0) + 32;
   else if (i == n) cost[i] = 0;
 }
 
-// Boundaries of MRN_XCDS contiguous ranges of the work list of equal cost
-// (pre: exclusive prefix of the costs, n + 1 entries): xs[x] is the first
-// item whose prefix reaches x/MRN_XCDS of the total.  One thread per entry.
-__global__ void k_xcd_split(const int64_t *__restrict__ pre, int n, int32_t *xs) {
-  const int x = threadIdx.x;
-  if (x > MRN_XCDS) return;
-  if (x == 0 || x == MRN_XCDS) {
-    xs[x] = x == 0 ? 0 : n;
-    return;
-  }
-  const int64_t target = pre[n] * x / MRN_XCDS;
-  int lo = 0, hi = n;  // first i in [0, n] with pre[i] >= target
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (pre[mid] >= target) hi = mid;
-    else lo = mid + 1;
-  }
-  xs[x] = lo;
+// Groups of consecutive work items of equal cost (pre: exclusive prefix of the
+// costs): group q starts at the first item whose prefix reaches q * per.  An
+// item longer than `per` leaves empty groups behind it.  start[ngrp] = n.
+__global__ void k_group_start(const int64_t *__restrict__ pre, int n, int64_t per, int ngrp, int32_t *start) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > n) return;
+  const int64_t q1 = i < n ? pre[i] / per : ngrp, q0 = i > 0 ? pre[i - 1] / per : -1;
+  for (int64_t q = q0 + 1; q <= q1; q++) start[q] = i;
+}
+
+// Cost of a group: the list's total over 4 rounds of the chip's 4096 scatter
+// wavefronts, from two items' fixed part to one whole item of MRN_AUTO_MAXV
+// visits (longer groups only lengthen the launch's tail).  Scatter at a cost of
+// 64 / 256 / 1056 / 2112 / this rule: 32^3 x 4 coils 25 / 43 / 124 / 227 / 25 us;
+// 128^3 x 8 165 / 145 / 178 / 248 / 144; 160^3 x 24 1235 / 935 / 827 / 890 / 845;
+// 256^3 x 32 6454 / 4836 / 3774 / 3715 / 3755.
+static int64_t group_cost(int64_t total) {
+  return std::min<int64_t>(std::max<int64_t>(total / (4 * 4096), 64), MRN_AUTO_MAXV + 32);
 }
 
 // Visits per scatter work item when the caller gave none.  A work item is one
@@ -2114,6 +2175,7 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
   fr.nsub = 0;
   fr.nheavy = 0;
   fr.nslots = 0;
+  fr.ngrp = 0;
   fr.M = M;
   MRN_BH(grow(b.keys, b.c_keys, M));
   MRN_BH(grow(b.keys2, b.c_keys2, M));
@@ -2283,7 +2345,7 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
                        fr.subs, nsub_total, fr.vlist);
     MRN_BH(hipGetLastError());
   }
-  // the work list cut into MRN_XCDS ranges of equal cost (xcd_run < 0)
+  // the work list in groups of equal cost, and those in MRN_XCDS ranges (xcd_run < 0)
   {
     const int64_t n = nsub_total;
     MRN_BH(grow(b.icost, b.c_icost, n + 1));
@@ -2295,13 +2357,19 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
     MRN_BH(hipcub::DeviceScan::ExclusiveSum(nullptr, cb, b.icost, b.ipre, (int)n + 1, st));
     MRN_BH(grow(b.vtmp, b.c_vtmp, (int64_t)cb));
     MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.vtmp, cb, b.icost, b.ipre, (int)n + 1, st));
-    hipLaunchKernelGGL(k_xcd_split, dim3(1), dim3(64), 0, st, b.ipre, (int)n, fr.xsplit);
+    int64_t total = 0;
+    MRN_BH(hipMemcpyAsync(&total, b.ipre + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    MRN_BH(hipStreamSynchronize(st));
+    const int64_t per = group_cost(total);
+    fr.ngrp = n > 0 ? (int)(total / per + 1) : 0;
+    MRN_BH(grow(fr.gstart, cp.gstart, (int64_t)fr.ngrp + 1));
+    hipLaunchKernelGGL(k_group_start, dim3(nblk(n + 1, 256)), dim3(256), 0, st, b.ipre, (int)n, per, fr.ngrp, fr.gstart);
     MRN_BH(hipGetLastError());
     int32_t xs[MRN_XCDS + 1];
-    MRN_BH(hipMemcpyAsync(xs, fr.xsplit, sizeof(xs), hipMemcpyDeviceToHost, st));
+    for (int x = 0; x <= MRN_XCDS; x++) xs[x] = (int32_t)((int64_t)fr.ngrp * x / MRN_XCDS);
+    MRN_BH(hipMemcpyAsync(fr.xsplit, xs, sizeof(xs), hipMemcpyHostToDevice, st));
     MRN_BH(hipStreamSynchronize(st));
-    fr.xsplit_max = 0;
-    for (int x = 0; x < MRN_XCDS; x++) fr.xsplit_max = std::max(fr.xsplit_max, xs[x + 1] - xs[x]);
+    fr.xsplit_max = (fr.ngrp + MRN_XCDS - 1) / MRN_XCDS;
   }
   MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.tmp, tb, hflag, hoff, nt + 1, st));
   int32_t nh = 0;

@@ -69,17 +69,18 @@ struct FrameDev {
   const float4 *coords;
   const float *taper;
   const int4 *subs;
+  const int32_t *gstart;   // groups of consecutive work items
   const int64_t *vofs;
   const int32_t *vlist;
   const int4 *heavy;
   const int32_t *wide;
-  const int32_t *xsplit;   // [MRN_XCDS + 1] per-XCD ranges of the scatter work list
+  const int32_t *xsplit;   // [MRN_XCDS + 1] per-XCD ranges of the groups
   float2 *part;            // this frame's split tiles' partial sums
   float2 *kwork;           // this frame's [nch][Mv][CC] k-space work array
   const float2 *kdata;     // measured k-space, same layout
   int64_t Mv;
   int64_t grid_off;        // first element of this frame's coil blocks in the grid
-  int nsub, nheavy, nwide, pad;
+  int ngrp, nheavy, nwide, pad;
 };
 
 // Device arrays that only grow: binding a trajectory no larger than an
@@ -101,7 +102,7 @@ inline hipError_t grow(T *&p, size_t &cap, int64_t n) {
 // Capacities (elements) of a frame's grow-only arrays.
 struct FrameCaps {
   size_t coords = 0, taper = 0, perm = 0, inv = 0, bin_start = 0, subs = 0, heavy = 0, vofs = 0, vlist = 0,
-         gsubs = 0, wide = 0, sparse = 0, xrng = 0, yrng = 0, kdata = 0, kraw = 0, traw = 0, xsplit = 0;
+         gsubs = 0, wide = 0, sparse = 0, xrng = 0, yrng = 0, kdata = 0, kraw = 0, traw = 0, xsplit = 0, gstart = 0;
 };
 
 // Scratch of a trajectory bind, kept by the op between binds (grow-only).
@@ -133,8 +134,10 @@ struct FrameData {
   int32_t *inv = nullptr;      // [M] caller index -> tile order, -1 if skipped
   int32_t *bin_start = nullptr;// [nbins + 1] first sample of each bin
   int4 *subs = nullptr;        // [nsub] {tile, first visit, end visit, 0 or its partial-sum slot + 1}
-  int32_t *xsplit = nullptr;   // [MRN_XCDS + 1] work-list ranges of equal cost, one per XCD
-  int xsplit_max = 0;          // longest of those ranges (work items)
+  int32_t *gstart = nullptr;   // [ngrp + 1] first work item of each group of equal cost (one wavefront each)
+  int ngrp = 0;
+  int32_t *xsplit = nullptr;   // [MRN_XCDS + 1] ranges of those groups, one per XCD
+  int xsplit_max = 0;          // longest of those ranges
   int4 *heavy = nullptr;       // [nheavy] tiles split over several work items {tile, first slot, slots}
   int nsub = 0, nheavy = 0;
   int nslots = 0;              // partial-sum slots of those tiles, [nch][64 cells][CC] each
@@ -186,7 +189,7 @@ struct mrn_op {
   int64_t kwork_all_cap = 0;   // elements
   int2 *xrng_all = nullptr;    // [F][Sz][Sy] x support rows (k_row_xrange) of every frame
   int2 *yrng_all = nullptr;    // [F][Sz] y support of every frame, when the y passes are pruned
-  int fmax_nsub = 0, fmax_nheavy = 0, fmax_nwide = 0, fmax_xsplit = 0;
+  int fmax_ngrp = 0, fmax_nheavy = 0, fmax_nwide = 0, fmax_xsplit = 0;
   int64_t fmax_Mv = 0;
   float2 *kplain = nullptr;    // plain form: one coil of k-space [M_max]
   int64_t kplain_cap = 0;
@@ -469,11 +472,11 @@ __device__ __forceinline__ int xcd_block(int b, int nb, int run) {
   return (b - w) + (w % MRN_XCDS) * run + w / MRN_XCDS;
 }
 
-// Scatter work item of wavefront `wave` (4 per workgroup) of workgroup b.
-// run < 0 with per-XCD ranges xs: the dispatcher deals workgroups to the XCDs
-// in turn, so workgroup b runs on XCD b % MRN_XCDS and takes the next 4 items
-// of that XCD's contiguous range of the work list (tiles in row order): a
-// sample's neighbouring tiles then share one L2.  -1: no item.  Otherwise
+// Scatter work of wavefront `wave` (4 per workgroup) of workgroup b: a group of
+// work items.  run < 0 with per-XCD ranges xs: the dispatcher deals workgroups
+// to the XCDs in turn, so workgroup b runs on XCD b % MRN_XCDS and takes the
+// next 4 groups of that XCD's contiguous range (tiles in row order): a
+// sample's neighbouring tiles then share one L2.  -1: no group.  Otherwise
 // xcd_block's runs (run <= 1: hardware order).
 __device__ __forceinline__ int scatter_item(int b, int nb, int wave, int run, const int32_t *xs) {
   if (run < 0 && xs) {

@@ -445,6 +445,7 @@ int mrn_op_destroy(mrn_op *op) {
     hipFree(fr.bin_start);
     hipFree(fr.subs);
     hipFree(fr.xsplit);
+    hipFree(fr.gstart);
     hipFree(fr.heavy);
     hipFree(fr.vofs);
     hipFree(fr.vlist);

@@ -11,6 +11,7 @@ magnifies each FP32 path's own rounding), within 1.5 times its distance.
 """
 import numpy as np
 import pytest
+import torch
 
 from oracle import oracle as orc
 from mri_recon_amd import GridFFT, MrnError, synth
@@ -369,3 +370,31 @@ def test_padded_coil_blocks(C, block):
     assert op.grid_raw().shape[-1] == block and op.grid().shape[0] == C
     op.close()
     check({}, N, C, 60 + C, forms=("batched",))
+
+
+@pytest.mark.parametrize("C,kw", [(2, {}), (8, {}), (16, {}), (24, {}), (16, {"xcd_run": -1}), (16, {"max_visits": 64})])
+@pytest.mark.parametrize("spokes", [0, 1, 40, 6000])
+def test_groups_of_work_items(C, kw, spokes):
+    """The scatter takes its work items in groups of equal cost, one wavefront
+    each: no samples at all, one spoke (a handful of items among tiles without
+    samples, several to a group), and spokes enough that an item fills a group
+    (8 to 12 thousand visits in the centre tiles).  A^H, twice (overwriting, and
+    adding into the image), against the vector-ALU form's, to FP32 rounding."""
+    N = 32
+    traj = [t.cuda() for t in synth.radial_traj(max(spokes, 1), N, N)]
+    if spokes == 0:
+        traj[3] = torch.zeros_like(traj[3])  # every sample skipped
+    smaps = synth.coil_maps(C, N, seed=3).cuda()
+    d = synth.cn_image((C, traj[0].numel()), seed=4).cuda()
+    out = []
+    for valu in (False, True):
+        op = GridFFT(N, ncoils=C, scatter_valu=valu, **kw)
+        op.set_traj(*traj)
+        op.set_smaps(smaps)
+        h = op.forward(d, accumulate=False)
+        out.append(op.forward(d, X=h).cpu().numpy())
+        op.close()
+    if spokes == 0:
+        assert np.count_nonzero(out[0]) == 0 and np.count_nonzero(out[1]) == 0
+    else:
+        assert rel(out[0], out[1]) <= 1e-6
