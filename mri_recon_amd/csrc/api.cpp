@@ -939,7 +939,9 @@ int mrn_get_tuning(const mrn_op *op, mrn_tuning *out) {
   out->max_visits = op->t.maxv;
   out->xcd_run = op->t.xrun;
   out->xcd_run_gather = op->t.xrun_gather;
-  out->gather_coils = op->gather_coils > 0 ? std::min(op->gather_coils, op->g.CC) : std::min(4, op->g.CC);
+  int64_t Mv = 0;
+  for (const auto &fr : op->frames) Mv = std::max(Mv, fr.Mv);
+  out->gather_coils = gather_coils(op, Mv);
   out->xcd_run_fft = op->xcd_run_fft;
   out->fft_stockham = op->fft_stockham ? 1 : 0;
   out->scatter_valu = (op->scatter_valu || (op->g.CC != 16 && op->g.CC != 8)) ? 1 : 0;

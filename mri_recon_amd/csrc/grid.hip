@@ -1816,6 +1816,24 @@ static int launch_gather_box(mrn_op *op, const float2 *grid, float2 *out, const 
   return MRN_OK;
 }
 
+// Coils per lane of the direct gather over n samples.  The gather is bound by
+// the L1, whose loads take a lane's coils at once: at 16-coil blocks 4 per lane
+// are best, since a wave then serves 16 samples whose taps overlap; a narrower
+// block's samples are a shorter run of one line, and 2 per lane are (the wider
+// lane asks for more bytes per line than the L1 returns per clock).  us with 1 / 2 / 4
+// coils per lane: 256^3 x 32 (16-coil blocks) 10038 / 5822 / 5640; 128^3 x 8 (8)
+// 136 / 126 / 146; 200^3 x 20 (8) 3614 / 2217 / 2368; 256^3 x 4 (4) 1341 / 895 /
+// 1112; 160^3 x 4 292 / 243 / 338; 160^3 x 2 161 / 155.  Fewer per lane where
+// that leaves under four waves to a CU: 32^3, 8192 samples, x 4 coils 13 / 15 /
+// 36; x 16 19 / 17 / 20.  Same bits with all.
+int gather_coils(const mrn_op *op, int64_t n) {
+  const int CC = op->g.CC;
+  if (op->gather_coils > 0) return op->gather_coils < CC ? op->gather_coils : CC;
+  int nc = CC >= 16 ? 4 : CC >= 2 ? 2 : 1;
+  while (nc > 1 && n * op->nch * (CC / nc) < 1024 * 64) nc /= 2;
+  return nc;
+}
+
 // Direct gather over all samples, or over the samples listed in `list`.
 // fdt: every frame of the op at once (op->fdev; out, sub from the table, sub
 // when fsub), grid dimension z = frame.
@@ -1823,14 +1841,9 @@ static int launch_gather_direct(mrn_op *op, const float2 *grid, float2 *out, con
                                 const float2 *sub, int wflag, const int32_t *list, int64_t nlist,
                                 hipStream_t st, const FrameDev *fdt = nullptr, int fsub = 0) {
   const Geom &g = op->g;
-  // coils per lane: 4 by default.  A wave then serves 16 samples (4 lanes
-  // each) instead of 8, whose taps overlap more, so fewer of its loads miss
-  // the L1 (16-coil blocks at 256^3, pipelined rows: 5.5 ms with 4 coils per
-  // lane, 5.7 with 2, 7.5 with 8)
-  int nc = op->gather_coils > 0 ? op->gather_coils : 4;
-  if (nc > g.CC) nc = g.CC;
   const int64_t n = fdt ? op->fmax_Mv : list ? nlist : fr.Mv;
   if (n == 0) return MRN_OK;
+  const int nc = gather_coils(op, fdt ? n * op->F : n);
   dim3 g3(nblk(n * (g.CC / nc), 256), op->nch, fdt ? op->F : 1);
   int64_t cg = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC, ck = fr.Mv * g.CC;
   switch (taps_main(g) * 16 + nc) {

@@ -531,6 +531,7 @@ struct PrePostArgs {
 int taps_main(const Geom &g);
 
 // host-side launchers (defined in the .hip files)
+int gather_coils(const mrn_op *op, int64_t n);
 int launch_gather(mrn_op *op, const float2 *grid, float2 *out, const FrameData &fr, const float2 *sub,
                   bool weighted, hipStream_t st);
 int launch_weight(mrn_op *op, float2 *kout, const float2 *kin, const FrameData &fr, hipStream_t st);
