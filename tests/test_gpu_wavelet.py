@@ -131,3 +131,58 @@ def test_l1_step_on_uneven_volumes(n, levels):
     c = W.cpu().numpy()
     assert np.float32(op.l1_wavelet(to_dev(x), 0.5, (levels,) * 3, shifts=shifts[:1].tolist())) == \
         np.float32(orc.fraction_threshold(c, 0.5, precision="f32"))
+
+
+def _bisect(c, fraction):
+    """The fraction threshold by plain counting, one float32 step at a time; a
+    NaN is below nothing and no extreme."""
+    with np.errstate(all="ignore"):
+        a = np.sqrt(c.real.astype(np.float64) ** 2 + c.imag.astype(np.float64) ** 2).astype(np.float32).ravel()
+        h, n = np.float32(0.5), a.size
+        mn, mx = np.nanmin(a), np.nanmax(a)
+        target, acc = int(np.float64(np.float32(fraction)) * n), int(0.001 * n)
+        v, hi, lo = h * (mx - mn), np.float32(fraction) * mx, mn
+        if target < 2:
+            return np.float32(0)
+        for it in range(1, 65):
+            found = int(np.count_nonzero(a < v))
+            if abs(found - target) <= acc or it == 64:
+                break
+            if found > target:
+                hi = v
+            else:
+                lo = v
+            v = h * (hi + lo)
+    return v
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("levels", [(3, 3, 3), (3, 1, 2), (2, 3, 2)])
+@pytest.mark.parametrize("fraction,scale,bad", [(0.02, 1.0, None), (0.4, 1e-25, None), (0.9, 1e25, None),
+                                                (0.97, 1.0, np.nan), (0.5, 1.0, np.inf), (0.5, 0.0, None)])
+def test_threshold_counts_all_values(levels, fraction, scale, bad):
+    """The histogram over sorted candidates counts what a comparison per candidate
+    counts: fractions that put the first value above the bracket, magnitudes
+    whose squares leave float32, a NaN, an infinity, equal values; axes with
+    levels that others do not have (finished in place).  The same bits as one
+    float32 step at a time on the device's coefficients."""
+    x = crandn((2, N, N, N), 9) * np.float32(scale)
+    if bad is not None:
+        x[1, 3, 4, 5] = bad
+    sh = ((1, 2, 3),)
+    op = _op(F=2)
+    X = to_dev(x)
+    thr = op.l1_wavelet(X, fraction, levels, shifts=sh)
+    W = to_dev(x)
+    op.wavelet(W, levels, sh[0])
+    c = W.cpu().numpy()
+    ref = _bisect(c, fraction)
+    assert np.float32(thr) == ref or (np.isnan(thr) and np.isnan(ref))
+    if bad is None:  # and the step: threshold on those coefficients, transformed back
+        a = np.sqrt(c.real.astype(np.float64) ** 2 + c.imag.astype(np.float64) ** 2).astype(np.float32)
+        with np.errstate(all="ignore"):
+            f = np.where(a <= ref, np.float32(0), np.float32(1) - ref / a)
+        W = to_dev((c * f).astype(np.complex64))
+        op.wavelet(W, levels, sh[0], inverse=True)
+        got, want = X.cpu().numpy().astype(np.complex128), W.cpu().numpy().astype(np.complex128)
+        assert rel(got, want) <= 1e-6
