@@ -1520,18 +1520,22 @@ __global__ __launch_bounds__(256, 6) void k_scatter_gd(
 // The samples with more than NTb taps on some axis (fr.wide): the tile
 // scatter adds their first NTb taps on every axis (the box its bins reach),
 // and this kernel adds the rest -- the taps past that box, on the window's far
-// edge -- with float atomics after the tiles are written.  Thread = (listed
-// sample, tap past the box, coil) of coil block blockIdx.y: such samples sit
+// edge -- with float atomics after the tiles are written.  Such samples sit
 // exactly on a window edge, so the list is short (often empty) and a thread per
-// sample walking its taps was all latency.  The taps past the NTb^3 box of an
-// NT^3 one: the planes z >= NTb, then the rows y >= NTb, then the cells
-// x >= NTb.  128^3 x 8 coils, W = 4: 28 us before, 5.4 now; 100 x 84 x 92 x 8,
-// W = 5: 43, 4.7.
-__global__ __launch_bounds__(256) void k_scatter_wide(float2 *grid, const float2 *__restrict__ kin,
-                                                      const float4 *__restrict__ coords,
-                                                      const int32_t *__restrict__ wide, int nwide, Geom g, int NT,
-                                                      int NTb, const float *__restrict__ tables, int64_t chunk_grid,
-                                                      int64_t chunk_k, const FrameDev *__restrict__ fdt) {
+// sample walking its taps was all latency.  A sample's NT^3 window holds one
+// cell of every class (x, y, z) mod NT: a wavefront takes a class and up to
+// WIDE_CHUNK listed samples, lanes = (sample, coil) of coil block blockIdx.y,
+// in list order, so that all that such a list adds to a cell comes from one
+// wavefront in one order.  Most of a list is one point, the centre that every
+// readout passes: samples at the position of the chunk's middle one are summed
+// first and added once.  128^3 x 8 coils, W = 4: 28 us before, 7.5 now;
+// 100 x 84 x 92 x 8, W = 5: 43, 5.8.
+#define WIDE_CHUNK 512
+__global__ __launch_bounds__(64) void k_scatter_wide(float2 *grid, const float2 *__restrict__ kin,
+                                                     const float4 *__restrict__ coords,
+                                                     const int32_t *__restrict__ wide, int nwide, Geom g, int NT,
+                                                     int NTb, const float *__restrict__ tables, int64_t chunk_grid,
+                                                     int64_t chunk_k, const FrameDev *__restrict__ fdt) {
   if (fdt) {  // every frame at once: frame blockIdx.z
     const FrameDev &fd = fdt[blockIdx.z];
     grid += fd.grid_off;
@@ -1541,45 +1545,73 @@ __global__ __launch_bounds__(256) void k_scatter_wide(float2 *grid, const float2
     nwide = fd.nwide;
     chunk_k = fd.Mv * g.CC;
   }
-  const int d = NT - NTb, nz = d * NT * NT, ny = NTb * d * NT, ntap = nz + ny + NTb * NTb * d;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t st = idx >> g.lgCC;
-  if (st >= (int64_t)nwide * ntap) return;
-  const int c = (int)(idx & (g.CC - 1));
-  int q = (int)(st % ntap), o[3];  // tap, as offsets from the first one
-  if (q < nz) {
-    o[2] = NTb + q / (NT * NT);
-    o[1] = (q / NT) % NT;
-    o[0] = q % NT;
-  } else if (q < nz + ny) {
-    q -= nz;
-    o[2] = q / (d * NT);
-    o[1] = NTb + (q / NT) % d;
-    o[0] = q % NT;
-  } else {
-    q -= nz + ny;
-    o[2] = q / (NTb * d);
-    o[1] = (q / d) % NTb;
-    o[0] = NTb + q % d;
-  }
-  const int64_t i = wide[st / ntap];
-  const int ch = blockIdx.y;
-  const float4 k = coords[i];
-  const float dk[3] = {k.x, k.y, k.z};
-  int l[3];
+  const int ncls = NT * NT * NT, q = (int)(blockIdx.x % ncls);
+  const int n0 = (int)(blockIdx.x / ncls) * WIDE_CHUNK, n1 = min(n0 + WIDE_CHUNK, nwide);
+  if (n0 >= n1) return;  // (uniform) a shorter frame
+  const int r[3] = {q % NT, (q / NT) % NT, q / (NT * NT)};
+  const int c = (int)threadIdx.x & (g.CC - 1), ch = blockIdx.y;
+  kin += ch * chunk_k + c;
+  grid += ch * chunk_grid + c;
+  // a sample's cell of this class (offset into grid), if it is past the box
+  auto tap = [&](const float4 k, int64_t &at, int (&l)[3]) -> bool {
+    const float dk[3] = {k.x, k.y, k.z};
+    bool past = false;
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
-    int s, e;
-    if (!axis_range(g, a, dk[a], s, e)) return;
-    l[a] = s + o[a];
-    if (l[a] > e) return;
+    for (int a = 0; a < 3; a++) {
+      int s, e;
+      if (!axis_range(g, a, dk[a], s, e)) return false;
+      const int m = (r[a] - s) % NT, o = m < 0 ? m + NT : m;
+      l[a] = s + o;
+      if (l[a] > e) return false;
+      past = past || o >= NTb;
+    }
+    at = (((int64_t)l[2] * g.S[1] + l[1]) * g.S[0] + l[0]) * g.CC;
+    return past;
+  };
+  auto weight = [&](const float4 k, const int (&l)[3]) {
+    const float wzy = tap_weight(g, 2, tables + g.toff[2], k.z, l[2]) * tap_weight(g, 1, tables + g.toff[1], k.y, l[1]);
+    return wzy * tap_weight(g, 0, tables + g.toff[0], k.x, l[0]);
+  };
+  const float4 rk = coords[wide[(n0 + n1) >> 1]];
+  int64_t at, rat;
+  int l[3], rl[3];
+  const bool rin = tap(rk, rat, rl);
+  float2 sum = make_float2(0.f, 0.f);
+  constexpr int U = 4;  // samples per lane in flight
+  const int step = 64 >> g.lgCC;
+  for (int s0 = n0 + (int)(threadIdx.x >> g.lgCC); s0 < n1; s0 += U * step) {
+    int64_t i[U];
+    float4 k[U];
+    float2 v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) i[u] = wide[min(s0 + u * step, n1 - 1)];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      k[u] = coords[i[u]];
+      v[u] = kin[i[u] * g.CC];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (s0 + u * step >= n1) continue;
+      if (k[u].x == rk.x && k[u].y == rk.y && k[u].z == rk.z) {
+        sum.x += v[u].x;
+        sum.y += v[u].y;
+      } else if (tap(k[u], at, l)) {
+        const float w = weight(k[u], l);
+        atomicAdd(&grid[at].x, w * v[u].x);
+        atomicAdd(&grid[at].y, w * v[u].y);
+      }
+    }
   }
-  const float wzy = tap_weight(g, 2, tables + g.toff[2], dk[2], l[2]) * tap_weight(g, 1, tables + g.toff[1], dk[1], l[1]);
-  const float w = wzy * tap_weight(g, 0, tables + g.toff[0], dk[0], l[0]);
-  const float2 v = kin[ch * chunk_k + i * g.CC + c];
-  float2 *cell = grid + ch * chunk_grid + (((int64_t)l[2] * g.S[1] + l[1]) * g.S[0] + l[0]) * g.CC + c;
-  atomicAdd(&cell->x, w * v.x);
-  atomicAdd(&cell->y, w * v.y);
+  if (!rin) return;  // (uniform)
+  for (int h = g.CC; h < 64; h <<= 1) {
+    sum.x += __shfl_xor(sum.x, h);
+    sum.y += __shfl_xor(sum.y, h);
+  }
+  if ((int)threadIdx.x >= g.CC) return;
+  const float w = weight(rk, rl);
+  atomicAdd(&grid[rat].x, w * sum.x);
+  atomicAdd(&grid[rat].y, w * sum.y);
 }
 
 // wide[i] = 1 when valid sample i has more than NTb taps on some axis
@@ -2000,8 +2032,8 @@ int launch_scatter_wide(mrn_op *op, float2 *grid, const float2 *kin, const mrn::
   if (nwide > 0) {
     const int64_t cg = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC, ck = fr.Mv * g.CC;
     const int NT = op->t.NT, NTb = op->t.NTb;
-    const int64_t n = (int64_t)nwide * (NT * NT * NT - NTb * NTb * NTb) * g.CC;  // NT > NTb, or there are no wide samples
-    hipLaunchKernelGGL(k_scatter_wide, dim3(nblk(n, 256), op->nch, fdt ? op->F : 1), dim3(256), 0, st, grid, kin,
+    const int64_t n = (int64_t)((nwide + WIDE_CHUNK - 1) / WIDE_CHUNK) * NT * NT * NT;
+    hipLaunchKernelGGL(k_scatter_wide, dim3((unsigned)n, op->nch, fdt ? op->F : 1), dim3(64), 0, st, grid, kin,
                        fr.coords, fr.wide, fr.nwide, g, NT, NTb, op->tables_d, cg, ck, fdt);
     MRN_HIP(op, hipGetLastError());
   }

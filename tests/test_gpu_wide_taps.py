@@ -53,3 +53,25 @@ def test_window_edge_samples(dwin, C, kw):
     ea = rel(a, o32.image_to_kspace(X, smaps, traj))
     print("dwin %.1f C=%d %s: A^H %.2e A %.2e" % (dwin, C, kw, eh, ea))
     assert eh <= 1e-5 and ea <= 1e-5
+
+
+@pytest.mark.parametrize("C,spokes", [(1, 300), (5, 480), (16, 40), (16, 480), (8, 513), (2, 1300)])
+def test_centre_of_many_readouts(C, spokes):
+    """Every readout starts at k = 0, a window edge at dwin = 2: most listed
+    samples are one point, summed before they are added, in chunks of 512; the
+    first readout runs along kz, an edge on x and y whose cells are the centre's
+    too.  Against the oracle, and the same bits on every call where the list fits
+    one chunk."""
+    N = 32
+    traj = [t.numpy() for t in synth.radial_traj(spokes, 24, N)]
+    traj[3] = np.maximum(traj[3], 0.5).astype(np.float32)  # the centre takes part
+    smaps = synth.coil_maps(C, N, seed=5).numpy()
+    d = crandn((C, traj[0].size), 7)
+    op = GridFFT(N, ncoils=C, overgrid=1.5, dwin=2.0)
+    op.set_traj(*traj_dev(traj))
+    op.set_smaps(to_dev(smaps))
+    h = [op.forward(to_dev(d), accumulate=False).cpu().numpy() for _ in range(5)]
+    if spokes + 23 <= 512:
+        assert all(np.array_equal(h[0], x) for x in h[1:])
+    o32 = orc.OracleOp(N, overgrid=1.5, dwin=2.0, precision="f32")
+    assert rel(h[0], o32.kspace_to_image(d, smaps, traj)) <= 1e-5
