@@ -183,8 +183,10 @@ __global__ void k_widen(const int32_t *__restrict__ v, int n, int64_t *out) {
 // load.  One wavefront per scatter work item (a tile's visits [sp.y, sp.z),
 // at most maxv of them, so that a dense tile's list is written by several
 // wavefronts), one lane per bin row: the lanes' run lengths are loaded
-// together and scanned, then the wavefront writes the runs' parts inside its
-// range one after the other, 64 consecutive entries per store.
+// together and scanned, then the wavefront writes 64 consecutive entries per
+// step, each lane looking up the row of its own (8 shuffles).  Writing the runs
+// one after the other took up to 64 turns of a few lanes each where rows are
+// short.  192^3, 4.19 M samples: 462 us before, 142 now.
 __global__ void k_fill_visits(const int32_t *__restrict__ bin_start, Tiles t, const int64_t *__restrict__ vofs,
                               const int4 *__restrict__ subs, int nsub, int32_t *vlist) {
   const int item = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -216,16 +218,18 @@ __global__ void k_fill_visits(const int32_t *__restrict__ bin_start, Tiles t, co
       const int y = __shfl_up(x, off);
       if (lane >= off) x += y;
     }
-    // row k's run: start sk, length nk, tile visits [ek, ek + nk); the part
-    // inside [vb, ve) is written by the whole wavefront, lane q taking
-    // entries q, q + 64, ... of it
-    const int nr = min(64, nrows - r0);
-    for (int k = 0; k < nr; k++) {
-      const int nk = __shfl(n, k), sk = __shfl(s0, k), ek = g0 + __shfl(x, k) - nk;
-      const int lo = max(ek, vb), hi = min(ek + nk, ve);
-      for (int q = lo + lane; q < hi; q += 64) vlist[o + q] = sk + (q - ek);
+    // the part of this group's visits inside [vb, ve), 64 consecutive entries
+    // at a time: entry q belongs to the first row whose prefix is beyond it
+    const int tot = __shfl(x, 63), lo = max(g0, vb), hi = min(g0 + tot, ve);
+    for (int q0 = lo; q0 < hi; q0 += 64) {  // (uniform: every lane takes part in the shuffles)
+      const int q = q0 + lane, rel = min(q, hi - 1) - g0;
+      int k = 0;
+#pragma unroll
+      for (int h = 32; h > 0; h >>= 1) k += __shfl(x, k + h - 1) <= rel ? h : 0;
+      const int v = __shfl(s0, k) + rel - __shfl(x - n, k);
+      if (q < hi) vlist[o + q] = v;
     }
-    g0 += __shfl(x, 63);
+    g0 += tot;
   }
 }
 
