@@ -2200,7 +2200,7 @@ static int64_t group_cost(int64_t total) {
 // wavefront's serial walk (2.4 us per batch of 32 visits), so a dense tile's
 // item must not outlast the rest of the launch; the chip holds about 4096
 // scatter wavefronts.  Hence the frame's visits over 4096, in whole batches:
-// at least 64 (below it the split tiles' atomics cost more than the shorter
+// at least 64 (below it the split tiles' partial sums cost more than the shorter
 // walks save) and at most 1024 (more gains nothing at 41 M visits).
 // Scatter at 64 / 256 / 1024 / 4096 visits per item: 32^3 x 8 coils, 8192
 // samples 23 / 33 / 74 / 86 us; 128^3 x 8, 262144 samples 180 / 169 / 179 /
