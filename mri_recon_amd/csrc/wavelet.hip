@@ -557,8 +557,8 @@ __global__ __launch_bounds__(THR_THREADS) void k_thr_minmax(const float2 *__rest
 // A thread looks its value up among the sorted candidates (LDS, 6 steps) and
 // adds to its lane's column of a histogram, so no two lanes of a wave meet on an
 // address; the last workgroup sums up and steps.  Against 15 candidates, each
-// compared with every value, and a division-free store of |c| in place of its root
-// per pass: 12.6 M values, 82 us per pass of 4 steps before, 25 to 40 of 6 now.
+// compared with every value, and |c| computed anew on each pass (its root in double):
+// 12.6 M values, 82 us per pass of 4 steps before, 25 to 40 per pass of 6 now.
 template <typename V>
 __global__ __launch_bounds__(THR_THREADS) void k_thr_count(const V *__restrict__ X, int64_t n, ThrState *s, float scale,
                                                            double *log, const int *counter, int cap) {
