@@ -441,6 +441,13 @@ __global__ __launch_bounds__(64) void k_llr_reg(float2 *__restrict__ X, LlrGeom 
       gi[i] += ar * xi - ai * xr;
     });
   });
+  // A NaN voxel makes its frame's row and column of G NaN.  k_llr_block never
+  // rotates such a pair and its column keeps a factor of 0, so the NaN stays at
+  // its voxel; here idle pairs are multiplied by 1 and 0, and 0 * NaN would
+  // carry it to every frame of the block.  As zeros those entries do nothing.
+#pragma unroll
+  for (int i = 0; i < NL; i++)
+    if (gr[i] != gr[i] || gi[i] != gi[i]) gr[i] = gi[i] = 0.0;
   // 2. Jacobi sweeps
   double vr[THRESH ? NL : 1], vi[THRESH ? NL : 1];
   if constexpr (THRESH) {

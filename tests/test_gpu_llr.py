@@ -72,6 +72,30 @@ def test_llr_update_only_and_huge_threshold():
     assert llr_threshold(Z, alpha_time=0.1) == 0.0 and torch.count_nonzero(Z).item() == 0
 
 
+@pytest.mark.parametrize("Nt", [2, 4, 5, 8, 10, 20])
+@pytest.mark.parametrize("shape,block", [((20, 22, 24), (2, 2, 2)), ((8, 12, 16), (4, 4, 4)), ((16, 8, 8), (8, 8, 8))])
+def test_llr_nan_stays_at_its_voxel(Nt, shape, block):
+    """A NaN voxel of one frame: the other frames of its block come out as if
+    that frame were zero there, the frame itself becomes zero in the block, the
+    voxel is NaN in every frame, and the block still counts for the threshold."""
+    X = lowrank_frames(Nt, 1, shape, seed=30 + Nt)
+    f, (z, y, x) = Nt // 2, (5, 6, 7)
+    kw = dict(block=block, block_iter=1, alpha_time=0.05)
+    Z = X.copy()
+    at = tuple(slice(v // b * b, v // b * b + b) for v, b in zip((z, y, x), block[::-1]))
+    Z[(f, 0) + at] = 0
+    ref, rsmax = orc.llr(orc.llr_params(**kw), Z, 0, 3, 5, "f32")
+    X[f, 0, z, y, x] = complex(np.nan, 0.25)
+    Xd = to_dev(X)
+    smax = llr_threshold(Xd, dim=0, iteration=3, call=5, **kw)
+    got = Xd.cpu().numpy()
+    bad = np.zeros(X.shape, bool)
+    bad[:, 0, z, y, x] = True
+    assert np.array_equal(np.isnan(got), bad)
+    assert abs(smax - rsmax) <= 1e-6 * rsmax
+    assert rel(got[~bad], ref[~bad]) <= 1e-5
+
+
 def test_llr_errors_and_flags():
     X = torch.zeros((40, 1, 8, 8, 8), dtype=torch.complex64, device="cuda")
     with pytest.raises(MrnError, match="32 frames"):
