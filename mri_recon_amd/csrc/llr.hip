@@ -3,9 +3,9 @@
 // recon_lib calls them after each gradient step (recon_lib.cpp:2117-2126).
 //
 // Block b of a pass is the Np x N matrix A (N = frames along `dim`, Np = the
-// other frames x block voxels).  Up to 8 frames go 8 or 16 blocks to a
-// wavefront with the matrices in registers (k_llr_reg); more take a wavefront,
-// or half of one, per block:
+// other frames x block voxels).  Up to 8 frames with enough small blocks go 8
+// or 16 blocks to a wavefront with the matrices in registers (k_llr_reg,
+// llr_in_registers); others take a wavefront, or half of one, per block:
 //   1-2. G = A^H A in FP64, A's rows streamed through LDS one chunk of LPB
 //      rows at a time (periodic wrap, the pass's shift), so a block holds
 //      N x (LPB + 1) values of A in LDS instead of all Np rows;
@@ -399,7 +399,7 @@ __global__ __launch_bounds__(64) void k_llr_reg(float2 *__restrict__ X, LlrGeom 
   const int nother = g.dim == 0 ? g.Ne : g.Nt;
   // this lane's column: frame j of the low-rank dimension
   const bool col = j < N;
-  // f(voxel address of this lane's frame) for the block's rows, LLR_STEP at a
+  // f(voxel address of this lane's frame) for the block's rows, STEP at a
   // time (every lane of a wavefront walks the same number)
   constexpr int STEP = 4;
   auto rows = [&](auto &&f) {
@@ -695,6 +695,35 @@ static int llr_geom(const mrn_llr_params *p, int Nt, int Ne, const int32_t N[3],
 static size_t llr_lds(const LlrGeom &g) { return (size_t)g.lds_block * (64 / g.lpb); }
 static long long llr_blocks(const LlrGeom &g) { return (long long)g.nb[0] * g.nb[1] * g.nb[2]; }
 
+// Whether a pass takes k_llr_reg.  Its 4 or 8 lanes walk a block's rows one
+// after the other, so it has to have blocks enough to hide that walk: with few
+// or long ones the row-parallel form above is up to 3 times as fast.  Measured
+// with 2 passes, k_llr_block / k_llr_reg in us:
+//   rows     8: 512 blocks x 1, 4, 8 frames 226 / 229, 278 / 226, 416 / 250
+//   rows    27: 125 blocks x 2, 5, 8 208 / 230, 253 / 262, 327 / 271; 1000 blocks 247 / 224, 349 / 268, 437 / 274
+//   rows    64: 4096 blocks x 1, 3, 5, 8 226 / 264, 290 / 283, 378 / 403, 502 / 447; 13824 blocks x 3, 5, 8
+//               414 / 318, 634 / 476, 1010 / 551; 32768 blocks x 1 360 / 312
+//   rows   125: 1728 blocks x 3, 8 293 / 353, 512 / 548; 6859 386 / 409, 741 / 625; 15625 530 / 429, 1250 / 732
+//   rows   216: 9261 blocks x 3, 5, 8 491 / 555, 672 / 824, 1159 / 901; 32768 x 3, 5, 6, 8 1011 / 643, 1508 / 1532,
+//               1741 / 1621, 2797 / 1737; 50653 x 1 860 / 701
+//   rows   512: 4096 blocks x 3, 8 490 / 791, 945 / 1303; 13824 x 8 2364 / 1944; 32768 x 3, 5, 7, 8 1744 / 1567,
+//               2424 / 3410, 3489 / 4132, 4767 / 4217
+//   rows  1000: 15625 blocks x 3, 5 1672 / 2070, 2309 / 3221; 4096: 512 blocks x 1, 4, 8 1305 / 4145, 1971 / 4677,
+//               3982 / 6805
+// (5 and 6 frames fill 8 lanes least, and one or two frames give the rotations
+// nothing to win.)
+static bool llr_in_registers(const LlrGeom &g) {
+  const int N = g.N;
+  const long long n = g.nblk;
+  if (N > 8) return false;
+  if (g.Np <= 32) return N >= 7 || n >= 1000;
+  if (g.Np <= 64 && N >= 7) return true;
+  if (g.Np <= 128) return n >= (N <= 2 ? 32768 : 12288);
+  if (g.Np <= 256) return N != 5 && n >= (N >= 7 ? 12288 : 32768);
+  if (g.Np <= 512) return (N <= 4 && n >= 32768) || (N == 8 && n >= 12288);
+  return false;
+}
+
 // update_threshold + thresh on stream st.  Scratch: sblocks [nblocks] doubles,
 // sel (SelState), tau (1 double), smax (1 float), all device.  counter: FISTA's
 // device iteration counter (iteration = *counter - 1, also the call index of
@@ -707,7 +736,7 @@ static hipError_t llr_launch(const LlrGeom &g, float2 *X, float alpha, float amp
   const size_t lds = llr_lds(g);
   const unsigned nwg = (unsigned)((nblk + (64 / g.lpb) - 1) / (64 / g.lpb));
   auto blocks = [&](bool thresh, int pass) {
-    if (g.N <= 8) {  // 4 or 8 lanes per block, in registers
+    if (llr_in_registers(g)) {  // 4 or 8 lanes per block
       const int nl = g.N <= 4 ? 4 : 8;
       const unsigned nw = (unsigned)((nblk + 64 / nl - 1) / (64 / nl));
 #define LLR_REG(T, n)                                                                                          \

@@ -36,6 +36,22 @@ CASES = [
     # block rows stream through LDS in chunks of 32 or 64: more rows than fit at once
     (4, 1, (16, 16, 16), 0, (16, 16, 16), 2, 0.1),  # one block of 4096 rows
     (6, 2, (8, 8, 16), 0, (8, 8, 8), 2, 0.05),      # 2 encodes x 512 voxels per block row set
+    # up to 8 frames in registers: 1000 blocks of at most 32 rows on, and one block fewer
+    (1, 1, (20, 20, 20), 0, (2, 2, 2), 2, 0.05),
+    (3, 2, (22, 20, 20), 0, (2, 2, 2), 2, 0.05),    # 1100 blocks of 2 encodes x 8 voxels, a lane without a frame
+    (6, 1, (30, 31, 30), 0, (3, 3, 3), 2, 0.05),    # 1000 blocks of 27 rows, sizes not multiples of 3
+    (6, 1, (27, 27, 37), 0, (3, 3, 3), 2, 0.05),    # 972 of them: half a wavefront per block
+    (7, 1, (8, 8, 12), 0, (4, 4, 4), 2, 0.05),      # 7 frames, 64 rows: at any number of blocks
+    (8, 1, (10, 10, 10), 0, (5, 5, 5), 2, 0.05),    # 125 rows, 8 blocks
+    (4, 1, (96, 92, 96), 0, (4, 4, 4), 1, 0.05),    # 13248 blocks of 64 rows
+    # more than 8 frames: odd counts (a player without a partner), one block too
+    # many for the pairs of a wavefront, the encode dimension, several chunks
+    (9, 1, (8, 8, 16), 0, (8, 8, 8), 2, 0.05),
+    (11, 2, (15, 5, 9), 0, (3, 5, 2), 3, 0.05),
+    (2, 13, (8, 12, 8), 1, (4, 4, 4), 2, 0.05),
+    (16, 1, (8, 8, 24), 0, (8, 8, 8), 2, 0.05),
+    (17, 1, (8, 8, 16), 0, (8, 8, 8), 2, 0.05),
+    (20, 1, (8, 16, 8), 0, (8, 8, 8), 2, 0.05),
 ]
 
 
@@ -55,6 +71,27 @@ def test_llr_matches_oracle(Nt, Ne, shape, dim, block, block_iter, alpha):
     assert abs(smax - rsmax) <= 1e-6 * rsmax
     assert e <= 1e-5
     assert rel(ref, X) > 1e-3  # the step did something
+
+
+@pytest.mark.parametrize("n,block", [(64, 16), (96, 12), (48, 8)])
+def test_llr_long_blocks_are_not_slower_with_fewer_frames(n, block):
+    """Few blocks of many rows: 4 or 8 frames have a part of 9 frames' work and
+    must not take longer (one after the other in a few lanes, they took 1.6 times
+    as long)."""
+    t = {}
+    for F in (4, 8, 9):
+        X = torch.from_numpy(lowrank_frames(F, 1, (n, n, n), seed=3)).cuda()
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        best = []
+        for _ in range(6):
+            ev[0].record()
+            llr_threshold(X, alpha_time=0.01, block=(block,) * 3, block_iter=4)
+            ev[1].record()
+            torch.cuda.synchronize()
+            best.append(ev[0].elapsed_time(ev[1]))
+        t[F] = min(best[1:])
+    print("llr %d^3 in %d^3 blocks: %s ms" % (n, block, t))
+    assert t[4] <= 1.1 * t[9] and t[8] <= 1.1 * t[9]
 
 
 def test_llr_update_only_and_huge_threshold():
