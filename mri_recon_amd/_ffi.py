@@ -63,7 +63,8 @@ class MrnFrameStats(ctypes.Structure):
         ("split_tiles", ctypes.c_int32),
         ("wide", ctypes.c_int32),
         ("gather_items", ctypes.c_int32),
-        ("reserved", ctypes.c_int32 * 7),
+        ("wide_by_sample", ctypes.c_int32),
+        ("reserved", ctypes.c_int32 * 6),
     ]
 
 

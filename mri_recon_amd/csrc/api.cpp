@@ -207,7 +207,7 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
   }
   std::vector<FrameDev> h(F);
   int64_t off = 0, poff = 0;
-  op->fmax_ngrp = op->fmax_nheavy = op->fmax_nwide = op->fmax_xsplit = 0;
+  op->fmax_ngrp = op->fmax_nheavy = op->fmax_nwide = op->fmax_neach = op->fmax_xsplit = 0;
   op->fmax_Mv = 0;
   for (int f = 0; f < F; f++) {
     const FrameData &fr = op->frames[f];
@@ -230,11 +230,12 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
     d.ngrp = fr.ngrp;
     d.nheavy = fr.nheavy;
     d.nwide = fr.nwide;
-    d.pad = 0;
+    d.wide_each = fr.wide_each ? 1 : 0;
     off += fr.Mv * g.CC * op->nch;
     op->fmax_ngrp = std::max(op->fmax_ngrp, fr.ngrp);
     op->fmax_nheavy = std::max(op->fmax_nheavy, fr.nheavy);
-    op->fmax_nwide = std::max(op->fmax_nwide, fr.nwide);
+    int &nw = fr.wide_each ? op->fmax_neach : op->fmax_nwide;
+    nw = std::max(nw, fr.nwide);
     op->fmax_xsplit = std::max(op->fmax_xsplit, fr.xsplit_max);
     op->fmax_Mv = std::max(op->fmax_Mv, fr.Mv);
   }
@@ -1002,6 +1003,7 @@ int mrn_get_frame_stats(mrn_op *op, int f, mrn_frame_stats *out) {
   out->split_tiles = fr.nheavy;
   out->wide = fr.nwide;
   out->gather_items = fr.ngsub;
+  out->wide_by_sample = fr.wide_each ? 1 : 0;
   if (fr.nsub > 0) {
     std::vector<int4> subs((size_t)fr.nsub);
     MRN_HIP(op, hipMemcpy(subs.data(), fr.subs, sizeof(int4) * fr.nsub, hipMemcpyDeviceToHost));

@@ -1525,8 +1525,9 @@ __global__ __launch_bounds__(256, 6) void k_scatter_gd(
 // scatter adds their first NTb taps on every axis (the box its bins reach),
 // and this kernel adds the rest -- the taps past that box, on the window's far
 // edge -- with float atomics after the tiles are written.  Such samples sit
-// exactly on a window edge, so the list is short (often empty) and a thread per
-// sample walking its taps was all latency.  A sample's NT^3 window holds one
+// exactly on a window edge; on most trajectories the list is short (often empty)
+// and a thread per sample walking its taps (k_scatter_wide_each, for long lists
+// of samples on grid positions) is all latency.  A sample's NT^3 window holds one
 // cell of every class (x, y, z) mod NT: a wavefront takes a class and up to
 // WIDE_CHUNK listed samples, lanes = (sample, coil) of coil block blockIdx.y,
 // in list order, so that all that such a list adds to a cell comes from one
@@ -1542,6 +1543,7 @@ __global__ __launch_bounds__(64) void k_scatter_wide(float2 *grid, const float2 
                                                      int64_t chunk_k, const FrameDev *__restrict__ fdt) {
   if (fdt) {  // every frame at once: frame blockIdx.z
     const FrameDev &fd = fdt[blockIdx.z];
+    if (fd.wide_each) return;
     grid += fd.grid_off;
     kin = fd.kwork;
     coords = fd.coords;
@@ -1616,6 +1618,61 @@ __global__ __launch_bounds__(64) void k_scatter_wide(float2 *grid, const float2 
   const float w = weight(rk, rl);
   atomicAdd(&grid[rat].x, w * sum.x);
   atomicAdd(&grid[rat].y, w * sum.y);
+}
+
+// The same taps with a thread per (listed sample, coil), each walking its own:
+// the work is the taps themselves, not every class's look at every sample.
+__global__ void k_scatter_wide_each(float2 *grid, const float2 *__restrict__ kin, const float4 *__restrict__ coords,
+                                    const int32_t *__restrict__ wide, int nwide, Geom g, int NTb,
+                                    const float *__restrict__ tables, int64_t chunk_grid, int64_t chunk_k,
+                                    const FrameDev *__restrict__ fdt) {
+  if (fdt) {  // every frame at once: frame blockIdx.z
+    const FrameDev &fd = fdt[blockIdx.z];
+    if (!fd.wide_each) return;
+    grid += fd.grid_off;
+    kin = fd.kwork;
+    coords = fd.coords;
+    wide = fd.wide;
+    nwide = fd.nwide;
+    chunk_k = fd.Mv * g.CC;
+  }
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= (int64_t)nwide * g.CC) return;
+  const int c = (int)(idx & (g.CC - 1));
+  const int64_t i = wide[idx >> g.lgCC];
+  const int ch = blockIdx.y;
+  const float4 k = coords[i];
+  const float dk[3] = {k.x, k.y, k.z};
+  int s[3], e[3];
+  for (int a = 0; a < 3; a++)
+    if (!axis_range(g, a, dk[a], s[a], e[a])) return;
+  const float2 v = kin[ch * chunk_k + i * g.CC + c];
+  float2 *G = grid + ch * chunk_grid + c;
+  for (int lz = s[2]; lz <= e[2]; lz++) {
+    const float wz = tap_weight(g, 2, tables + g.toff[2], dk[2], lz);
+    for (int ly = s[1]; ly <= e[1]; ly++) {
+      const float wzy = wz * tap_weight(g, 1, tables + g.toff[1], dk[1], ly);
+      float2 *row = G + ((int64_t)lz * g.S[1] + ly) * g.S[0] * g.CC;
+      for (int lx = s[0]; lx <= e[0]; lx++) {
+        // inside the first NTb taps on every axis: the tile scatter's
+        if (lx < s[0] + NTb && ly < s[1] + NTb && lz < s[2] + NTb) continue;
+        const float w = wzy * tap_weight(g, 0, tables + g.toff[0], dk[0], lx);
+        atomicAdd(&row[(int64_t)lx * g.CC].x, w * v.x);
+        atomicAdd(&row[(int64_t)lx * g.CC].y, w * v.y);
+      }
+    }
+  }
+}
+
+// Listed samples whose position differs from the one before them in the list.
+__global__ void k_wide_runs(const float4 *__restrict__ coords, const int32_t *__restrict__ wide, int nwide, int *runs) {
+  int n = 0;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nwide; i += gridDim.x * blockDim.x) {
+    const float4 a = coords[wide[i]], b = coords[wide[max(i - 1, 0)]];
+    n += i == 0 || a.x != b.x || a.y != b.y || a.z != b.z ? 1 : 0;
+  }
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+  if ((threadIdx.x & 63) == 0 && n) atomicAdd(runs, n);
 }
 
 // wide[i] = 1 when valid sample i has more than NTb taps on some axis
@@ -2028,17 +2085,24 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
   return MRN_OK;
 }
 
-// The window-edge taps (k_scatter_wide), after the tiles' plain stores.
+// The window-edge taps, after the tiles' plain stores: by classes
+// (k_scatter_wide) or sample by sample (fr.wide_each).
 int launch_scatter_wide(mrn_op *op, float2 *grid, const float2 *kin, const mrn::FrameData &fr, hipStream_t st,
                         const FrameDev *fdt) {
   const Geom &g = op->g;
-  const int nwide = fdt ? op->fmax_nwide : fr.nwide;
+  const int nwide = fdt ? op->fmax_nwide : fr.wide_each ? 0 : fr.nwide;
+  const int neach = fdt ? op->fmax_neach : fr.wide_each ? fr.nwide : 0;
+  const int64_t cg = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC, ck = fr.Mv * g.CC;
+  const int NT = op->t.NT, NTb = op->t.NTb;
   if (nwide > 0) {
-    const int64_t cg = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC, ck = fr.Mv * g.CC;
-    const int NT = op->t.NT, NTb = op->t.NTb;
     const int64_t n = (int64_t)((nwide + WIDE_CHUNK - 1) / WIDE_CHUNK) * NT * NT * NT;
     hipLaunchKernelGGL(k_scatter_wide, dim3((unsigned)n, op->nch, fdt ? op->F : 1), dim3(64), 0, st, grid, kin,
                        fr.coords, fr.wide, fr.nwide, g, NT, NTb, op->tables_d, cg, ck, fdt);
+    MRN_HIP(op, hipGetLastError());
+  }
+  if (neach > 0) {
+    hipLaunchKernelGGL(k_scatter_wide_each, dim3(nblk((int64_t)neach * g.CC, 256), op->nch, fdt ? op->F : 1), dim3(256),
+                       0, st, grid, kin, fr.coords, fr.wide, fr.nwide, g, NTb, op->tables_d, cg, ck, fdt);
     MRN_HIP(op, hipGetLastError());
   }
   return MRN_OK;
@@ -2214,6 +2278,20 @@ static int visits_per_item(const Tiles &t, int64_t Mv) {
   return (int)std::min<int64_t>(std::max<int64_t>(v, 64), MRN_AUTO_MAXV);
 }
 
+// Which form of the window-edge taps a list takes: the classes look at every
+// sample NT^3 times, which is worth it where many samples lie at one point
+// (runs: changes of position along the list), whose atomics the other form
+// issues one by one, and while the list is too short to fill the chip.
+// Scatter of `nwide` samples alone on a 144^3 grid, W = 4, classes / samples, us:
+//   one point:           4096 x 1, 8, 16 coils 37 / 1239, 37 / 597, 50 / 1037
+//   16 samples a point:  4096 x 1, 8, 16 75 / 164, 120 / 138, 210 / 177; 65536 560 / 546, 921 / 908, 1879 / 1901
+//   distinct:            513 x 1, 4, 8, 16 39 / 104, 70 / 67, 100 / 62, 167 / 65; 4096 64 / 109, 89 / 73, 158 / 93,
+//                        255 / 126; 65536 431 / 352, 487 / 457, 590 / 497, 1338 / 1142
+// Lists of one chunk stay with the classes: one order, the same bits each call.
+static bool wide_each(int nwide, int runs, int CC) {
+  return nwide > WIDE_CHUNK && (int64_t)nwide * CC * CC >= 32768 && runs > nwide / 4;
+}
+
 // Sort one frame's samples into tiles and build the scatter work list.  The
 // frame's arrays and the bind's scratch only grow (FrameCaps, BindScratch), so
 // binding a trajectory no larger than the last one allocates nothing; the
@@ -2238,6 +2316,7 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
   MRN_BH(hipDeviceSynchronize());
   fr.has_traj = false;
   fr.nwide = 0;
+  fr.wide_each = false;
   fr.ngsub = 0;
   fr.nsparse = 0;
   fr.nsub = 0;
@@ -2308,6 +2387,17 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
       MRN_BH(hipGetLastError());
     }
     fr.nwide = nw;
+    if (nw > WIDE_CHUNK) {
+      int *runs_d = b.woff;  // (its entries are used up)
+      int runs = 0;
+      hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, runs_d, 0, (int64_t)1);
+      hipLaunchKernelGGL(k_wide_runs, dim3(std::min<unsigned>(nblk(nw, 256), 1024u)), dim3(256), 0, st, fr.coords, fr.wide,
+                         nw, runs_d);
+      MRN_BH(hipGetLastError());
+      MRN_BH(hipMemcpyAsync(&runs, runs_d, sizeof(int), hipMemcpyDeviceToHost, st));
+      MRN_BH(hipStreamSynchronize(st));
+      fr.wide_each = wide_each(nw, runs, g.CC);
+    }
   }
   // k-space support per grid row, for the x passes
   {

@@ -80,7 +80,7 @@ struct FrameDev {
   const float2 *kdata;     // measured k-space, same layout
   int64_t Mv;
   int64_t grid_off;        // first element of this frame's coil blocks in the grid
-  int ngrp, nheavy, nwide, pad;
+  int ngrp, nheavy, nwide, wide_each;
 };
 
 // Device arrays that only grow: binding a trajectory no larger than an
@@ -147,6 +147,7 @@ struct FrameData {
   int ngsub = 0;
   int32_t *wide = nullptr;     // [nwide] samples with more than Tiles::NTb taps on some axis
   int nwide = 0;
+  bool wide_each = false;      // those taps sample by sample, not by classes of cells
   int32_t *sparse = nullptr;   // [nsparse] samples of tiles below the dense limit (direct gather)
   int64_t nsparse = 0;
   int2 *xrng = nullptr;        // [Sz][Sy] x cells any tap reaches in grid row (z, y); x > y: none
@@ -189,7 +190,7 @@ struct mrn_op {
   int64_t kwork_all_cap = 0;   // elements
   int2 *xrng_all = nullptr;    // [F][Sz][Sy] x support rows (k_row_xrange) of every frame
   int2 *yrng_all = nullptr;    // [F][Sz] y support of every frame, when the y passes are pruned
-  int fmax_ngrp = 0, fmax_nheavy = 0, fmax_nwide = 0, fmax_xsplit = 0;
+  int fmax_ngrp = 0, fmax_nheavy = 0, fmax_nwide = 0, fmax_neach = 0, fmax_xsplit = 0;
   int64_t fmax_Mv = 0;
   float2 *kplain = nullptr;    // plain form: one coil of k-space [M_max]
   int64_t kplain_cap = 0;
