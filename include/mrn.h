@@ -288,7 +288,8 @@ typedef struct mrn_frame_stats {
   int32_t wide;            /* samples with one tap more than usual on some axis */
   int32_t gather_items;    /* tile-staged gather work items */
   int32_t wide_by_sample;  /* 1: the window-edge taps are added sample by sample, 0: by classes of cells */
-  int32_t reserved[6];
+  int32_t scatter_groups;  /* wavefronts' groups of scatter work items (= scatter_items: one item each) */
+  int32_t reserved[5];
 } mrn_frame_stats;
 int mrn_get_frame_stats(mrn_op *op, int frame, mrn_frame_stats *out);
 

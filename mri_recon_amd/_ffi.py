@@ -64,7 +64,8 @@ class MrnFrameStats(ctypes.Structure):
         ("wide", ctypes.c_int32),
         ("gather_items", ctypes.c_int32),
         ("wide_by_sample", ctypes.c_int32),
-        ("reserved", ctypes.c_int32 * 6),
+        ("scatter_groups", ctypes.c_int32),
+        ("reserved", ctypes.c_int32 * 5),
     ]
 
 

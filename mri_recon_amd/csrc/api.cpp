@@ -209,6 +209,7 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
   int64_t off = 0, poff = 0;
   op->fmax_ngrp = op->fmax_nheavy = op->fmax_nwide = op->fmax_neach = op->fmax_xsplit = 0;
   op->fmax_Mv = 0;
+  op->fgroups = false;
   for (int f = 0; f < F; f++) {
     const FrameData &fr = op->frames[f];
     FrameDev &d = h[f];
@@ -233,6 +234,7 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
     d.wide_each = fr.wide_each ? 1 : 0;
     off += fr.Mv * g.CC * op->nch;
     op->fmax_ngrp = std::max(op->fmax_ngrp, fr.ngrp);
+    op->fgroups = op->fgroups || fr.groups;
     op->fmax_nheavy = std::max(op->fmax_nheavy, fr.nheavy);
     int &nw = fr.wide_each ? op->fmax_neach : op->fmax_nwide;
     nw = std::max(nw, fr.nwide);
@@ -1004,6 +1006,7 @@ int mrn_get_frame_stats(mrn_op *op, int f, mrn_frame_stats *out) {
   out->wide = fr.nwide;
   out->gather_items = fr.ngsub;
   out->wide_by_sample = fr.wide_each ? 1 : 0;
+  out->scatter_groups = fr.ngrp;
   if (fr.nsub > 0) {
     std::vector<int4> subs((size_t)fr.nsub);
     MRN_HIP(op, hipMemcpy(subs.data(), fr.subs, sizeof(int4) * fr.nsub, hipMemcpyDeviceToHost));

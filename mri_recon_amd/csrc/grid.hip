@@ -1140,20 +1140,18 @@ __global__ __launch_bounds__(256) void k_sum_tiles(float2 *grid, const float2 *_
 // per cell.  Sums are FP32; only the order of the additions differs from a
 // per-sample loop.  Each tile is written once with plain stores; a tile split
 // over several work items goes to its items' slots, which k_sum_tiles adds.
-// A wavefront takes a group of consecutive work items (gstart: equal cost,
-// group_cost) as one stream of batches: its visits are one run of the visit
-// list, so the loads of the next items' first batches fly while this item's
-// last ones are summed, and the kernel tables are loaded once per group.  One
-// item per wavefront waited for five dependent loads (item, offset, visits,
+// GROUPS: a wavefront takes a group of consecutive work items (gstart: equal
+// cost, group_cost) as one stream of batches: its visits are one run of the
+// visit list, so the loads of the next items' first batches fly while this
+// item's last ones are summed, and the kernel tables are loaded once per group.
+// One item per wavefront waits for five dependent loads (item, offset, visits,
 // coordinates, values) for one or two batches of work in sparse k-space.
-// Scatter with one item per wavefront / with groups: 160^3 x 24 coils, 768000
-// samples 1007 / 845 us; 128^3 x 8, 262144 samples 165 / 144; 100 x 84 x 92 x 8
-// 163 / 148; 256^3 x 32, 5.12 M samples 3.86 / 3.69 ms.
+// group_items chooses, with the figures of both.
 // PAIR (8-coil blocks): a work item takes coil blocks 2 y and 2 y + 1 as its
 // two 16-real blocks, so step A's weights serve both (the second is skipped
 // when nch is odd and y is the last pair).
 #define SM_BATCH 32
-template <int CCT, int KM, bool PAIR>
+template <int CCT, int KM, bool PAIR, bool GROUPS>
 __global__ __launch_bounds__(256, 4) void k_scatter_mm(
     float2 *__restrict__ grid, const float2 *__restrict__ kin, const float4 *__restrict__ coords,
     const int64_t *__restrict__ vofs, const int32_t *__restrict__ vlist, const int4 *__restrict__ subs,
@@ -1188,7 +1186,8 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
   }
   const int unit = scatter_item(blockIdx.x, gridDim.x, wave, t.xrun, xs);
   if (unit < 0 || unit >= ngrp) return;
-  const int ibeg = gstart[unit], iend = gstart[unit + 1];
+  // GROUPS: the unit's items; else the unit is an item
+  const int ibeg = GROUPS ? gstart[unit] : unit, iend = GROUPS ? gstart[unit + 1] : unit + 1;
   if (ibeg >= iend) return;
   const int ch = PAIR ? 2 * (int)blockIdx.y : (int)blockIdx.y;
   const bool have1 = !PAIR || ch + 1 < nch;  // (uniform) the pair's second block exists
@@ -1201,31 +1200,39 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
   // 1056), so that no load stands between two items.
   enum : int { LAST = 1 << 8, VALID = 1 << 9 };
   const int nit = iend - ibeg;
-  const int4 mine = subs[ibeg + min(lane, nit - 1)];
-  const int first = __builtin_amdgcn_readlane(mine.x, 0);
-  const int32_t *vl = vlist + (vofs[first] + __builtin_amdgcn_readlane(mine.y, 0));
+  const int4 mine = subs[GROUPS ? ibeg + min(lane, nit - 1) : ibeg];
+  const int first = GROUPS ? __builtin_amdgcn_readlane(mine.x, 0) : mine.x;
+  const int32_t *vl = vlist + (vofs[first] + (GROUPS ? __builtin_amdgcn_readlane(mine.y, 0) : mine.y));
   int gk = 0, gq = 0, gp = 0;  // item; visits handed out of it, of the group
   // the next batch, and the internal index of its visit of this lane (past the
   // end: the last one, a valid index, so that every lane loads)
   auto gen = [&](int &idx) -> int {
     idx = 0;
-    if (gk >= nit) return 0;
-    const int len = __builtin_amdgcn_readlane(mine.z, gk) - __builtin_amdgcn_readlane(mine.y, gk);
-    const int n = min(SM_BATCH, len - gq);
-    if (n > 0) idx = vl[gp + min(sl, n - 1)];
-    gp += n;
-    gq += n;
-    int b = n | VALID | (gk << 16);
-    if (gq >= len) {
-      b |= LAST;
-      gk++;
-      gq = 0;
+    if constexpr (!GROUPS) {
+      const int n = min(SM_BATCH, mine.z - mine.y - gq);
+      if (n <= 0) return 0;
+      idx = vl[gq + min(sl, n - 1)];
+      gq += SM_BATCH;
+      return n;
+    } else {
+      if (gk >= nit) return 0;
+      const int len = __builtin_amdgcn_readlane(mine.z, gk) - __builtin_amdgcn_readlane(mine.y, gk);
+      const int n = min(SM_BATCH, len - gq);
+      if (n > 0) idx = vl[gp + min(sl, n - 1)];
+      gp += n;
+      gq += n;
+      int b = n | VALID | (gk << 16);
+      if (gq >= len) {
+        b |= LAST;
+        gk++;
+        gq = 0;
+      }
+      return b;
     }
-    return b;
   };
   // origin of a batch's tile
   auto origin = [&](int b, int (&o)[3]) {
-    const int tile = __builtin_amdgcn_readlane(mine.x, b >> 16);
+    const int tile = GROUPS ? __builtin_amdgcn_readlane(mine.x, b >> 16) : first;
     o[0] = (tile % t.nt[0]) * 4;
     o[1] = ((tile / t.nt[0]) % t.nt[1]) * 4;
     o[2] = (tile / (t.nt[0] * t.nt[1])) * 4;
@@ -1263,6 +1270,47 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
   int i0, t0[3];
   int b0 = gen(i0), b1 = gen(inext), b2 = gen(inext2);
   origin(b0, t0);
+  // the item's sums to its tile or, of a split tile, to its slot, [nch][64 cells][CCT]
+  auto finish = [&]() {
+    const int slot = GROUPS ? __builtin_amdgcn_readlane(mine.w, b0 >> 16) : mine.w;
+    const int64_t cell0 = slot ? ((int64_t)(slot - 1) * nch + ch) * 64
+                               : ((int64_t)t0[2] * g.S[1] + t0[1]) * g.S[0] + t0[0];
+    const int64_t ys = 2 * CCT * (slot ? 4 : g.S[0]);  // floats from one row, plane of cells to the next
+    const int64_t zs = slot ? 2 * CCT * 16 : (int64_t)g.S[1] * ys;
+    const int64_t next = 2 * (slot ? 64 * CCT : chunk_grid);  // PAIR: the second block's cell
+    float *base = slot ? reinterpret_cast<float *>(part + cell0 * CCT)
+                       : reinterpret_cast<float *>(grid + ch * chunk_grid + cell0 * CCT);
+    // (opaque copies: the addresses below are not worth registers in the loop)
+    int cie = ci, kqe = kq;
+    asm volatile("" : "+v"(cie), "+v"(kqe));
+    // accumulator block (p, nb), register r of lane l: cell 16 p + 4 (l / 16) + r,
+    // real 16 nb + l % 16 of the cell's CCT coils (PAIR: real l % 16 of block
+    // ch + nb)
+    float *row = base + kqe * ys + cie;
+#pragma unroll
+    for (int p = 0; p < 4; p++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        if (t0[0] + r < g.S[0] && t0[1] + kqe < g.S[1] && t0[2] + p < g.S[2]) {
+          float *dst = row + p * zs + r * (2 * CCT);
+#pragma unroll
+          for (int nb = 0; nb < NB; nb++) {
+            if (nb > 0 && !have1) continue;
+            const float v = acc[p][nb][r];
+            float *d = PAIR ? dst + nb * next : dst + 16 * nb;
+            if (accum && !slot) {  // the tile's only work item: a plain read-modify-write
+              *d += v;
+            } else {
+              *d = v;
+            }
+          }
+        }
+      }
+#pragma unroll
+    for (int p = 0; p < 4; p++)
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) acc[p][nb] = mrn_v4f{0.f, 0.f, 0.f, 0.f};
+  };
   auto batch = [&](const float (&cur)[NG][NB], float (&nxt)[NG][NB]) {
     // ---- A: weights of the batch
     const bool ok = sl < (b0 & 0xFF);
@@ -1326,44 +1374,11 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
       }
     }
     wave_sync();
-    if (b0 & LAST) {
-      const int slot = __builtin_amdgcn_readlane(mine.w, b0 >> 16);
-      // (opaque copies: the addresses below are not worth registers in the loop)
-      int cie = ci, kqe = kq;
-      asm volatile("" : "+v"(cie), "+v"(kqe));
-      // accumulator block (p, nb), register r of lane l: cell 16 p + 4 (l / 16) + r,
-      // real 16 nb + l % 16 of the cell's CCT coils (PAIR: real l % 16 of block
-      // ch + nb)
-#pragma unroll
-      for (int p = 0; p < 4; p++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int cx = t0[0] + r, cy = t0[1] + kqe, cz = t0[2] + p;
-          if (cx < g.S[0] && cy < g.S[1] && cz < g.S[2]) {
-            // a split tile's item writes its slot, [nch][64 cells][CCT]
-            const int64_t cell = slot ? (((int64_t)(slot - 1) * nch + ch) * 64 + 16 * p + 4 * kqe + r) * CCT
-                                      : ch * chunk_grid + (((int64_t)cz * g.S[1] + cy) * g.S[0] + cx) * CCT;
-            const int64_t next = slot ? 64 * CCT : chunk_grid;  // PAIR: the second block's cell
-            float *dst = reinterpret_cast<float *>((slot ? part : grid) + cell) + cie;
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) {
-              if (nb > 0 && !have1) continue;
-              const float v = acc[p][nb][r];
-              float *d = PAIR ? dst + nb * 2 * next : dst + 16 * nb;
-              if (accum && !slot) {  // the tile's only work item: a plain read-modify-write
-                *d += v;
-              } else {
-                *d = v;
-              }
-            }
-          }
-        }
-#pragma unroll
-      for (int p = 0; p < 4; p++)
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++) acc[p][nb] = mrn_v4f{0.f, 0.f, 0.f, 0.f};
-      origin(b1, t0);
-    }
+    if constexpr (GROUPS)
+      if (b0 & LAST) {
+        finish();
+        origin(b1, t0);
+      }
     b0 = b1;
     b1 = b2;
     b2 = b3;
@@ -1378,10 +1393,19 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
     load_data(i0, dA);
   }
   if (b1 & 0xFF) kraw1 = *reinterpret_cast<const float4 *>(cb + (uint32_t)inext * 16u);
-  while (b0 & VALID) {
-    batch(dA, dB);
-    if (!(b0 & VALID)) break;
-    batch(dB, dA);
+  if constexpr (GROUPS) {
+    while (b0 & VALID) {
+      batch(dA, dB);
+      if (!(b0 & VALID)) break;
+      batch(dB, dA);
+    }
+  } else {
+    while (b0) {
+      batch(dA, dB);
+      if (!b0) break;
+      batch(dB, dA);
+    }
+    finish();
   }
 }
 
@@ -1402,7 +1426,7 @@ __global__ __launch_bounds__(256, 4) void k_scatter_mm(
 // sample that misses the tile costs only its share of step A.  The sums
 // accumulate in visit order, as a lane-per-sample walk would.
 #define SG_BATCH 16
-template <int CCT>
+template <int CCT, bool GROUPS>
 __global__ __launch_bounds__(256, 6) void k_scatter_gd(
     float2 *__restrict__ grid, const float2 *__restrict__ kin, const float4 *__restrict__ coords,
     const int64_t *__restrict__ vofs, const int32_t *__restrict__ vlist, const int4 *__restrict__ subs,
@@ -1435,8 +1459,9 @@ __global__ __launch_bounds__(256, 6) void k_scatter_gd(
   const int ch = blockIdx.y;
   const float2 *kch = kin + ch * chunk_k;
   const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
-  const int iend = gstart[unit + 1];
-  for (int item = gstart[unit]; item < iend; item++) {
+  // GROUPS: the unit's items; else the unit is an item
+  const int iend = GROUPS ? gstart[unit + 1] : unit + 1;
+  for (int item = GROUPS ? gstart[unit] : unit; item < iend; item++) {
     const int4 sp = subs[item];
     const int tile = sp.x;
     const int tix = tile % t.nt[0], tiy = (tile / t.nt[0]) % t.nt[1], tiz = tile / (t.nt[0] * t.nt[1]);
@@ -2028,6 +2053,13 @@ int launch_scatter_sum(mrn_op *op, float2 *grid, const mrn::FrameData &fr, hipSt
   return MRN_OK;
 }
 
+// Whether the scatter of a frame of Mv samples goes to the matrix cores: 8- or
+// 16-coil blocks whose k-space and coordinates 32-bit byte offsets reach.
+static bool scatter_mm(const mrn_op *op, int64_t Mv) {
+  const int CC = op->g.CC;
+  return (CC == 16 || CC == 8) && !op->scatter_valu && Mv * CC * 8 < (1ll << 32) && Mv * 16 < (1ll << 32);
+}
+
 // The tile scatter proper: every tile but the split ones is written (accum:
 // read, added to and stored); launch_scatter_sum and launch_scatter_wide follow.
 int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn::FrameData &fr,
@@ -2049,18 +2081,24 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
   // no work item: a frame without valid samples whose x passes are limited to
   // its (empty) k-space support -- nothing reads the grid
   if (ngrp == 0) return MRN_OK;
+  const bool groups = fdt ? op->fgroups : fr.groups;  // (every frame's groups are there, of one item each too)
   const bool exact = g.kmode == MRN_KMODE_EXACT_KB;
-  // the matrix-core form addresses a coil block's k-space and the coordinates
-  // with 32-bit byte offsets
-  const bool off32 = Mv * g.CC * 8 < (1ll << 32) && Mv * 16 < (1ll << 32);
-  if ((g.CC == 16 || g.CC == 8) && !op->scatter_valu && off32) {
+  if (scatter_mm(op, Mv)) {
     // 8-coil blocks go in pairs (one work item, both blocks) when there are two or more
     const bool pair = g.CC == 8 && op->nch >= 2;
     dim3 gm = g3;
     if (pair) gm.y = (unsigned)((op->nch + 1) / 2);
 #define MRN_MM(n, km, pr)                                                                                \
-  hipLaunchKernelGGL((k_scatter_mm<n, km, pr>), gm, dim3(256), sh, st, grid, kin, fr.coords, fr.vofs,   \
-                     fr.vlist, fr.subs, fr.gstart, fr.ngrp, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit, op->nch, op->part)
+  do {                                                                                                   \
+    if (groups)                                                                                          \
+      hipLaunchKernelGGL((k_scatter_mm<n, km, pr, true>), gm, dim3(256), sh, st, grid, kin, fr.coords, fr.vofs,   \
+                         fr.vlist, fr.subs, fr.gstart, fr.ngrp, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit,   \
+                         op->nch, op->part);                                                             \
+    else                                                                                                 \
+      hipLaunchKernelGGL((k_scatter_mm<n, km, pr, false>), gm, dim3(256), sh, st, grid, kin, fr.coords, fr.vofs,  \
+                         fr.vlist, fr.subs, fr.gstart, fr.ngrp, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit,   \
+                         op->nch, op->part);                                                             \
+  } while (0)
     if (g.CC == 16 && !exact) MRN_MM(16, 0, false);
     else if (g.CC == 16) MRN_MM(16, 1, false);
     else if (pair && !exact) MRN_MM(8, 0, true);
@@ -2072,8 +2110,14 @@ int launch_scatter_tiles(mrn_op *op, float2 *grid, const float2 *kin, const mrn:
     switch (g.CC) {
 #define MRN_S(n)                                                                                 \
   case n:                                                                                        \
-    hipLaunchKernelGGL((k_scatter_gd<n>), g3, dim3(256), sh, st, grid, kin, fr.coords, fr.vofs,  \
-                       fr.vlist, fr.subs, fr.gstart, fr.ngrp, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit, op->nch, op->part); \
+    if (groups)                                                                                  \
+      hipLaunchKernelGGL((k_scatter_gd<n, true>), g3, dim3(256), sh, st, grid, kin, fr.coords, fr.vofs,  \
+                         fr.vlist, fr.subs, fr.gstart, fr.ngrp, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit,  \
+                         op->nch, op->part);                                                     \
+    else                                                                                         \
+      hipLaunchKernelGGL((k_scatter_gd<n, false>), g3, dim3(256), sh, st, grid, kin, fr.coords, fr.vofs,  \
+                         fr.vlist, fr.subs, fr.gstart, fr.ngrp, g, t, op->tables_d, cg, ck, af, fdt, fr.xsplit,  \
+                         op->nch, op->part);                                                     \
     break;
     MRN_S(1) MRN_S(2) MRN_S(4) MRN_S(8) MRN_S(16)
 #undef MRN_S
@@ -2243,11 +2287,34 @@ __global__ void k_item_cost(const int4 *__restrict__ subs, int n, int64_t *cost)
 // Groups of consecutive work items of equal cost (pre: exclusive prefix of the
 // costs): group q starts at the first item whose prefix reaches q * per.  An
 // item longer than `per` leaves empty groups behind it.  start[ngrp] = n.
+// per = 0: every item a group of its own.
 __global__ void k_group_start(const int64_t *__restrict__ pre, int n, int64_t per, int ngrp, int32_t *start) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i > n) return;
+  if (per == 0) {
+    start[i] = i;
+    return;
+  }
   const int64_t q1 = i < n ? pre[i] / per : ngrp, q0 = i > 0 ? pre[i - 1] / per : -1;
   for (int64_t q = q0 + 1; q <= q1; q++) start[q] = i;
+}
+
+// Whether a wavefront takes a group of work items (as one stream, with their
+// loads ahead) or a single one.  Groups are for the matrix-core form where the
+// items are many and short; with few items they leave the chip half empty, with
+// long ones the stream's bookkeeping costs more than the waits it hides, and
+// neighbouring tiles, which share samples, no longer run side by side.  Scatter
+// in us, groups / single:
+//   8 coils:  13824 items of 88, 199 visits on average (with the fixed 32) 56 / 47, 102 / 83; 30611 of 110 127 / 118;
+//             66321 of 64 137 / 149; 110592 of 103, 209, 387 304 / 324, 588 / 572, 1071 / 989; 373248 of 117
+//             1017 / 1161; 512000 of 186 2221 / 2318
+//   16 coils: 13824 of 199 137 / 115; 46656 of 366 657 / 601; 66321 of 64 214 / 237; 80416 of 430 1362 / 1367;
+//             110592 of 103, 387 456 / 494, 1567 / 1481; 224738 of 174 1467 / 1630; 373248 of 201 2623 / 2746
+//   vector ALUs (other blocks): 1 coil 110592 of 174 623 / 580, 379562 of 116 1328 / 1365; 2 coils 13824 of 589
+//             384 / 288; 4 coils 110592 of 68, 174 225 / 212, 710 / 618
+static bool group_items(const mrn_op *op, int64_t Mv, int64_t n, int64_t total) {
+  if (!scatter_mm(op, Mv) || n <= 49152) return false;
+  return n > 196608 || total < 192 * n;
 }
 
 // Cost of a group: the list's total over 4 rounds of the chip's 4096 scatter
@@ -2518,8 +2585,9 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
     int64_t total = 0;
     MRN_BH(hipMemcpyAsync(&total, b.ipre + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
     MRN_BH(hipStreamSynchronize(st));
-    const int64_t per = group_cost(total);
-    fr.ngrp = n > 0 ? (int)(total / per + 1) : 0;
+    fr.groups = group_items(op, fr.Mv, n, total);
+    const int64_t per = fr.groups ? group_cost(total) : 0;
+    fr.ngrp = n == 0 ? 0 : fr.groups ? (int)(total / per + 1) : (int)n;
     MRN_BH(grow(fr.gstart, cp.gstart, (int64_t)fr.ngrp + 1));
     hipLaunchKernelGGL(k_group_start, dim3(nblk(n + 1, 256)), dim3(256), 0, st, b.ipre, (int)n, per, fr.ngrp, fr.gstart);
     MRN_BH(hipGetLastError());

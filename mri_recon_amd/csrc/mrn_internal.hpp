@@ -136,6 +136,7 @@ struct FrameData {
   int4 *subs = nullptr;        // [nsub] {tile, first visit, end visit, 0 or its partial-sum slot + 1}
   int32_t *gstart = nullptr;   // [ngrp + 1] first work item of each group of equal cost (one wavefront each)
   int ngrp = 0;
+  bool groups = false;         // groups of several items, or one item each
   int32_t *xsplit = nullptr;   // [MRN_XCDS + 1] ranges of those groups, one per XCD
   int xsplit_max = 0;          // longest of those ranges
   int4 *heavy = nullptr;       // [nheavy] tiles split over several work items {tile, first slot, slots}
@@ -192,6 +193,7 @@ struct mrn_op {
   int2 *yrng_all = nullptr;    // [F][Sz] y support of every frame, when the y passes are pruned
   int fmax_ngrp = 0, fmax_nheavy = 0, fmax_nwide = 0, fmax_neach = 0, fmax_xsplit = 0;
   int64_t fmax_Mv = 0;
+  bool fgroups = false;        // some frame's groups hold several work items
   float2 *kplain = nullptr;    // plain form: one coil of k-space [M_max]
   int64_t kplain_cap = 0;
   mrn::BindScratch bind;       // trajectory-bind scratch (grow-only)

@@ -400,6 +400,40 @@ def test_groups_of_work_items(C, kw, spokes):
         assert rel(out[0], out[1]) <= 3.6e-6
 
 
+@pytest.mark.parametrize("N,C,M,kw,groups", [
+    (128, 8, 0, {}, True), (128, 16, 40, {}, True), (128, 24, 300000, {}, True),        # many short items
+    (128, 16, 300000, {"xcd_run": -1}, True), (128, 8, 3000000, {}, False),             # many, long on average
+    (96, 8, 100000, {}, False), (96, 24, 100000, {"xcd_run": -1}, False),               # not so many
+    (128, 4, 300000, {}, False), (128, 8, 300000, {"scatter_valu": True}, False)])      # vector ALUs
+def test_scatter_groups_rule(N, C, M, kw, groups):
+    """Which scatter calls take their items in groups, on both sides of each
+    line: A^H, overwriting and adding into the image, against items of at most
+    96 visits on the vector ALUs (or, for those, on the matrix cores).  Every
+    tile has an item, samples or not (LDS Stockham passes)."""
+    g = torch.Generator(device="cuda").manual_seed(N + C)
+    k = [(torch.rand(max(M, 1), device="cuda", generator=g) - 0.5) * N for _ in range(3)]
+    kw_ = torch.full((max(M, 1),), 0.0 if M == 0 else 1.0, device="cuda")  # M = 0: every sample skipped
+    smaps = torch.randn((C, N, N, N), dtype=torch.complex64, device="cuda", generator=g)
+    d = torch.randn((C, k[0].numel()), dtype=torch.complex64, device="cuda", generator=g)
+    out = []
+    for other in (False, True):
+        opt = dict(kw, scatter_valu=not kw.get("scatter_valu", False), max_visits=96) if other else kw
+        op = GridFFT(N, ncoils=C, fft_stockham=True, **opt)
+        op.set_traj(*k, kw_)
+        op.set_smaps(smaps)
+        if not other:
+            st = op.frame_stats()
+            assert (st["scatter_groups"] < st["scatter_items"]) == groups
+            assert groups or st["scatter_groups"] == st["scatter_items"]
+        h = op.forward(d, accumulate=False)
+        out.append(op.forward(d, X=h).cpu().numpy())
+        op.close()
+    if M == 0:
+        assert np.count_nonzero(out[0]) == 0 and np.count_nonzero(out[1]) == 0
+    else:  # a cell sums at most some 10^2 visits
+        assert rel(out[0], out[1]) <= 1e-6
+
+
 @pytest.mark.parametrize("C,spokes,nc", [(1, 10, 1), (2, 40, 1), (2, 4000, 2), (8, 200, 1), (8, 1100, 2), (16, 100, 1),
                                          (16, 300, 2), (16, 1100, 4), (24, 1100, 2)])
 def test_gather_coils_rule(C, spokes, nc):
