@@ -9,7 +9,8 @@
 // [frame][block] gives every block its output offset in frame-major order;
 // pass 2 recomputes the selection and writes each kept sample at its offset
 // plus its rank in the block (wavefront ballots), so the order is the input
-// order.  Trajectory and k-space are read once per frame.
+// order.  A workgroup takes several frames of its block (gate_per), so the
+// trajectory and the k-space are read once for those.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -71,16 +72,18 @@ __device__ __forceinline__ Pick pick_sample(const GateDev &g, const double *__re
   return p;
 }
 
-// Both passes take every frame of a 256-sample block in one workgroup: the
-// trajectory, the k-space and the weight's arithmetic are read and done once,
-// not once per frame.  20000 readouts of 256 samples, 8 coils, 12 frames with
-// view sharing: counting 185 -> 64 us, writing 439 -> 370 us.
+// Both passes take `per` frames of a 256-sample block in one workgroup: the
+// trajectory, the k-space and the weight's arithmetic are read and done once
+// for them.  20000 readouts of 256 samples, 8 coils, 12 frames with view
+// sharing, a workgroup per frame and block before: counting 185 -> 64 us,
+// writing 439 -> 370 us.
 __global__ __launch_bounds__(256) void k_gate_count(GateDev g, const double *__restrict__ gt,
                                                     const float *__restrict__ resp, const float *__restrict__ kx,
                                                     const float *__restrict__ ky, const float *__restrict__ kz,
-                                                    int64_t *__restrict__ bcnt) {
+                                                    int per, int64_t *__restrict__ bcnt) {
   const Pick p = pick_sample(g, gt, resp, kx, ky, kz, (long long)blockIdx.x * 256 + threadIdx.x);
-  for (int t = 0; t < g.frames; t++) {
+  const int t0 = blockIdx.y * per, t1 = min(t0 + per, g.frames);
+  for (int t = t0; t < t1; t++) {
     const int n = __syncthreads_count(p.in(g, t));
     if (threadIdx.x == 0) bcnt[(long long)t * g.nb + blockIdx.x] = n;
   }
@@ -99,12 +102,13 @@ __global__ __launch_bounds__(256) void k_gate_scatter(GateDev g, const double *_
                                                       const float2 *__restrict__ kd, const int64_t *__restrict__ boff,
                                                       const int64_t *__restrict__ fb, float *__restrict__ ox,
                                                       float *__restrict__ oy, float *__restrict__ oz,
-                                                      float *__restrict__ ow, float2 *__restrict__ okd) {
+                                                      float *__restrict__ ow, float2 *__restrict__ okd, int per) {
   __shared__ int wcount[2][4];
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   const Pick p = pick_sample(g, gt, resp, kx, ky, kz, i);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int t = 0; t < g.frames; t++) {
+  const int t0 = blockIdx.y * per, t1 = min(t0 + per, g.frames);
+  for (int t = t0; t < t1; t++) {
     const bool s = p.in(g, t);
     const unsigned long long m = __ballot(s);
     // two rows in turn: a wavefront writes a row again only after the next
@@ -124,6 +128,16 @@ __global__ __launch_bounds__(256) void k_gate_scatter(GateDev g, const double *_
     ow[pos] = g.reset ? 1.0f : __fmul_rn(scale, kw[i]);
     for (int c = 0; c < C; c++) okd[base * C + (int64_t)c * n + o] = kd[(int64_t)c * g.M + i];
   }
+}
+
+// Frames per workgroup.  A workgroup's frames go one after the other, so fewer
+// where there are not GATE_GROUPS workgroups of blocks alone.  The call in us
+// with 1 frame / this rule / all: 25 blocks x 100 frames 583 / 582 / 658; 125 x
+// 12 (16 coils) 156 / 157 / 170; 12 x 1000 5056 / 5088 / 5780; 2000 x 12 221 /
+// 195 / 196; 2000 x 100 1021 / 716 / 725; 20000 x 12 999 / 663 / 664.
+#define GATE_GROUPS 2048
+int gate_per(long long nb, int frames) {
+  return (int)std::min<long long>(std::max<long long>(nb * frames / GATE_GROUPS, 1), frames);
 }
 
 double median_sorted(const std::vector<double> &v) {
@@ -283,6 +297,8 @@ int mrn_pregate(const mrn_gate_params *p, int64_t xres, int64_t R, const double 
   if (g.nb > 0x7fffffffll) return free_fail(MRN_EUNSUPPORTED, "too many samples");
   hipStream_t st = (hipStream_t)stream;
   const int64_t nflat = (int64_t)g.frames * g.nb;
+  const int per = gate_per(g.nb, g.frames);
+  const dim3 grid((unsigned)g.nb, (unsigned)((g.frames + per - 1) / per));
   int64_t *bcnt = nullptr;  // 64-bit: the scan accumulates in its input type
   int64_t *boff = nullptr, *fb = nullptr;
   void *tmp = nullptr;
@@ -295,8 +311,7 @@ int mrn_pregate(const mrn_gate_params *p, int64_t xres, int64_t R, const double 
     if ((e = hipMalloc(&boff, sizeof(int64_t) * (nflat + 1))) != hipSuccess) return e;
     if ((e = hipMalloc(&fb, sizeof(int64_t) * (g.frames + 1))) != hipSuccess) return e;
     if ((e = hipMemsetAsync(bcnt + nflat, 0, sizeof(int64_t), st)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_gate_count, dim3((unsigned)g.nb), dim3(256), 0, st, g, gt, resp, kx, ky, kz,
-                       bcnt);
+    hipLaunchKernelGGL(k_gate_count, grid, dim3(256), 0, st, g, gt, resp, kx, ky, kz, per, bcnt);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if ((e = hipcub::DeviceScan::ExclusiveSum(nullptr, tb, bcnt, boff, nflat + 1, st)) != hipSuccess) return e;
     if ((e = hipMalloc(&tmp, tb)) != hipSuccess) return e;
@@ -307,8 +322,8 @@ int mrn_pregate(const mrn_gate_params *p, int64_t xres, int64_t R, const double 
         hipSuccess)
       return e;
     if (fill) {
-      hipLaunchKernelGGL(k_gate_scatter, dim3((unsigned)g.nb), dim3(256), 0, st, g, gt, resp, kx, ky, kz,
-                         kw, C, (const float2 *)kdata, boff, fb, kx_out, ky_out, kz_out, kw_out, (float2 *)kdata_out);
+      hipLaunchKernelGGL(k_gate_scatter, grid, dim3(256), 0, st, g, gt, resp, kx, ky, kz,
+                         kw, C, (const float2 *)kdata, boff, fb, kx_out, ky_out, kz_out, kw_out, (float2 *)kdata_out, per);
       if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     return hipStreamSynchronize(st);

@@ -50,6 +50,25 @@ def test_pregate_bit_exact(vs, shape, kw_, with_resp):
         base += n[t]
 
 
+@pytest.mark.parametrize("R,T", [(1, 1), (1000, 1), (1000, 2), (1000, 5), (1030, 12), (2100, 3), (40, 300)])
+def test_pregate_frames_per_workgroup(R, T):
+    """Several frames to a workgroup, the last one with fewer, or one each where
+    the blocks are few: 1000 readouts of 256 samples have 1000 blocks, so 2 of 5
+    frames go together; 40 have 40."""
+    xres, C = 256, 2
+    kx, ky, kz, kw, kd = problem(R, xres, C)
+    times = RNG.uniform(0, 100, R)
+    p_o = orc.gate_params(T, vs="tornado", shape="vipr", kmax=45.0)
+    gt, _ = orc.gate_scale(p_o, times)
+    ref = orc.pregate(p_o, gt, kx, ky, kz, kw, kd)
+    n, frames = pregate(gate_params(T, vs="tornado", shape="vipr", kmax=45.0), dev(gt), dev(kx), dev(ky), dev(kz),
+                        dev(kw), dev(kd))
+    assert np.array_equal(np.array(n), ref[0])
+    for q in range(4):
+        assert np.array_equal(np.concatenate([f[q].cpu().numpy() for f in frames]), ref[1 + q][:sum(n)])
+    assert np.array_equal(np.concatenate([f[4].cpu().numpy().ravel() for f in frames]), ref[5][:C * sum(n)])
+
+
 def test_pregate_full_size_partition():
     """The bench trajectory (20000 readouts x 256 samples, 32 coils of k-space):
     without sharing every sample lands in exactly one of 20 frames and each
