@@ -29,6 +29,7 @@
 // fixed order, and rounds once.  The gather sums in the reference's tap order.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstdint>
@@ -391,7 +392,7 @@ constexpr int DM_CELLS = DM_X * 16;
 constexpr int DM_REACH = 5;    // last minus first tap on an axis, at most
 constexpr int DM_XT = DM_REACH + 1;
 constexpr int DM_BATCH = 32;   // visits weighted at a time
-constexpr int DM_ITEM = 2048;  // visits per work item
+constexpr int DM_ITEM = 2048;  // visits per work item, at most
 constexpr int DM_RUNS = 9;     // bin rows (z, y) of a tile
 // consecutive workgroups per XCD: neighbouring samples read the same cells, and
 // neighbouring tiles the same samples, through one L2
@@ -400,6 +401,7 @@ constexpr int DM_XRUN = 16;
 struct DmGeom {
   int nb[3], nt[3];  // bins and tiles per axis
   int reach;         // last minus first tap
+  int item;          // visits per work item
 };
 
 typedef double dm_v4d __attribute__((ext_vector_type(4)));
@@ -496,7 +498,7 @@ __global__ void k_dm_count(const int32_t *__restrict__ start, DmGeom m, int ntil
         const int64_t b = ((int64_t)z * m.nb[1] + y) * m.nb[0];
         v += start[b + x1 + 1] - start[b + x0];
       }
-    n = (int)((v + DM_ITEM - 1) / DM_ITEM);
+    n = (int)((v + m.item - 1) / m.item);
   }
   items[t] = n;
   slots[t] = n > 1 ? n : 0;
@@ -553,7 +555,7 @@ __global__ __launch_bounds__(256, 4) void k_dm_scatter(float *__restrict__ X, do
       total += n;
     }
   }
-  const int vbeg = it.y * DM_ITEM, vend = min(vbeg + DM_ITEM, total);
+  const int vbeg = it.y * m.item, vend = min(vbeg + m.item, total);
   auto load = [&](int v) -> float4 {  // visit v (the last one past the end)
     v = min(v, vend - 1);
     int q = add[0];
@@ -813,6 +815,16 @@ bool dm_fits(const DcfGeom &g, DmGeom &m) {
   return m.reach <= DM_REACH && bins < (1 << 30) && tiles < (1 << 30);
 }
 
+// Visits per work item.  An item is one wavefront's serial walk, so a dense
+// tile's must not outlast the rest of the launch: about 5 visits per sample over
+// the chip's 4096 wavefronts, in whole batches.  us per iteration at 128 / 512 /
+// 2048 visits per item and by this rule: 32^3, 10000 radial samples 31 / 47 / 107
+// / 31, 200000 78 / 72 / 141 / 70; 64^3, 50000 41 / 54 / 124 / 41; 128^3, 500000
+// 171 / 164 / 255 / 164; 256^3, 5 M 1450 / 1283 / 1264 / 1264.
+int dm_item(int64_t M) {
+  return (int)std::min<int64_t>(std::max<int64_t>(5 * M / 4096 / DM_BATCH * DM_BATCH, 128), DM_ITEM);
+}
+
 int dm_calc(const mrn_dcf_params *p, const DcfGeom &g, const DmGeom &m, int64_t M, const float *kx, const float *ky,
             const float *kz, float *kw, double *sums, const float *tab_h, hipStream_t st) {
   Scratch mem(st);
@@ -981,6 +993,7 @@ int mrn_dcf_calc(const mrn_dcf_params *p, int64_t M, const float *kx, const floa
   dcf_table(p->dwin, p->kernel, tab_h);
   DmGeom m;
   if (dm_fits(g, m)) {
+    m.item = dm_item(M);
     const int rc = dm_calc(p, g, m, M, kx, ky, kz, kw, sums, tab_h, st);
     delete[] tab_h;
     return rc;

@@ -14,7 +14,7 @@ import torch
 
 from oracle import oracle as orc
 from mri_recon_amd import MrnError, dcf_calc, dcf_params, synth
-from mri_recon_amd.dcf import dcf_grid_size
+from mri_recon_amd.dcf import dcf_grid_size, dcf_last_atomics
 from tests.helpers import rel
 
 pytestmark = pytest.mark.gpu
@@ -133,3 +133,46 @@ def test_dcf_tiles_match_oracle(N, spokes, npts, dwin, os_):
     ref, _ = orc.dcf_calc(p, kx[:-1], ky[:-1], kz[:-1], "f32")
     assert not got[-1] > 0  # the sample at infinity has no taps
     assert rel(got[:-1], ref) <= 3e-5
+
+
+def general(kx, ky, kz, **kw):
+    """The general form of the same calculation: a kernel scale that grows by
+    one part in 10^7 over |k| = 128."""
+    return dcf_calc(kx, ky, kz, acc=float(np.nextafter(np.float32(1), np.float32(2))), **kw)
+
+
+def best_ms(fn, reps=6):
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    best = 1e9
+    for _ in range(reps):
+        ev[0].record()
+        fn()
+        ev[1].record()
+        torch.cuda.synchronize()
+        best = min(best, ev[0].elapsed_time(ev[1]))
+    return best
+
+
+@pytest.mark.parametrize("N,spokes", [(32, 1500), (64, 800)])
+def test_dcf_dense_centre_is_not_slower_by_tiles(N, spokes):
+    """A small trajectory whose centre tiles hold thousands of visits: the tiles'
+    walks are short enough that the call is not slower than the general form
+    (with up to 2048 visits per walk it took 1.5 times as long)."""
+    k = [dev(v) for v in radial(spokes, N, N)]
+    t = best_ms(lambda: dcf_calc(*k, N=N, iters=20))
+    assert dcf_last_atomics() == 0
+    tg = best_ms(lambda: general(*k, N=N, iters=20))
+    assert dcf_last_atomics() > 0
+    print("dcf %d^3, %d spokes: %.2f ms, general %.2f" % (N, spokes, t, tg))
+    assert t <= 1.1 * tg
+
+
+@pytest.mark.parametrize("M", [100, 8191, 52000])
+def test_dcf_item_lengths_match_oracle(M):
+    """128 visits per work item up to 104857 samples, more beyond; here the tiles
+    hold fewer, about as many, and several times that."""
+    kx, ky, kz = [v[:M] for v in radial(M // 20 + 1, 20, 16)]
+    got = dcf_calc(dev(kx), dev(ky), dev(kz), N=16, iters=4).cpu().numpy()
+    assert dcf_last_atomics() == 0
+    ref, _ = orc.dcf_calc(orc.dcf_params(16, iters=4), kx, ky, kz, "f32")
+    assert rel(got, ref) <= 3e-5
