@@ -4,7 +4,8 @@
 //
 // Two forms.  With dcf_acc = 1 and half widths below 3 (the defaults) every
 // kernel has one width and the scatter is a matrix product per tile (k_dm_*).
-// Other settings take the general form: the samples sorted by 8x8x8-cell brick
+// Other settings, one or two iterations of few samples and samples too scattered
+// for the tiles take the general form: the samples sorted by 8x8x8-cell brick
 // of the grid and 4x4x4 sub-brick, so that a wavefront's samples touch
 // neighbouring cells, and scattered with float atomics.  Both sort once; the
 // iterations run on the sorted copy and the weights are put back in the
@@ -825,6 +826,26 @@ int dm_item(int64_t M) {
   return (int)std::min<int64_t>(std::max<int64_t>(5 * M / 4096 / DM_BATCH * DM_BATCH, 128), DM_ITEM);
 }
 
+// Whether a call of so many iterations takes the one-width form: it spends 50 to
+// 200 us more on its lists than the general form on its sort, and wins 50 us per
+// iteration on the smallest calls.  The call in us, general / one-width: 32^3,
+// 1000 samples 0 / 1 / 20 iterations 117 / 173, 200 / 219, 1784 / 715; 64^3, 50000
+// radial samples, 1 iteration 246 / 363; 2 M 1502 / 1398.
+bool dm_iters(int iters, int64_t M) { return iters >= 3 || iters * M >= (1 << 20); }
+
+// Whether its work items are too empty: an item costs a batch of 32 visits even
+// where scattered samples leave it with one or two.  Fitted to both forms' times
+// per iteration, general / one-width: 256^3, random samples 50000 253 / 288 us
+// (206193 items), 200000 507 / 662 (499762), 500000 905 / 896 (621276), 2 M 2850 /
+// 1268; 256^3 radial 200000 446 / 194 (108247); 384^3 random 50000 447 / 319
+// (235967), 500000 1179 / 1807 (1455385), 2 M 3283 / 3096 (2090240).
+bool dm_sparse(const DcfGeom &g, int64_t M, int64_t items) {
+  const int64_t cells = (int64_t)g.S[0] * g.S[1] * g.S[2];
+  return items > M * 6 / 7 + cells / 2000 + 50000;
+}
+
+// A status that is none of the interface's: the call goes on in the general form.
+constexpr int DM_GENERAL = -1;
 int dm_calc(const mrn_dcf_params *p, const DcfGeom &g, const DmGeom &m, int64_t M, const float *kx, const float *ky,
             const float *kz, float *kw, double *sums, const float *tab_h, hipStream_t st) {
   Scratch mem(st);
@@ -837,7 +858,6 @@ int dm_calc(const mrn_dcf_params *p, const DcfGeom &g, const DmGeom &m, int64_t 
   int *nheavy_d;
   double *dsum, *part;
   uint8_t *tmp;
-  DCF_HIP(mem.get(X, (int64_t)g.S[0] * g.S[1] * g.S[2]));
   DCF_HIP(mem.get(tab, g.len));
   DCF_HIP(mem.get(dsum, p->iters));
   DCF_HIP(mem.get(coords, M));
@@ -874,6 +894,8 @@ int dm_calc(const mrn_dcf_params *p, const DcfGeom &g, const DmGeom &m, int64_t 
   DCF_HIP(hipMemcpyAsync(&nitems, ofs + ntiles, sizeof(int32_t), hipMemcpyDeviceToHost, st));
   DCF_HIP(hipMemcpyAsync(&nslots, slot0 + ntiles, sizeof(int32_t), hipMemcpyDeviceToHost, st));
   DCF_HIP(hipStreamSynchronize(st));
+  if (dm_sparse(g, M, nitems)) return DM_GENERAL;
+  DCF_HIP(mem.get(X, (int64_t)g.S[0] * g.S[1] * g.S[2]));
   DCF_HIP(mem.get(list, nitems));
   DCF_HIP(mem.get(heavy, nslots));  // at least two slots per split tile
   DCF_HIP(mem.get(part, (int64_t)nslots * DM_CELLS));
@@ -992,11 +1014,13 @@ int mrn_dcf_calc(const mrn_dcf_params *p, int64_t M, const float *kx, const floa
   float *tab_h = new float[len];
   dcf_table(p->dwin, p->kernel, tab_h);
   DmGeom m;
-  if (dm_fits(g, m)) {
+  if (dm_iters(p->iters, M) && dm_fits(g, m)) {
     m.item = dm_item(M);
     const int rc = dm_calc(p, g, m, M, kx, ky, kz, kw, sums, tab_h, st);
-    delete[] tab_h;
-    return rc;
+    if (rc != DM_GENERAL) {
+      delete[] tab_h;
+      return rc;
+    }
   }
   float *X = nullptr, *tab = nullptr, *srt = nullptr;  // srt: sorted kx, ky, kz, kw
   uint32_t *keys = nullptr, *perm = nullptr;           // [2][M] each

@@ -176,3 +176,23 @@ def test_dcf_item_lengths_match_oracle(M):
     assert dcf_last_atomics() == 0
     ref, _ = orc.dcf_calc(orc.dcf_params(16, iters=4), kx, ky, kz, "f32")
     assert rel(got, ref) <= 3e-5
+
+
+@pytest.mark.parametrize("N,M,kind,iters,tiles", [
+    (24, 5000, "radial", 0, False), (24, 5000, "radial", 2, False), (24, 5000, "radial", 3, True),
+    (24, 524288, "radial", 1, False), (24, 524288, "radial", 2, True),   # iters * M at 2^20
+    (256, 200000, "random", 3, False), (256, 200000, "radial", 3, True), (128, 200000, "random", 3, True)])
+def test_dcf_form_rule(N, M, kind, iters, tiles):
+    """Which calls go by tiles: from 3 iterations or 2^20 sample visits on, and
+    not with samples so scattered that the tiles' items are nearly empty.  Both
+    forms' weights agree (to their summation order)."""
+    if kind == "radial":
+        kx, ky, kz = radial(-(-M // N), N, N)
+    else:
+        kx, ky, kz = np.random.default_rng(5).uniform(-N / 2, N / 2, (3, M)).astype(np.float32)
+    k = [dev(v[:M]) for v in (kx, ky, kz)]
+    got = dcf_calc(*k, N=N, iters=iters).cpu().numpy()
+    if iters > 0:
+        assert (dcf_last_atomics() == 0) == tiles
+    ref = general(*k, N=N, iters=iters).cpu().numpy()
+    assert rel(got, ref) <= 1e-4
