@@ -4,8 +4,9 @@
 //
 // Two forms.  With dcf_acc = 1 and half widths below 3 (the defaults) every
 // kernel has one width and the scatter is a matrix product per tile (k_dm_*).
-// Other settings, one or two iterations of few samples and samples too scattered
-// for the tiles take the general form: the samples sorted by 8x8x8-cell brick
+// Other settings, one or two iterations of few samples, samples too scattered
+// for the tiles, and calls without the memory for the tiles' lists take the
+// general form: the samples sorted by 8x8x8-cell brick
 // of the grid and 4x4x4 sub-brick, so that a wavefront's samples touch
 // neighbouring cells, and scattered with float atomics.  Both sort once; the
 // iterations run on the sorted copy and the weights are put back in the
@@ -37,7 +38,6 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
-#include <vector>
 
 #include <hipcub/hipcub.hpp>
 
@@ -781,21 +781,24 @@ int64_t nblocks(int64_t n, int b) { return (n + b - 1) / b; }
 
 // Device memory of one call, freed with it.
 struct Scratch {
-  std::vector<void *> p;
+  void *p[20];
+  int n = 0;
   hipStream_t st;
   explicit Scratch(hipStream_t s) : st(s) {}
   Scratch(const Scratch &) = delete;
   template <class T>
-  hipError_t get(T *&q, int64_t n) {
+  hipError_t get(T *&q, int64_t count) {
+    q = nullptr;
+    if (n == (int)(sizeof(p) / sizeof(p[0]))) return hipErrorInvalidValue;
     void *v = nullptr;
-    const hipError_t e = hipMalloc(&v, sizeof(T) * (size_t)(n > 0 ? n : 1));
-    if (e == hipSuccess) p.push_back(v);
+    const hipError_t e = dev_malloc(&v, sizeof(T) * (size_t)(count > 0 ? count : 1));
+    if (e == hipSuccess) p[n++] = v;
     q = (T *)v;
     return e;
   }
   ~Scratch() {
-    if (!p.empty()) (void)hipStreamSynchronize(st);
-    for (void *v : p) hipFree(v);
+    if (n > 0) (void)hipStreamSynchronize(st);
+    for (int i = 0; i < n; i++) hipFree(p[i]);
   }
 };
 
@@ -846,6 +849,16 @@ bool dm_sparse(const DcfGeom &g, int64_t M, int64_t items) {
 
 // A status that is none of the interface's: the call goes on in the general form.
 constexpr int DM_GENERAL = -1;
+#define DM_MEM(call)                                  \
+  do {                                                \
+    const hipError_t m_ = (call);                     \
+    if (m_ == hipErrorOutOfMemory) {                  \
+      (void)hipGetLastError();                        \
+      return DM_GENERAL;                              \
+    }                                                 \
+    DCF_HIP(m_);                                      \
+  } while (0)
+
 int dm_calc(const mrn_dcf_params *p, const DcfGeom &g, const DmGeom &m, int64_t M, const float *kx, const float *ky,
             const float *kz, float *kw, double *sums, const float *tab_h, hipStream_t st) {
   Scratch mem(st);
@@ -858,17 +871,17 @@ int dm_calc(const mrn_dcf_params *p, const DcfGeom &g, const DmGeom &m, int64_t 
   int *nheavy_d;
   double *dsum, *part;
   uint8_t *tmp;
-  DCF_HIP(mem.get(tab, g.len));
-  DCF_HIP(mem.get(dsum, p->iters));
-  DCF_HIP(mem.get(coords, M));
-  DCF_HIP(mem.get(keys, 2 * M));
-  DCF_HIP(mem.get(perm, 2 * M));
-  DCF_HIP(mem.get(start, (int64_t)nbins + 1));
-  DCF_HIP(mem.get(items, (int64_t)ntiles + 1));
-  DCF_HIP(mem.get(ofs, (int64_t)ntiles + 1));
-  DCF_HIP(mem.get(slots, (int64_t)ntiles + 1));
-  DCF_HIP(mem.get(slot0, (int64_t)ntiles + 1));
-  DCF_HIP(mem.get(nheavy_d, 1));
+  DM_MEM(mem.get(tab, g.len));
+  DM_MEM(mem.get(dsum, p->iters));
+  DM_MEM(mem.get(coords, M));
+  DM_MEM(mem.get(keys, 2 * M));
+  DM_MEM(mem.get(perm, 2 * M));
+  DM_MEM(mem.get(start, (int64_t)nbins + 1));
+  DM_MEM(mem.get(items, (int64_t)ntiles + 1));
+  DM_MEM(mem.get(ofs, (int64_t)ntiles + 1));
+  DM_MEM(mem.get(slots, (int64_t)ntiles + 1));
+  DM_MEM(mem.get(slot0, (int64_t)ntiles + 1));
+  DM_MEM(mem.get(nheavy_d, 1));
   DCF_HIP(hipMemcpyAsync(tab, tab_h, sizeof(float) * g.len, hipMemcpyHostToDevice, st));
   const size_t lds = sizeof(float) * g.len;
   const dim3 gs((unsigned)nblocks(M, 256));
@@ -880,7 +893,7 @@ int dm_calc(const mrn_dcf_params *p, const DcfGeom &g, const DmGeom &m, int64_t 
   DCF_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, keys, keys + M, perm, perm + M, (int)M, 0, bits, st));
   DCF_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, sb, items, ofs, ntiles + 1, st));
   tb = tb > sb ? tb : sb;
-  DCF_HIP(mem.get(tmp, (int64_t)tb));
+  DM_MEM(mem.get(tmp, (int64_t)tb));
   DCF_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, keys, keys + M, perm, perm + M, (int)M, 0, bits, st));
   const uint32_t *order = perm + M;
   hipLaunchKernelGGL(k_dm_coords, gs, dim3(256), 0, st, order, kx, ky, kz, M, g, coords);
@@ -895,10 +908,10 @@ int dm_calc(const mrn_dcf_params *p, const DcfGeom &g, const DmGeom &m, int64_t 
   DCF_HIP(hipMemcpyAsync(&nslots, slot0 + ntiles, sizeof(int32_t), hipMemcpyDeviceToHost, st));
   DCF_HIP(hipStreamSynchronize(st));
   if (dm_sparse(g, M, nitems)) return DM_GENERAL;
-  DCF_HIP(mem.get(X, (int64_t)g.S[0] * g.S[1] * g.S[2]));
-  DCF_HIP(mem.get(list, nitems));
-  DCF_HIP(mem.get(heavy, nslots));  // at least two slots per split tile
-  DCF_HIP(mem.get(part, (int64_t)nslots * DM_CELLS));
+  DM_MEM(mem.get(X, (int64_t)g.S[0] * g.S[1] * g.S[2]));
+  DM_MEM(mem.get(list, nitems));
+  DM_MEM(mem.get(heavy, nslots));  // at least two slots per split tile
+  DM_MEM(mem.get(part, (int64_t)nslots * DM_CELLS));
   hipLaunchKernelGGL(k_dm_items, dim3((unsigned)nblocks(ntiles, 256)), dim3(256), 0, st, items, ofs, slot0, ntiles, list);
   hipLaunchKernelGGL(k_dcf_fill, dim3(1), dim3(1), 0, st, reinterpret_cast<float *>(nheavy_d), (int64_t)1, 0.0f);
   int nheavy = 0;

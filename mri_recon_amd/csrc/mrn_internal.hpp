@@ -83,6 +83,10 @@ struct FrameDev {
   int ngrp, nheavy, nwide, wide_each;
 };
 
+// hipMalloc of the arrays whose absence has a way out.  MRN_ALLOC_MAX (bytes, for
+// the tests of those ways) makes larger requests fail as if there were no memory.
+hipError_t dev_malloc(void **p, size_t bytes);
+
 // Device arrays that only grow: binding a trajectory no larger than an
 // earlier one of the same op reuses their memory, with no hipFree/hipMalloc
 // (each of which waits for the whole device).  grow() keeps the contents only
@@ -94,7 +98,7 @@ inline hipError_t grow(T *&p, size_t &cap, int64_t n) {
   hipFree(p);
   p = nullptr;
   cap = 0;
-  const hipError_t e = hipMalloc((void **)&p, sizeof(T) * want);
+  const hipError_t e = dev_malloc((void **)&p, sizeof(T) * want);
   if (e == hipSuccess) cap = want;
   return e;
 }

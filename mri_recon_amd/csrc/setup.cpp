@@ -24,6 +24,15 @@ int fail(mrn_op *op, int code, const char *msg) {
   return code;
 }
 
+hipError_t dev_malloc(void **p, size_t bytes) {
+  const char *s = getenv("MRN_ALLOC_MAX");
+  if (s && *s && bytes > strtoull(s, nullptr, 10)) {
+    *p = nullptr;
+    return hipErrorOutOfMemory;
+  }
+  return hipMalloc(p, bytes);
+}
+
 // Modified Bessel I0, Abramowitz & Stegun 9.8.1 / 9.8.2 (double polynomial,
 // float result, as the reference evaluates it).
 static float host_i0(float x) {

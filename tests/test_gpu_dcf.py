@@ -196,3 +196,14 @@ def test_dcf_form_rule(N, M, kind, iters, tiles):
         assert (dcf_last_atomics() == 0) == tiles
     ref = general(*k, N=N, iters=iters).cpu().numpy()
     assert rel(got, ref) <= 1e-4
+
+
+def test_dcf_without_memory_for_the_tiles(monkeypatch):
+    """The tiles' lists take memory the general form does not: without it the
+    call is the general form's, not an error."""
+    kx, ky, kz = radial(400, 60, 24)
+    monkeypatch.setenv("MRN_ALLOC_MAX", "100000")
+    got = dcf_calc(dev(kx), dev(ky), dev(kz), N=24, iters=4).cpu().numpy()
+    assert dcf_last_atomics() > 0
+    ref, _ = orc.dcf_calc(orc.dcf_params(24, iters=4), kx, ky, kz, "f32")
+    assert rel(got, ref) <= 3e-5
