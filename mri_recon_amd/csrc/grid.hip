@@ -2276,20 +2276,30 @@ __global__ void k_plane_yrange(int2 *xrng, int S1, int S2, int2 *yrng) {
     if (y < y0 || y > y1) row[y] = make_int2(INT_MAX, INT_MIN);
 }
 
+// The work list's lengths, for one copy to the host.
+__global__ void k_lengths(const int32_t *slots, const int32_t *items, const int64_t *visits, int64_t *out) {
+  out[0] = *slots;
+  out[1] = *items;
+  out[2] = *visits;
+}
+
 // Cost of scatter work item i (entry n: 0, for the exclusive scan): its
 // visits plus a fixed part for the tile's epilogue stores.
+#define ITEM_COST 32
 __global__ void k_item_cost(const int4 *__restrict__ subs, int n, int64_t *cost) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) cost[i] = max(subs[i].z - subs[i].y, 0) + 32;
+  if (i < n) cost[i] = max(subs[i].z - subs[i].y, 0) + ITEM_COST;
   else if (i == n) cost[i] = 0;
 }
 
 // Groups of consecutive work items of equal cost (pre: exclusive prefix of the
 // costs): group q starts at the first item whose prefix reaches q * per.  An
 // item longer than `per` leaves empty groups behind it.  start[ngrp] = n.
-// per = 0: every item a group of its own.
-__global__ void k_group_start(const int64_t *__restrict__ pre, int n, int64_t per, int ngrp, int32_t *start) {
+// per = 0: every item a group of its own (pre is not read).
+// xs: the boundaries of MRN_XCDS equal ranges of the groups.
+__global__ void k_group_start(const int64_t *__restrict__ pre, int n, int64_t per, int ngrp, int32_t *start, int32_t *xs) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= MRN_XCDS) xs[i] = (int32_t)((int64_t)ngrp * i / MRN_XCDS);
   if (i > n) return;
   if (per == 0) {
     start[i] = i;
@@ -2507,16 +2517,32 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
   MRN_BH(hipMemsetAsync(b.slots, 0, sizeof(int32_t) * (nt + 1), st));
   // work items, with room for the split tiles' partial sums: where that takes
   // more than a quarter of the grids (or is not to be had) the items are made longer, in the
-  // end one per tile
+  // end one per tile.  The visit list's offsets are 64-bit (about 8 visits per
+  // sample); it is filled once the work items exist.  One copy brings every length.
+  MRN_BH(grow(fr.vofs, cp.vofs, (int64_t)nt + 1));
+  MRN_BH(grow(b.vw, b.c_vw, (int64_t)nt + 1));
+  size_t vb = 0;
+  MRN_BH(hipcub::DeviceScan::ExclusiveSum(nullptr, vb, b.vw, fr.vofs, nt + 1, st));
+  MRN_BH(grow(b.vtmp, b.c_vtmp, (int64_t)vb));
+  MRN_BH(grow(b.len, b.c_len, 3));
+  int64_t nvisits = 0;
+  int32_t nsub_total = 0;
   for (;;) {
     hipLaunchKernelGGL(k_tile_nsub, dim3(nblk(nt, 256)), dim3(256), 0, st, fr.bin_start, t, nsub, visits, b.slots,
                        fft_x_pruned(op) ? fr.xrng : nullptr, g.S[1], g.S[2]);
+    hipLaunchKernelGGL(k_widen, dim3(nblk((int64_t)nt + 1, 256)), dim3(256), 0, st, visits, nt, b.vw);
     MRN_BH(hipGetLastError());
     MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.tmp, tb, b.slots, b.slot0, nt + 1, st));
-    int32_t ns = 0;
-    MRN_BH(hipMemcpyAsync(&ns, b.slot0 + nt, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.tmp, tb, nsub, off, nt + 1, st));
+    MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.vtmp, vb, b.vw, fr.vofs, nt + 1, st));
+    hipLaunchKernelGGL(k_lengths, dim3(1), dim3(1), 0, st, b.slot0 + nt, off + nt, fr.vofs + nt, b.len);
+    MRN_BH(hipGetLastError());
+    int64_t len[3];  // partial-sum slots, work items, visits
+    MRN_BH(hipMemcpyAsync(len, b.len, sizeof(len), hipMemcpyDeviceToHost, st));
     MRN_BH(hipStreamSynchronize(st));
-    const int64_t elems = (int64_t)ns * op->nch * 64 * g.CC, cells = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC * op->nch;
+    nsub_total = (int32_t)len[1];
+    nvisits = len[2];
+    const int64_t elems = len[0] * op->nch * 64 * g.CC, cells = (int64_t)g.S[0] * g.S[1] * g.S[2] * g.CC * op->nch;
     hipError_t e = hipErrorOutOfMemory;
     if ((size_t)elems <= op->part_cap) {
       e = hipSuccess;
@@ -2524,7 +2550,7 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
       // the other frames' slots must keep fitting: the old buffer goes only
       // once the larger one is there
       float2 *p = nullptr;
-      e = hipMalloc((void **)&p, sizeof(float2) * elems);
+      e = dev_malloc((void **)&p, sizeof(float2) * elems);
       if (e == hipSuccess) {
         hipFree(op->part);
         op->part = p;
@@ -2532,34 +2558,14 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
       }
     }
     if (e == hipSuccess) {
-      fr.nslots = ns;
+      fr.nslots = (int)len[0];
       break;
     }
-    if (e != hipErrorOutOfMemory || ns == 0) MRN_BH(e);
+    if (e != hipErrorOutOfMemory || len[0] == 0) MRN_BH(e);
     (void)hipGetLastError();
     t.maxv = t.maxv > (1 << 29) ? INT32_MAX : t.maxv * 2;
   }
-  // visit list (offsets in 64 bits: about 8 visits per sample); it is
-  // filled once the work items exist
-  int64_t nvisits = 0;
-  {
-    MRN_BH(grow(fr.vofs, cp.vofs, (int64_t)nt + 1));
-    MRN_BH(grow(b.vw, b.c_vw, (int64_t)nt + 1));
-    hipLaunchKernelGGL(k_widen, dim3(nblk((int64_t)nt + 1, 256)), dim3(256), 0, st, visits, nt, b.vw);
-    size_t vb = 0;
-    MRN_BH(hipcub::DeviceScan::ExclusiveSum(nullptr, vb, b.vw, fr.vofs, nt + 1, st));
-    MRN_BH(grow(b.vtmp, b.c_vtmp, (int64_t)vb));
-    MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.vtmp, vb, b.vw, fr.vofs, nt + 1, st));
-    int64_t nv = 0;
-    MRN_BH(hipMemcpyAsync(&nv, fr.vofs + nt, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    MRN_BH(hipStreamSynchronize(st));
-    MRN_BH(grow(fr.vlist, cp.vlist, nv));
-    nvisits = nv;
-  }
-  MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.tmp, tb, nsub, off, nt + 1, st));
-  int32_t nsub_total = 0;
-  MRN_BH(hipMemcpyAsync(&nsub_total, off + nt, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  MRN_BH(hipStreamSynchronize(st));
+  MRN_BH(grow(fr.vlist, cp.vlist, nvisits));
   MRN_BH(grow(fr.subs, cp.subs, nsub_total));
   fr.nsub = nsub_total;
   hipLaunchKernelGGL(k_fill_subs, dim3(nblk(nt, 256)), dim3(256), 0, st, nsub, off, visits, b.slot0, t,
@@ -2573,28 +2579,25 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
   // the work list in groups of equal cost, and those in MRN_XCDS ranges (xcd_run < 0)
   {
     const int64_t n = nsub_total;
-    MRN_BH(grow(b.icost, b.c_icost, n + 1));
-    MRN_BH(grow(b.ipre, b.c_ipre, n + 1));
     MRN_BH(grow(fr.xsplit, cp.xsplit, MRN_XCDS + 1));
-    hipLaunchKernelGGL(k_item_cost, dim3(nblk(n + 1, 256)), dim3(256), 0, st, fr.subs, (int)n, b.icost);
-    MRN_BH(hipGetLastError());
-    size_t cb = 0;
-    MRN_BH(hipcub::DeviceScan::ExclusiveSum(nullptr, cb, b.icost, b.ipre, (int)n + 1, st));
-    MRN_BH(grow(b.vtmp, b.c_vtmp, (int64_t)cb));
-    MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.vtmp, cb, b.icost, b.ipre, (int)n + 1, st));
-    int64_t total = 0;
-    MRN_BH(hipMemcpyAsync(&total, b.ipre + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    MRN_BH(hipStreamSynchronize(st));
+    const int64_t total = nvisits + ITEM_COST * n;  // every tile with visits has items
     fr.groups = group_items(op, fr.Mv, n, total);
     const int64_t per = fr.groups ? group_cost(total) : 0;
     fr.ngrp = n == 0 ? 0 : fr.groups ? (int)(total / per + 1) : (int)n;
+    if (fr.groups) {
+      MRN_BH(grow(b.icost, b.c_icost, n + 1));
+      MRN_BH(grow(b.ipre, b.c_ipre, n + 1));
+      hipLaunchKernelGGL(k_item_cost, dim3(nblk(n + 1, 256)), dim3(256), 0, st, fr.subs, (int)n, b.icost);
+      MRN_BH(hipGetLastError());
+      size_t cb = 0;
+      MRN_BH(hipcub::DeviceScan::ExclusiveSum(nullptr, cb, b.icost, b.ipre, (int)n + 1, st));
+      MRN_BH(grow(b.vtmp, b.c_vtmp, (int64_t)cb));
+      MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.vtmp, cb, b.icost, b.ipre, (int)n + 1, st));
+    }
     MRN_BH(grow(fr.gstart, cp.gstart, (int64_t)fr.ngrp + 1));
-    hipLaunchKernelGGL(k_group_start, dim3(nblk(n + 1, 256)), dim3(256), 0, st, b.ipre, (int)n, per, fr.ngrp, fr.gstart);
+    hipLaunchKernelGGL(k_group_start, dim3(nblk(std::max<int64_t>(n, MRN_XCDS) + 1, 256)), dim3(256), 0, st, b.ipre,
+                       (int)n, per, fr.ngrp, fr.gstart, fr.xsplit);
     MRN_BH(hipGetLastError());
-    int32_t xs[MRN_XCDS + 1];
-    for (int x = 0; x <= MRN_XCDS; x++) xs[x] = (int32_t)((int64_t)fr.ngrp * x / MRN_XCDS);
-    MRN_BH(hipMemcpyAsync(fr.xsplit, xs, sizeof(xs), hipMemcpyHostToDevice, st));
-    MRN_BH(hipStreamSynchronize(st));
     fr.xsplit_max = (fr.ngrp + MRN_XCDS - 1) / MRN_XCDS;
   }
   MRN_BH(hipcub::DeviceScan::ExclusiveSum(b.tmp, tb, hflag, hoff, nt + 1, st));

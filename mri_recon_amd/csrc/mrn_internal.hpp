@@ -115,14 +115,14 @@ struct BindScratch {
   int32_t *vals = nullptr, *counts = nullptr, *nsub = nullptr, *visits = nullptr, *off = nullptr,
           *hflag = nullptr, *hoff = nullptr, *wflag = nullptr, *woff = nullptr, *slots = nullptr, *slot0 = nullptr;
   int2 *brow = nullptr;
-  int64_t *vw = nullptr, *icost = nullptr, *ipre = nullptr;
+  int64_t *vw = nullptr, *icost = nullptr, *ipre = nullptr, *len = nullptr;
   uint8_t *tmp = nullptr, *wtmp = nullptr, *vtmp = nullptr;
   size_t c_keys = 0, c_keys2 = 0, c_vals = 0, c_counts = 0, c_nsub = 0, c_visits = 0, c_off = 0, c_hflag = 0,
          c_hoff = 0, c_wflag = 0, c_woff = 0, c_brow = 0, c_vw = 0, c_icost = 0, c_ipre = 0, c_tmp = 0, c_wtmp = 0,
-         c_vtmp = 0, c_slots = 0, c_slot0 = 0;
+         c_vtmp = 0, c_slots = 0, c_slot0 = 0, c_len = 0;
   void release() {
     void *ps[] = {keys, keys2, vals, counts, nsub, visits, off, hflag, hoff, wflag, woff, brow, vw, icost, ipre,
-                  tmp, wtmp, vtmp, slots, slot0};
+                  tmp, wtmp, vtmp, slots, slot0, len};
     for (void *q : ps) hipFree(q);
     *this = BindScratch{};
   }
