@@ -181,16 +181,19 @@ static int fused_prepare(mrn_op *op, hipStream_t st) {
     if (!op->frames[f].has_traj) return MRN_OK;  // not ready: frame by frame
   int64_t tot = 0;
   for (int f = 0; f < F; f++) tot += op->frames[f].Mv * g.CC * op->nch;
-  if (tot > op->kwork_all_cap || !op->kwork_all) {
-    hipFree(op->kwork_all);
-    op->kwork_all = nullptr;
-    op->kwork_all_cap = 0;
-    MRN_HIP(op, hipMalloc(&op->kwork_all, sizeof(float2) * (tot > 0 ? tot : 1)));
-    op->kwork_all_cap = tot;
-  }
   int64_t ptot = 0;
   for (int f = 0; f < F; f++) ptot += (int64_t)op->frames[f].nslots * op->nch * 64 * g.CC;
-  MRN_HIP(op, grow(op->part_all, op->part_all_cap, ptot));
+  hipError_t e = grow(op->kwork_all, op->kwork_all_cap, tot);
+  if (e == hipSuccess) e = grow(op->part_all, op->part_all_cap, ptot);
+  if (e == hipErrorOutOfMemory) {  // no memory to take the frames together: one by one, in the arrays of the largest
+    (void)hipGetLastError();
+    hipFree(op->kwork_all);
+    hipFree(op->part_all);
+    op->kwork_all = op->part_all = nullptr;
+    op->kwork_all_cap = op->part_all_cap = 0;
+    return MRN_OK;
+  }
+  MRN_HIP(op, e);
   if (!op->fdev) MRN_HIP(op, hipMalloc(&op->fdev, sizeof(FrameDev) * F));
   const int64_t nrow = (int64_t)g.S[1] * g.S[2];
   if (fft_x_pruned(op)) {

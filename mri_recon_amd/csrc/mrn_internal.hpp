@@ -192,7 +192,7 @@ struct mrn_op {
   float2 *part_all = nullptr;  // ... of every frame, frame after frame (fused launches)
   size_t part_all_cap = 0;
   float2 *kwork_all = nullptr; // frames' k-space work arrays, frame after frame
-  int64_t kwork_all_cap = 0;   // elements
+  size_t kwork_all_cap = 0;    // elements
   int2 *xrng_all = nullptr;    // [F][Sz][Sy] x support rows (k_row_xrange) of every frame
   int2 *yrng_all = nullptr;    // [F][Sz] y support of every frame, when the y passes are pruned
   int fmax_ngrp = 0, fmax_nheavy = 0, fmax_nwide = 0, fmax_neach = 0, fmax_xsplit = 0;
