@@ -482,12 +482,8 @@ static int adjoint_data_frame(mrn_op *op, int f, float2 *R, hipStream_t st) {
 
 static int ensure_solver(mrn_op *op) {
   const int64_t n = (int64_t)op->F * op->nvox;
-  if (!op->vR) {
-    MRN_HIP(op, hipMalloc(&op->vR, sizeof(float2) * n));
-    MRN_HIP(op, hipMalloc(&op->vP, sizeof(float2) * n));
-    MRN_HIP(op, hipMalloc(&op->vL, sizeof(float2) * n));
-    MRN_HIP(op, hipMalloc(&op->vX0, sizeof(float2) * n));
-  }
+  for (float2 **v : {&op->vR, &op->vP, &op->vL, &op->vX0})
+    if (!*v) MRN_HIP(op, dev_malloc((void **)v, sizeof(float2) * n));
   if (!op->dtrace) {
     MRN_HIP(op, hipMalloc(&op->dtrace, sizeof(double) * 4 * MRN_TRACE_CAP));
     op->dtrace_cap = MRN_TRACE_CAP;
@@ -507,6 +503,69 @@ static int copy_trace(mrn_op *op, double *host, int64_t first, int64_t count, in
   }
   MRN_HIP(op, hipStreamSynchronize(st));
   return MRN_OK;
+}
+
+// A bound frame's lists and arrays from its stored trajectory (and data).
+static int bind_frame(mrn_op *op, FrameData &fr, hipStream_t st) {
+  MRN_TRY(ensure_grid(op));
+  MRN_TRY(build_bins(op, fr, fr.M, fr.traw, fr.traw + fr.M, fr.traw + 2 * fr.M, fr.traw + 3 * fr.M, st));
+  fr.has_traj = false;  // until all of it is there
+  const int64_t need = fr.Mv * op->g.CC * op->nch, had = op->kwork_cap;
+  if (need > had || !op->kwork) {
+    hipFree(op->kwork);
+    op->kwork = nullptr;
+    op->kwork_cap = 0;
+    auto get = [&](int64_t n) -> int {
+      MRN_HIP(op, dev_malloc((void **)&op->kwork, sizeof(float2) * (n > 0 ? n : 1)));
+      op->kwork_cap = n;
+      return MRN_OK;
+    };
+    const int rc = get(need);
+    if (rc != MRN_OK) {  // the other frames keep theirs, or are not bound any more
+      const std::string e = op->err;
+      if (get(had) != MRN_OK)
+        for (auto &f : op->frames) f.has_traj = false;
+      return fail(op, rc, e.c_str());
+    }
+  }
+  if (fr.has_kdata) {  // re-sort stored data for the new trajectory
+    MRN_HIP(op, grow(fr.kdata, fr.cap.kdata, need));
+    MRN_TRY(op_permute_in(op, fr.kdata, fr.kraw, fr, st));
+  }
+  fr.has_traj = true;
+  return MRN_OK;
+}
+
+// Runs fn.  If it failed for want of device memory, gives back what the op can do
+// without -- the wavelet step's second image, then the padding of its coil
+// blocks -- and runs it again.  fn starts over from its arguments.
+template <class Fn>
+static int with_room(mrn_op *op, hipStream_t st, Fn fn) {
+  op->oom = false;
+  int rc = fn();
+  if (rc != MRN_OK && op->oom && op->wave_T) {
+    MRN_HIP(op, hipDeviceSynchronize());
+    hipFree(op->wave_T);
+    op->wave_T = nullptr;
+    op->wave_T_cap = 0;
+    op->oom = false;
+    rc = fn();
+  }
+  if (rc != MRN_OK && op->oom && can_unpad(op)) {
+    std::vector<FrameData *> bound;
+    for (auto &fr : op->frames)
+      if (fr.has_traj) bound.push_back(&fr);
+    const std::string e = op->err;
+    const int un = unpad_blocks(op, st);
+    for (FrameData *fr : bound)  // without the memory for it a frame stays unbound
+      if (bind_frame(op, *fr, st) != MRN_OK) fr->has_traj = false;
+    if (un != MRN_OK) return fail(op, rc, e.c_str());
+    for (FrameData *fr : bound)
+      if (!fr->has_traj) return fail(op, rc, e.c_str());
+    op->oom = false;
+    rc = fn();
+  }
+  return rc;
 }
 
 static void drop_cg_graph(mrn_op *op) {
@@ -564,38 +623,32 @@ int mrn_set_traj(mrn_op *op, int f, int64_t M, const float *kx, const float *ky,
   // the frame's arrays are reused when large enough: first let every launch
   // that may still read the old trajectory finish
   MRN_HIP(op, hipDeviceSynchronize());
-  MRN_HIP(op, grow(fr.traw, fr.cap.traw, 4 * M));
-  const float *src[4] = {kx, ky, kz, kw};
-  for (int q = 0; q < 4; q++)
-    if (M > 0) MRN_HIP(op, hipMemcpyAsync(fr.traw + q * M, src[q], sizeof(float) * M, hipMemcpyDeviceToDevice, st));
-  fr.M = M;
-  // stored data of another sample count no longer matches the trajectory
-  // (kraw is [C][kraw_M]): the caller sets it again
-  if (fr.has_kdata && fr.kraw_M != M) fr.has_kdata = false;
-  if (batched(op)) {
-    MRN_TRY(build_bins(op, fr, M, fr.traw, fr.traw + M, fr.traw + 2 * M, fr.traw + 3 * M, st));
-    const int64_t need = fr.Mv * op->g.CC * op->nch;
-    if (need > op->kwork_cap) {
-      hipFree(op->kwork);
-      op->kwork = nullptr;
-      MRN_HIP(op, hipMalloc(&op->kwork, sizeof(float2) * (need > 0 ? need : 1)));
-      op->kwork_cap = need;
-    }
-    if (fr.has_kdata) {  // re-sort stored data for the new trajectory
-      MRN_HIP(op, grow(fr.kdata, fr.cap.kdata, need));
-      MRN_TRY(op_permute_in(op, fr.kdata, fr.kraw, fr, st));
-    }
-  }
-  if (M > op->kplain_cap) {
-    hipFree(op->kplain);
-    op->kplain = nullptr;
-    MRN_HIP(op, hipMalloc(&op->kplain, sizeof(float2) * M));
-    op->kplain_cap = M;
-  }
-  fr.has_traj = true;
+  fr.has_traj = false;
   op->version++;
-  MRN_HIP(op, hipStreamSynchronize(st));
-  return MRN_OK;
+  return with_room(op, st, [&]() -> int {
+    MRN_HIP(op, grow(fr.traw, fr.cap.traw, 4 * M));
+    const float *src[4] = {kx, ky, kz, kw};
+    for (int q = 0; q < 4; q++)
+      if (M > 0) MRN_HIP(op, hipMemcpyAsync(fr.traw + q * M, src[q], sizeof(float) * M, hipMemcpyDeviceToDevice, st));
+    fr.M = M;
+    // stored data of another sample count no longer matches the trajectory
+    // (kraw is [C][kraw_M]): the caller sets it again
+    if (fr.has_kdata && fr.kraw_M != M) fr.has_kdata = false;
+    if (M > op->kplain_cap) {
+      hipFree(op->kplain);
+      op->kplain = nullptr;
+      op->kplain_cap = 0;
+      const hipError_t e = dev_malloc((void **)&op->kplain, sizeof(float2) * M);
+      if (e != hipSuccess && !batched(op))
+        for (auto &q : op->frames) q.has_traj = false;  // they share it
+      MRN_HIP(op, e);
+      op->kplain_cap = M;
+    }
+    if (batched(op)) MRN_TRY(bind_frame(op, fr, st));
+    fr.has_traj = true;
+    MRN_HIP(op, hipStreamSynchronize(st));
+    return MRN_OK;
+  });
 }
 
 int mrn_set_smaps(mrn_op *op, const void *smaps, void *stream) {
@@ -616,19 +669,21 @@ int mrn_set_kdata(mrn_op *op, int f, const void *data, void *stream) {
   hipStream_t st = pick(op, stream);
   FrameData &fr = op->frames[f];
   MRN_HIP(op, hipDeviceSynchronize());  // arrays reused in place: no launch may still read them
-  MRN_HIP(op, grow(fr.kraw, fr.cap.kraw, (int64_t)op->C * fr.M));
-  MRN_HIP(op, hipMemcpyAsync(fr.kraw, data, sizeof(float2) * op->C * fr.M, hipMemcpyDeviceToDevice, st));
-  if (batched(op)) {
-    const int64_t need = fr.Mv * op->g.CC * op->nch;
-    MRN_HIP(op, grow(fr.kdata, fr.cap.kdata, need));
-    MRN_TRY(op_permute_in(op, fr.kdata, fr.kraw, fr, st));
-  }
-  fr.kraw_M = fr.M;
-  fr.has_kdata = true;
+  fr.has_kdata = false;
   op->version++;
   op->cg_ready = false;
-  MRN_HIP(op, hipStreamSynchronize(st));
-  return MRN_OK;
+  return with_room(op, st, [&]() -> int {
+    MRN_HIP(op, grow(fr.kraw, fr.cap.kraw, (int64_t)op->C * fr.M));
+    MRN_HIP(op, hipMemcpyAsync(fr.kraw, data, sizeof(float2) * op->C * fr.M, hipMemcpyDeviceToDevice, st));
+    if (batched(op)) {
+      MRN_HIP(op, grow(fr.kdata, fr.cap.kdata, fr.Mv * op->g.CC * op->nch));
+      MRN_TRY(op_permute_in(op, fr.kdata, fr.kraw, fr, st));
+    }
+    fr.kraw_M = fr.M;
+    fr.has_kdata = true;
+    MRN_HIP(op, hipStreamSynchronize(st));
+    return MRN_OK;
+  });
 }
 
 int mrn_image_to_kspace(mrn_op *op, int f, const void *X, void *data, const void *sub, void *stream) {
@@ -738,8 +793,8 @@ static int cg_step(mrn_op *op, float2 *X, bool with_trace, hipStream_t s) {
 int mrn_cg_init(mrn_op *op, void *Xv, void *stream) {
   if (!op || !Xv) return MRN_EINVAL;
   for (int f = 0; f < op->F; f++) MRN_TRY(check_frame(op, f, true));
-  MRN_TRY(ensure_solver(op));
   hipStream_t st = pick(op, stream);
+  MRN_TRY(with_room(op, st, [&]() { return ensure_solver(op); }));
   MRN_TRY(fused_prepare(op, st));
   const int64_t n = (int64_t)op->F * op->nvox;
   MRN_HIP(op, hipMemsetAsync(op->dcounter, 0, sizeof(int), st));
@@ -799,8 +854,8 @@ int mrn_cg(mrn_op *op, void *Xv, int iters, int use_graph, double *trace, void *
 int mrn_power_method(mrn_op *op, int iters, double *step, void *stream) {
   if (!op || iters <= 0) return MRN_EINVAL;
   for (int f = 0; f < op->F; f++) MRN_TRY(check_frame(op, f, false));
-  MRN_TRY(ensure_solver(op));
   hipStream_t st = pick(op, stream);
+  MRN_TRY(with_room(op, st, [&]() { return ensure_solver(op); }));
   const int64_t n = (int64_t)op->F * op->nvox;
   MRN_HIP(op, hipMemsetAsync(op->dcounter, 0, sizeof(int), st));
   MRN_TRY(fused_prepare(op, st));
@@ -819,19 +874,23 @@ int mrn_power_method(mrn_op *op, int iters, double *step, void *stream) {
 int mrn_fista(mrn_op *op, void *Xv, int iters, double step, int use_graph, double *resid, void *stream) {
   if (!op || !Xv || iters < 0) return MRN_EINVAL;
   for (int f = 0; f < op->F; f++) MRN_TRY(check_frame(op, f, true));
-  MRN_TRY(ensure_solver(op));
   hipStream_t st = pick(op, stream);
+  const bool l1 = op->l1_fraction > 0.0f;
+  const bool cauchy = op->step_type == MRN_STEP_CAUCHY;
+  // everything the iterations use is there before any capture
+  MRN_TRY(with_room(op, st, [&]() -> int {
+    MRN_TRY(ensure_solver(op));
+    if (l1) MRN_TRY(ensure_l1_state(op));
+    return llr_fista_prepare(op);
+  }));
+  MRN_TRY(fused_prepare(op, st));
+  if (l1) l1_fista_prepare(op);  // last: it can do without
   float2 *X = (float2 *)Xv;
   const int64_t n = (int64_t)op->F * op->nvox;
   MRN_HIP(op, hipMemsetAsync(op->dcounter, 0, sizeof(int), st));
   MRN_TRY(op_zero(op, X, n, st));
   MRN_TRY(op_zero(op, op->vP, n, st));  // X_old
   const float stf = (float)step;
-  const bool l1 = op->l1_fraction > 0.0f;
-  const bool cauchy = op->step_type == MRN_STEP_CAUCHY;
-  if (l1) MRN_TRY(l1_fista_prepare(op));  // before any capture
-  MRN_TRY(llr_fista_prepare(op));
-  MRN_TRY(fused_prepare(op, st));
   if (cauchy) MRN_TRY(op_set_step(op, stf, 0.0f, st));  // the step until the first Cauchy update
   auto body = [&](hipStream_t s) -> int {
     MRN_TRY(op_fista_momentum(op, X, op->vP, n, s));
@@ -933,9 +992,10 @@ int mrn_autotune(mrn_op *op, int f, const char *cache_path, void *stream) {
   if (!op) return MRN_EINVAL;
   MRN_TRY(check_frame(op, f, false));
   if (!batched(op)) return MRN_OK;
-  MRN_TRY(ensure_solver(op));
+  hipStream_t st = pick(op, stream);
+  MRN_TRY(with_room(op, st, [&]() { return ensure_solver(op); }));
   op->version++;
-  return autotune_impl(op, f, cache_path, pick(op, stream));
+  return autotune_impl(op, f, cache_path, st);
 }
 
 int mrn_get_tuning(const mrn_op *op, mrn_tuning *out) {
@@ -965,7 +1025,7 @@ int mrn_stage_times(mrn_op *op, int f, const void *Xv, int reps, float ms[MRN_NS
   hipStream_t st = pick(op, stream);
   FrameData &fr = op->frames[f];
   const float2 *X = (const float2 *)Xv;
-  MRN_TRY(ensure_solver(op));
+  MRN_TRY(with_room(op, st, [&]() { return ensure_solver(op); }));
   Events ev;
   MRN_HIP(op, ev.create(MRN_NSTAGES + 1));
   double acc[MRN_NSTAGES] = {0};
@@ -1060,6 +1120,7 @@ int mrn_get_support(mrn_op *op, int f, int32_t *xrng, int32_t *yrng) {
 int mrn_get_grid(mrn_op *op, void **grid, int64_t dims[5]) {
   if (!op || !grid || !dims) return MRN_EINVAL;
   const bool b = batched(op);
+  if (b) MRN_TRY(ensure_grid(op));
   *grid = b ? (void *)op->grid : (void *)op->cgrid;
   op->grid_exposed = true;  // the caller may write it: no grid is reused from now on
   dims[0] = b ? op->nch : 1;
@@ -1070,6 +1131,7 @@ int mrn_get_grid(mrn_op *op, void **grid, int64_t dims[5]) {
 
 int mrn_grid_zero(mrn_op *op, void *stream) {
   if (!op) return MRN_EINVAL;
+  if (batched(op)) MRN_TRY(ensure_grid(op));
   const int64_t n = batched(op) ? ncell(op) * op->g.CC * op->nch : ncell(op);
   return op_zero(op, batched(op) ? op->grid : op->cgrid, n, pick(op, stream));
 }

@@ -2387,6 +2387,10 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
     hipError_t e_ = (call);                                                                  \
     if (e_ != hipSuccess) {                                                                  \
       fr.has_traj = false;                                                                   \
+      if (e_ == hipErrorOutOfMemory) {                                                       \
+        op->oom = true;                                                                      \
+        (void)hipGetLastError();                                                             \
+      }                                                                                      \
       return fail(op, e_ == hipErrorOutOfMemory ? MRN_ENOMEM : MRN_EHIP, hipGetErrorString(e_)); \
     }                                                                                        \
   } while (0)

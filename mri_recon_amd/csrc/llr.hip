@@ -792,7 +792,8 @@ int llr_fista_prepare(mrn_op *op) {
   if (op->llr_nblk < nblk) {
     hipFree(op->llr_sblocks);
     op->llr_sblocks = nullptr;
-    MRN_HIP(op, hipMalloc(&op->llr_sblocks, sizeof(double) * (nblk > 0 ? nblk : 1)));
+    op->llr_nblk = 0;
+    MRN_HIP(op, dev_malloc((void **)&op->llr_sblocks, sizeof(double) * (nblk > 0 ? nblk : 1)));
     op->llr_nblk = nblk;
   }
   if (!op->llr_sel) MRN_HIP(op, hipMalloc(&op->llr_sel, sizeof(SelState)));

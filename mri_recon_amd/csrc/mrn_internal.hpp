@@ -232,6 +232,7 @@ struct mrn_op {
   int64_t cg_count = 0;
   int64_t nvox = 0;
   std::string err;
+  bool oom = false;            // an allocation of the running call failed (with_room)
   void *scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;
   // L1 wavelet proximal step of FISTA (fraction 0 = none)
@@ -271,6 +272,10 @@ int fail(mrn_op *op, int code, const char *msg);
   do {                                                                             \
     hipError_t e_ = (call);                                                        \
     if (e_ != hipSuccess) {                                                        \
+      if (e_ == hipErrorOutOfMemory) {                                             \
+        (op)->oom = true;                                                          \
+        (void)hipGetLastError();                                                   \
+      }                                                                            \
       return mrn::fail(op, MRN_EHIP, (std::string(#call) + ": " + hipGetErrorString(e_)).c_str()); \
     }                                                                              \
   } while (0)
@@ -536,6 +541,10 @@ struct PrePostArgs {
 // when that is an integer (a sample exactly on the window edge has one more),
 // floor(2 dwin) + 1 otherwise
 int taps_main(const Geom &g);
+int ensure_grid(mrn_op *op);
+bool can_unpad(const mrn_op *op);
+int unpad_blocks(mrn_op *op, hipStream_t st);
+int op_smaps_reblock(mrn_op *, float2 *, const float2 *, int, hipStream_t);
 
 // host-side launchers (defined in the .hip files)
 int gather_coils(const mrn_op *op, int64_t n);
@@ -571,6 +580,6 @@ int l1_wavelet_host(mrn_op *op, float2 *X, int frames, float fraction, const int
                     const int32_t *shifts, double *thr, hipStream_t st);
 int l1_fista_step(mrn_op *op, float2 *X, hipStream_t st);
 int ensure_l1_state(mrn_op *op);
-int l1_fista_prepare(mrn_op *op);
+void l1_fista_prepare(mrn_op *op);
 
 }  // namespace mrn

@@ -56,6 +56,16 @@ __global__ void k_smaps_in(float2 *dst, const float2 *src, int64_t nvox, int Nx,
   }
 }
 
+// coil maps in blocks of `from` coils -> in blocks of CC (rows: the voxels, in any order)
+__global__ void k_smaps_reblock(float2 *dst, const float2 *src, int64_t nvox, int C, int from, int CC, int64_t total) {
+  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
+       idx += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t v = idx / CC % nvox;
+    const int c = (int)(idx / (CC * nvox)) * CC + (int)(idx % CC);
+    dst[idx] = c < C ? src[((c / from) * nvox + v) * from + c % from] : make_float2(0.f, 0.f);
+  }
+}
+
 // caller k-space [C][M] -> internal [nch][Mv][CC] in tile order
 __global__ void k_permute_in(float2 *kint, const float2 *data, const int32_t *perm, int64_t M,
                              int64_t Mv, int C, int CC, int lgCC, int64_t total) {
@@ -484,6 +494,13 @@ int op_smaps_in(mrn_op *op, float2 *dst, const float2 *src, hipStream_t st) {
   const int64_t total = (int64_t)op->nch * op->nvox * op->g.CC;
   hipLaunchKernelGGL(k_smaps_in, dim3(gs(total)), dim3(256), 0, st, dst, src, op->nvox, op->g.N[0],
                      op->g.N[1], op->g.N[2], op->C, op->g.CC, op->g.lgCC, total);
+  LAUNCH_CHECK(op);
+  return MRN_OK;
+}
+int op_smaps_reblock(mrn_op *op, float2 *dst, const float2 *src, int from, hipStream_t st) {
+  const int64_t total = (int64_t)op->nch * op->nvox * op->g.CC;
+  hipLaunchKernelGGL(k_smaps_reblock, dim3(gs(total)), dim3(256), 0, st, dst, src, op->nvox, op->C, from, op->g.CC,
+                     total);
   LAUNCH_CHECK(op);
   return MRN_OK;
 }

@@ -176,6 +176,73 @@ static int exact_cc(int C) {
   return cc;
 }
 
+// The batched form's grid where it is missing, zeroed: the forward x pass leaves
+// the cells outside a frame's k-space support as they are, and readers of whole
+// tile regions weight them by zero, so they must hold finite values.
+int ensure_grid(mrn_op *op) {
+  if (op->grid) return MRN_OK;
+  const int64_t n = (int64_t)op->g.S[0] * op->g.S[1] * op->g.S[2] * op->g.CC * op->nch * (op->fuse ? op->F : 1);
+  MRN_HIP(op, dev_malloc((void **)&op->grid, sizeof(float2) * n));
+  const hipError_t e = hipMemset(op->grid, 0, sizeof(float2) * n);
+  if (e != hipSuccess) {
+    hipFree(op->grid);
+    op->grid = nullptr;
+  }
+  MRN_HIP(op, e);
+  return MRN_OK;
+}
+
+// Whether the op's coil blocks are padded and can go back to blocks that divide
+// the coil count (not once the caller holds the grid's address).
+bool can_unpad(const mrn_op *op) {
+  return op->p.form == MRN_FORM_BATCHED && op->p.coil_chunk <= 0 && !op->grid_exposed && op->grid &&
+         exact_cc(op->C) != op->g.CC;
+}
+
+// ... and back they go: the coil maps laid out anew, the grid smaller, the frames'
+// k-space arrays gone and every frame unbound (the caller binds them anew).  If
+// not even the smaller maps can be had the blocks stay as they were.
+int unpad_blocks(mrn_op *op, hipStream_t st) {
+  const int cc = exact_cc(op->C), old = op->g.CC;
+  MRN_HIP(op, hipDeviceSynchronize());
+  op->version++;
+  op->fwd_f = -1;
+  auto drop = [](float2 *&p) {
+    hipFree(p);
+    p = nullptr;
+  };
+  drop(op->grid);
+  drop(op->kwork);
+  drop(op->kwork_all);
+  drop(op->part);
+  drop(op->part_all);
+  drop(op->wave_T);
+  op->kwork_cap = op->kwork_all_cap = 0;
+  op->part_cap = op->part_all_cap = op->wave_T_cap = 0;
+  for (auto &fr : op->frames) {
+    drop(fr.kdata);
+    fr.cap.kdata = 0;
+    fr.has_traj = false;
+  }
+  set_blocks(op, cc);
+  const int64_t per = (int64_t)cc * op->nch;
+  float2 *maps = nullptr;
+  auto run = [&]() -> int {
+    MRN_HIP(op, dev_malloc((void **)&maps, sizeof(float2) * op->nvox * per));
+    MRN_TRY(op_smaps_reblock(op, maps, op->smaps, old, st));
+    MRN_HIP(op, hipStreamSynchronize(st));
+    drop(op->smaps);
+    op->smaps = maps;
+    return ensure_grid(op);
+  };
+  const int rc = run();
+  if (rc != MRN_OK && maps != op->smaps) {
+    hipFree(maps);
+    set_blocks(op, old);
+  }
+  return rc;
+}
+
 }  // namespace mrn
 
 using namespace mrn;
@@ -400,6 +467,7 @@ int mrn_op_create(const mrn_params *pin, mrn_op **out) {
     hipMemcpy(op->tw_d[a], tw.data(), sizeof(float2) * g.S[a], hipMemcpyHostToDevice);
   }
   const int64_t ncell = (int64_t)g.S[0] * g.S[1] * g.S[2];
+  if (amalloc((void **)&op->cgrid, sizeof(float2) * ncell) != hipSuccess) return cleanup_fail(MRN_ENOMEM);
   if (batched) {
     for (;;) {
       // frames fused into one launch per stage keep F grids side by side:
@@ -411,15 +479,9 @@ int mrn_op_create(const mrn_params *pin, mrn_op **out) {
         size_t fm = 0, tm = 0;
         op->fuse = p.fuse_frames > 0 || (hipMemGetInfo(&fm, &tm) == hipSuccess && bytes <= 0.5 * (double)fm);
       }
-      const int64_t ngrid = ncell * g.CC * op->nch * (op->fuse ? op->F : 1);
-      if (amalloc((void **)&op->grid, sizeof(float2) * ngrid) == hipSuccess &&
-          amalloc((void **)&op->smaps, sizeof(float2) * op->nvox * g.CC * op->nch) == hipSuccess) {
-        // zeroed once: the forward x pass leaves the cells outside a frame's
-        // k-space support as they are, and readers of whole tile regions weight
-        // them by zero, so they must hold finite values
-        if (hipMemset(op->grid, 0, sizeof(float2) * ngrid) != hipSuccess) return cleanup_fail(MRN_EHIP);
-        break;
-      }
+      const int rc = ensure_grid(op);
+      if (rc != MRN_OK && !op->oom) return cleanup_fail(rc);
+      if (rc == MRN_OK && dev_malloc((void **)&op->smaps, sizeof(float2) * op->nvox * g.CC * op->nch) == hipSuccess) break;
       // no room for padded coil blocks: those that divide the coil count
       (void)hipGetLastError();
       hipFree(op->grid);
@@ -432,7 +494,6 @@ int mrn_op_create(const mrn_params *pin, mrn_op **out) {
     if (amalloc((void **)&op->smaps, sizeof(float2) * op->nvox * op->C) != hipSuccess)
       return cleanup_fail(MRN_ENOMEM);
   }
-  if (amalloc((void **)&op->cgrid, sizeof(float2) * ncell) != hipSuccess) return cleanup_fail(MRN_ENOMEM);
   if (amalloc((void **)&op->dscal, sizeof(double) * 16) != hipSuccess) return cleanup_fail(MRN_ENOMEM);
   if (amalloc((void **)&op->dpart, sizeof(double) * 3 * 1024) != hipSuccess) return cleanup_fail(MRN_ENOMEM);
   if (amalloc((void **)&op->dcounter, sizeof(int) * 4) != hipSuccess) return cleanup_fail(MRN_ENOMEM);

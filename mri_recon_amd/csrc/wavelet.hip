@@ -679,14 +679,6 @@ int ensure_l1_state(mrn_op *op) {
   return MRN_OK;
 }
 
-// ... and what FISTA's step uses, before any capture
-static void ensure_wave_T(mrn_op *op, int frames);
-int l1_fista_prepare(mrn_op *op) {
-  MRN_TRY(ensure_l1_state(op));
-  ensure_wave_T(op, op->F);
-  return MRN_OK;
-}
-
 static int wave_axis(mrn_op *op, float2 *X, int frames, const int s[3], int axis, const int *sh, bool inv,
                      hipStream_t st) {
   static const D4 f = d4_filters();
@@ -850,6 +842,8 @@ static void ensure_wave_T(mrn_op *op, int frames) {
   if (op->wave_T_cap >= (size_t)n) return;
   if (grow(op->wave_T, op->wave_T_cap, n) != hipSuccess) (void)hipGetLastError();
 }
+
+void l1_fista_prepare(mrn_op *op) { ensure_wave_T(op, op->F); }
 
 // FISTA's step: shifts for the current iteration from the device counter
 int l1_fista_step(mrn_op *op, float2 *X, hipStream_t st) {

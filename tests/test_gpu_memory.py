@@ -35,6 +35,92 @@ def blocks(op):
     return op.grid_raw().shape[-1]
 
 
+def test_create_without_room_for_padding(monkeypatch):
+    limit(monkeypatch, 10)
+    op = GridFFT(N, ncoils=C)
+    limit(monkeypatch, None)
+    t, d = traj(300), crandn((C, 300 * 32), 3)
+    op.set_smaps(maps())
+    op.set_traj(*t)
+    h = op.forward(to_dev(d), accumulate=False).cpu().numpy()
+    assert blocks(op) == 1
+    o = orc.OracleOp(N, overgrid=1.5, precision="f32")
+    assert rel(h, o.kspace_to_image(d, maps().cpu().numpy(), [v.cpu().numpy() for v in t])) <= 1e-5
+
+
+@pytest.mark.parametrize("step", ["traj", "kdata", "solver"])
+def test_padding_given_back_later(monkeypatch, step):
+    """The k-space arrays do not fit beside padded blocks: the op goes back to
+    blocks that divide the coil count, keeping its maps, trajectories and data,
+    and the results of blocks of one coil.  The solver's images cannot be had
+    with either: an error, and the blocks stay."""
+    t0, t1 = traj(200), traj(5200)  # 5200 spokes: 166400 samples, 12.0 MB of 9 coils, 21.3 of 16
+    d0, d1 = (to_dev(crandn((C, t[0].numel()), 7)) for t in (t0, t1))
+    out = []
+    for cc in (0, 1):
+        op = GridFFT(N, ncoils=C, nframes=2, fuse_frames=0, coil_chunk=cc)
+        op.set_smaps(maps())
+        op.set_traj(*t0, frame=0)
+        op.set_kdata(d0, frame=0)
+        if cc == 0 and step == "traj":
+            limit(monkeypatch, 16)
+        op.set_traj(*t1, frame=1)
+        if cc == 0 and step == "kdata":
+            limit(monkeypatch, 16)
+        op.set_kdata(d1, frame=1)
+        if cc == 0 and step == "solver":
+            limit(monkeypatch, 0.1)
+            with pytest.raises(MrnError):
+                op.cg(1)
+            limit(monkeypatch, None)
+            for f, (t, d) in enumerate(((t0, d0), (t1, d1))):
+                op.set_traj(*t, frame=f)
+                op.set_kdata(d, frame=f)
+        limit(monkeypatch, None)
+        out.append(op.cg(3, trace=False)[0].cpu().numpy())
+        out.append(op.backward(to_dev(crandn((N, N, N), 9)), frame=1).cpu().numpy())
+        assert blocks(op) == (16 if cc == 0 and step == "solver" else 1)
+        op.close()
+    assert rel(out[0], out[2]) <= 1e-5
+    assert rel(out[1], out[3]) <= 1e-6
+    assert step == "solver" or np.array_equal(out[1], out[3])
+
+
+def test_no_room_at_all_is_an_error_and_recovers(monkeypatch):
+    """A trajectory that fits in no form: an error, the frame unbound (an error,
+    not a launch on missing arrays), another frame still there, and the next
+    trajectory welcome."""
+    t0, t1 = traj(200), traj(5200)
+    op = GridFFT(N, ncoils=C, nframes=2, fuse_frames=0)
+    op.set_smaps(maps())
+    op.set_traj(*t0, frame=0)
+    x = to_dev(crandn((N, N, N), 9))
+    want = op.normal(x, frame=0).cpu().numpy()
+    limit(monkeypatch, 9)  # the exact grid fits, 12 MB of k-space do not
+    with pytest.raises(MrnError):
+        op.set_traj(*t1, frame=1)
+    limit(monkeypatch, None)
+    with pytest.raises(MrnError):
+        op.normal(x, frame=1)
+    got = op.normal(x, frame=0).cpu().numpy()
+    assert rel(got, want) <= 1e-5
+    op.set_traj(*t1, frame=1)
+    op.normal(x, frame=1)
+    op.set_traj(*t0, frame=1)
+    assert rel(op.normal(x, frame=1).cpu().numpy(), want) <= 1e-5
+
+
+def test_explicit_blocks_are_kept(monkeypatch):
+    op = GridFFT(N, ncoils=C, coil_chunk=16)
+    op.set_smaps(maps())
+    limit(monkeypatch, 16)
+    with pytest.raises(MrnError):
+        op.set_traj(*traj(5200))
+    limit(monkeypatch, None)
+    op.set_traj(*traj(5200))
+    assert blocks(op) == 16
+
+
 @pytest.mark.parametrize("graph", [True, False])
 def test_frames_one_by_one_without_room_together(monkeypatch, graph):
     """Four frames' k-space arrays do not fit in one piece: the solver takes
@@ -53,3 +139,24 @@ def test_frames_one_by_one_without_room_together(monkeypatch, graph):
         out.append(op.cg(2, graph=graph, trace=False)[0].cpu().numpy())  # together again
         op.close()
     assert rel(out[2], out[0]) <= 1e-6 and rel(out[3], out[1]) <= 1e-6
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_wavelet_step_without_its_second_image(monkeypatch, graph):
+    """The second image comes after everything the iterations cannot do
+    without: where only that does not fit (64^3: 2.4 MB, the solver's images
+    2.1), FISTA runs in place, with the same bits."""
+    n = 64
+    t = [v.cuda() for v in synth.radial_traj(200, 32, n)]
+    out = []
+    for mb in (None, 2.2):
+        op = GridFFT(n, ncoils=1)
+        op.set_smaps(synth.coil_maps(1, n, seed=5).cuda())
+        op.set_traj(*t)
+        op.set_kdata(to_dev(crandn((1, t[0].numel()), 7)))
+        op.set_fista_l1(0.5, levels=(3, 3, 3), spins=2, seed=3)
+        limit(monkeypatch, mb)
+        out.append(op.fista(2, 1e-3, graph=graph)[0].cpu().numpy())
+        limit(monkeypatch, None)
+        op.close()
+    assert np.array_equal(out[0], out[1])
