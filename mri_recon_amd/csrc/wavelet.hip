@@ -636,16 +636,18 @@ __global__ __launch_bounds__(THR_THREADS) void k_thr_count(const V *__restrict__
   thr_next(s, s_b);
 }
 
-// soft threshold of the sub-block [0, s0) x [0, s1) x [0, s2) of each frame (blockIdx.y)
+// soft threshold of the sub-block [0, s0) x [0, s1) x [0, s2) of each frame
 __global__ __launch_bounds__(256) void k_soft(float2 *X, int N0, int N1, int s0, int s1, int s2, int64_t frame_stride,
-                                              const ThrState *__restrict__ s) {
+                                              int frames, const ThrState *__restrict__ s) {
   const float thr = s->thr;
-  float2 *Xf = X + (int64_t)blockIdx.y * frame_stride;
   const int64_t n = (int64_t)s0 * s1 * s2;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t yz = i / s0;
-    float2 *v = Xf + ((yz / s1) * N1 + yz % s1) * N0 + i % s0;
-    *v = soft(*v, thr);
+  for (int fr = blockIdx.y; fr < frames; fr += gridDim.y) {  // (a grid holds 65535 of them)
+    float2 *Xf = X + (int64_t)fr * frame_stride;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+      const int64_t yz = i / s0;
+      float2 *v = Xf + ((yz / s1) * N1 + yz % s1) * N0 + i % s0;
+      *v = soft(*v, thr);
+    }
   }
 }
 
@@ -825,8 +827,8 @@ int l1_wavelet_step(mrn_op *op, float2 *X, int frames, float fraction, const int
     if (q == 0)  // with the second image X is free until the synthesis
       MRN_TRY(fraction_threshold(op, T, two ? (float *)X : nullptr, n, fraction, 1.0f / (float)spins, log_counter, st));
     if (rest) {
-      hipLaunchKernelGGL(k_soft, dim3(grid_for((n / frames) >> (3 * s)), frames), dim3(256), 0, st, T, N[0], N[1],
-                         N[0] >> s, N[1] >> s, N[2] >> s, op->nvox, (const ThrState *)op->dthr);
+      hipLaunchKernelGGL(k_soft, dim3(grid_for((n / frames) >> (3 * s)), std::min(frames, 65535)), dim3(256), 0, st, T,
+                         N[0], N[1], N[0] >> s, N[1] >> s, N[2] >> s, op->nvox, frames, (const ThrState *)op->dthr);
       MRN_HIP(op, hipGetLastError());
       MRN_TRY(wavelet3d(op, T, frames, levels, sh, true, st, s));
     }

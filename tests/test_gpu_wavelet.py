@@ -186,3 +186,17 @@ def test_threshold_counts_all_values(levels, fraction, scale, bad):
         op.wavelet(W, levels, sh[0], inverse=True)
         got, want = X.cpu().numpy().astype(np.complex128), W.cpu().numpy().astype(np.complex128)
         assert rel(got, want) <= 1e-6
+
+
+@pytest.mark.gpu
+def test_l1_step_without_levels_on_many_frames():
+    """Odd axes have no level: the step is the threshold alone, of more frames
+    than a launch grid has rows."""
+    F = 66000
+    op = _op(F=1, N_=(3, 5, 3))
+    x = crandn((F, 3, 5, 3), 5)
+    X = to_dev(x)
+    thr = np.float32(op.l1_wavelet(X, 0.5, (2, 2, 2), shifts=((0, 1, 2),)))
+    a = np.sqrt(x.real.astype(np.float64) ** 2 + x.imag.astype(np.float64) ** 2).astype(np.float32)
+    assert abs(np.count_nonzero(a < thr) / a.size - 0.5) <= 2e-3
+    assert rel(X.cpu().numpy(), np.where(a <= thr, 0, x * (np.float32(1) - thr / a))) <= 1e-6
