@@ -805,6 +805,14 @@ static int wave3_level(mrn_op *op, float2 *X, float2 *T, int frames, int l, int 
   return MRN_OK;
 }
 
+// Whether the step has a use for the second image: a level on every axis, and a
+// launch grid that holds the frames.
+static bool wave_two(const mrn_op *op, int frames, const int levels[3]) {
+  int L[3];
+  wavelet_levels(op->g.N, levels, L);
+  return wave_common(L) > 0 && wave_blocks(op->g.N[2], W3_IZ) * (int64_t)frames <= 65535;
+}
+
 // The L1 step over `frames` images; shifts of spin q at dsh[3q..3q+2].  With a
 // level on every axis and the second image (op->wave_T) the coefficients live
 // there; otherwise everything runs in place.
@@ -815,8 +823,7 @@ int l1_wavelet_step(mrn_op *op, float2 *X, int frames, float fraction, const int
   int L[3];
   wavelet_levels(N, levels, L);
   const int nf = wave_common(L), maxl = std::max(L[0], std::max(L[1], L[2]));
-  const bool two = nf > 0 && op->wave_T && op->wave_T_cap >= (size_t)wave_T_size(op, frames) &&
-                   wave_blocks(N[2], W3_IZ) * (int64_t)frames <= 65535;
+  const bool two = wave_two(op, frames, levels) && op->wave_T && op->wave_T_cap >= (size_t)wave_T_size(op, frames);
   float2 *T = two ? op->wave_T : X;
   const int s = two ? nf : 0;  // levels from here on in place, in T's (or X's) corner
   const bool rest = !two || maxl > nf;
@@ -839,13 +846,13 @@ int l1_wavelet_step(mrn_op *op, float2 *X, int frames, float fraction, const int
 
 // The second image of l1_wavelet_step (grow-only; without the memory the step
 // runs in place).  Never called while capturing with a larger `frames`.
-static void ensure_wave_T(mrn_op *op, int frames) {
+static void ensure_wave_T(mrn_op *op, int frames, const int levels[3]) {
   const int64_t n = wave_T_size(op, frames);
-  if (op->wave_T_cap >= (size_t)n) return;
+  if (op->wave_T_cap >= (size_t)n || !wave_two(op, frames, levels)) return;
   if (grow(op->wave_T, op->wave_T_cap, n) != hipSuccess) (void)hipGetLastError();
 }
 
-void l1_fista_prepare(mrn_op *op) { ensure_wave_T(op, op->F); }
+void l1_fista_prepare(mrn_op *op) { ensure_wave_T(op, op->F, op->l1_levels); }
 
 // FISTA's step: shifts for the current iteration from the device counter
 int l1_fista_step(mrn_op *op, float2 *X, hipStream_t st) {
@@ -860,7 +867,7 @@ int l1_fista_step(mrn_op *op, float2 *X, hipStream_t st) {
 int l1_wavelet_host(mrn_op *op, float2 *X, int frames, float fraction, const int levels[3], int spins,
                     const int32_t *shifts, double *thr, hipStream_t st) {
   MRN_TRY(ensure_l1_state(op));
-  ensure_wave_T(op, frames);
+  ensure_wave_T(op, frames, levels);
   if (shifts) {
     MRN_HIP(op, hipMemcpyAsync(op->dsh, shifts, sizeof(int) * 3 * spins, hipMemcpyHostToDevice, st));
   } else {

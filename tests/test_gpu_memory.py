@@ -160,3 +160,14 @@ def test_wavelet_step_without_its_second_image(monkeypatch, graph):
         limit(monkeypatch, None)
         op.close()
     assert np.array_equal(out[0], out[1])
+
+
+def test_wavelet_step_takes_no_image_it_does_not_use():
+    """Without a level on every axis the step runs in place: no second image of
+    153 MB is kept."""
+    op = GridFFT((255, 256, 256), ncoils=1, overgrid=1.0, form="plain")
+    x = torch.zeros((1, 256, 256, 255), dtype=torch.complex64, device="cuda")
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    op.l1_wavelet(x, 0.5, levels=(2, 2, 2), spins=1)
+    assert free - torch.cuda.mem_get_info()[0] < 50e6
