@@ -2,9 +2,10 @@
 // reference, whose gridding has no launch shapes).
 //
 // Timed on the frame's own trajectory, one stage at a time, in this order:
-//   1. scatter: sample bin edge B in {1, 2} x samples per work item
-//      {1024, 4096, 16384} (the bins are rebuilt for each), and for 8- and
-//      16-coil blocks the matrix-core or vector-ALU accumulate of the 4^3 tiles;
+//   1. scatter: sample bin edge B in {1, 2} x samples per work item {each
+//      frame's own, 1024, 4096, 16384} (the bins are rebuilt for each), and for
+//      8- and 16-coil blocks the matrix-core or vector-ALU accumulate of the 4^3
+//      tiles;
 //   2. gather: coils per lane {1, 2, 4, 8} (<= coils per block) x XCD run
 //      length {16, 64, 256} workgroups;
 //   3. FFT: XCD run length of the y and z passes {1, 4, 8, 16};
@@ -14,10 +15,10 @@
 // Every candidate computes the same operator: the gather and FFT run
 // candidates give the same bits, the others differ by FP32 summation order.
 //
-// The choice is cached in a JSON file keyed by the geometry, kernel, sample
-// count, coil count and device; a cache hit applies it without timing.  On
-// any failure the op's settings are restored and every frame is rebuilt for
-// them, so the op stays usable.
+// The choice is cached in a JSON file keyed by the tuner's revision, the
+// geometry, kernel, sample count, coil count and device; a cache hit applies it
+// without timing.  On any failure the op's settings are restored and every frame
+// is rebuilt for them, so the op stays usable.
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -87,6 +88,10 @@ int fail_after() {
 }
 
 // ---------------------------------------------------------------- cache
+// Raised whenever the candidates or the kernels they time change: what was chosen
+// among others is not the choice any more (4096 visits per item, the default of
+// revision 1, fix what is now sized per frame: 338 against 170 us at 128^3 x 8).
+#define TUNE_REVISION 2
 std::string cache_key(const mrn_op *op, const FrameData &fr) {
   int dev = 0;
   hipDeviceProp_t prop;
@@ -100,8 +105,8 @@ std::string cache_key(const mrn_op *op, const FrameData &fr) {
     if (c == '"' || c == '\\' || c == ':') c = '_';
   char buf[512];
   snprintf(buf, sizeof buf,
-           "N=%dx%dx%d S=%dx%dx%d W=%.4gx%.4gx%.4g kernel=%d kmode=%d M=%lld C=%d CC=%d device=%s/%dcu",
-           op->g.N[0], op->g.N[1], op->g.N[2], op->g.S[0], op->g.S[1], op->g.S[2], 2 * op->g.dwin[0],
+           "rev=%d N=%dx%dx%d S=%dx%dx%d W=%.4gx%.4gx%.4g kernel=%d kmode=%d M=%lld C=%d CC=%d device=%s/%dcu",
+           TUNE_REVISION, op->g.N[0], op->g.N[1], op->g.N[2], op->g.S[0], op->g.S[1], op->g.S[2], 2 * op->g.dwin[0],
            2 * op->g.dwin[1], 2 * op->g.dwin[2], op->p.kernel, op->g.kmode, (long long)fr.M, op->C, op->g.CC,
            dname.c_str(), cus);
   return buf;

@@ -89,6 +89,25 @@ def test_autotune_cache_hit_skips_timing(problem, tmp_path):
     op3.close()
 
 
+def test_autotune_ignores_choices_of_another_revision(problem, tmp_path):
+    """An entry written for other kernels -- here one that fixes 4096 visits per
+    item, under the key without a revision and under another one -- is not the
+    choice among these."""
+    cache = str(tmp_path / "tune.json")
+    op = _op(problem)
+    op.autotune(cache=cache)
+    (key, val), = json.load(open(cache)).items()
+    rev = key.split()[0]
+    assert rev.startswith("rev=")
+    old = dict(val, max_visits=4096)
+    with open(cache, "w") as f:
+        json.dump({key[len(rev) + 1:]: old, key.replace(rev, "rev=0"): old}, f)
+    assert op.autotune(cache=cache)["from_cache"] == 0
+    assert op.autotune(cache=cache)["from_cache"] == 1
+    assert len(json.load(open(cache))) == 3
+    op.close()
+
+
 def test_autotune_failure_restores_previous_shapes(problem):
     traj, X, smaps, d, A32, H32 = problem
     op = _op(problem, bin_edge=2, max_visits=1024)
