@@ -233,10 +233,11 @@ int mrn_traj_grad(mrn_op *op, int frame, const void *X, const void *g, float *gr
 /* Launch shapes of the batched form (mrn_get_tuning). */
 typedef struct mrn_tuning {
   int32_t bin_edge;       /* sample bin edge in cells */
-  int32_t max_visits;     /* samples per scatter work item */
+  int32_t max_visits;     /* sample visits per scatter work item; 0: each frame's own (mrn_frame_stats) */
   int32_t xcd_run;        /* scatter work items per XCD run */
   int32_t xcd_run_gather; /* gather workgroups per XCD run */
-  int32_t gather_coils;   /* coils per lane in the gather */
+  int32_t gather_coils;   /* coils per lane in the direct gather of the longest frame, or of all
+                             frames where a solver takes them together */
   int32_t xcd_run_fft;    /* y and z FFT pass workgroups per XCD run */
   int32_t fft_stockham;   /* 1: LDS Stockham passes; 0: four-step passes with support pruning */
   int32_t scatter_valu;   /* 1: vector-ALU tile accumulate; 0: matrix cores */
@@ -289,7 +290,8 @@ typedef struct mrn_frame_stats {
   int32_t gather_items;    /* tile-staged gather work items */
   int32_t wide_by_sample;  /* 1: the window-edge taps are added sample by sample, 0: by classes of cells */
   int32_t scatter_groups;  /* wavefronts' groups of scatter work items (= scatter_items: one item each) */
-  int32_t reserved[5];
+  int32_t visits_per_item; /* visits per scatter work item, at most */
+  int32_t reserved[4];
 } mrn_frame_stats;
 int mrn_get_frame_stats(mrn_op *op, int frame, mrn_frame_stats *out);
 

@@ -65,7 +65,8 @@ class MrnFrameStats(ctypes.Structure):
         ("gather_items", ctypes.c_int32),
         ("wide_by_sample", ctypes.c_int32),
         ("scatter_groups", ctypes.c_int32),
-        ("reserved", ctypes.c_int32 * 5),
+        ("visits_per_item", ctypes.c_int32),
+        ("reserved", ctypes.c_int32 * 4),
     ]
 
 

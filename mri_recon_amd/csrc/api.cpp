@@ -1002,12 +1002,12 @@ int mrn_get_tuning(const mrn_op *op, mrn_tuning *out) {
   if (!op || !out) return MRN_EINVAL;
   memset(out, 0, sizeof(*out));
   out->bin_edge = op->t.B;
-  out->max_visits = op->t.maxv;
+  out->max_visits = op->auto_maxv ? 0 : op->t.maxv;
   out->xcd_run = op->t.xrun;
   out->xcd_run_gather = op->t.xrun_gather;
   int64_t Mv = 0;
   for (const auto &fr : op->frames) Mv = std::max(Mv, fr.Mv);
-  out->gather_coils = gather_coils(op, Mv);
+  out->gather_coils = gather_coils(op, op->fuse && op->gather_tiles == 0 ? Mv * op->F : Mv);
   out->xcd_run_fft = op->xcd_run_fft;
   out->fft_stockham = op->fft_stockham ? 1 : 0;
   out->scatter_valu = (op->scatter_valu || (op->g.CC != 16 && op->g.CC != 8)) ? 1 : 0;
@@ -1070,6 +1070,7 @@ int mrn_get_frame_stats(mrn_op *op, int f, mrn_frame_stats *out) {
   out->gather_items = fr.ngsub;
   out->wide_by_sample = fr.wide_each ? 1 : 0;
   out->scatter_groups = fr.ngrp;
+  out->visits_per_item = fr.maxv;
   if (fr.nsub > 0) {
     std::vector<int4> subs((size_t)fr.nsub);
     MRN_HIP(op, hipMemcpy(subs.data(), fr.subs, sizeof(int4) * fr.nsub, hipMemcpyDeviceToHost));

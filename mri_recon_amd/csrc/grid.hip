@@ -2572,6 +2572,7 @@ int build_bins(mrn_op *op, mrn::FrameData &fr, int64_t M, const float *kx, const
   MRN_BH(grow(fr.vlist, cp.vlist, nvisits));
   MRN_BH(grow(fr.subs, cp.subs, nsub_total));
   fr.nsub = nsub_total;
+  fr.maxv = t.maxv;
   hipLaunchKernelGGL(k_fill_subs, dim3(nblk(nt, 256)), dim3(256), 0, st, nsub, off, visits, b.slot0, t,
                      fr.subs, hflag);
   MRN_BH(hipGetLastError());

@@ -139,6 +139,7 @@ struct FrameData {
   int32_t *bin_start = nullptr;// [nbins + 1] first sample of each bin
   int4 *subs = nullptr;        // [nsub] {tile, first visit, end visit, 0 or its partial-sum slot + 1}
   int32_t *gstart = nullptr;   // [ngrp + 1] first work item of each group of equal cost (one wavefront each)
+  int maxv = 0;                // visits per work item, at most
   int ngrp = 0;
   bool groups = false;         // groups of several items, or one item each
   int32_t *xsplit = nullptr;   // [MRN_XCDS + 1] ranges of those groups, one per XCD

@@ -89,6 +89,26 @@ def test_autotune_cache_hit_skips_timing(problem, tmp_path):
     op3.close()
 
 
+def test_tuning_reports_what_runs():
+    """Items sized per frame are reported as such (0, which the parameter
+    accepts), their length with the frame; the gather's coils per lane for the
+    launch they are picked for, over all frames where those go together."""
+    from mri_recon_amd import synth
+    for mv in (0, 256):
+        op = GridFFT(N, ncoils=8, nframes=4, fuse_frames=1, max_visits=mv)
+        for f in range(4):  # 9600 samples: one coil per lane for a frame alone, 2 for four
+            op.set_traj(*[t.cuda() for t in synth.radial_traj(300, 32, N)], frame=f)
+        t = op.tuning()
+        assert t["max_visits"] == mv
+        assert op.frame_stats(0)["visits_per_item"] == (mv or 64)
+        assert t["gather_coils"] == 2
+        op.close()
+    op = GridFFT(N, ncoils=8)
+    op.set_traj(*[t.cuda() for t in synth.radial_traj(300, 32, N)])
+    assert op.tuning()["gather_coils"] == 1
+    op.close()
+
+
 def test_autotune_ignores_choices_of_another_revision(problem, tmp_path):
     """An entry written for other kernels -- here one that fixes 4096 visits per
     item, under the key without a revision and under another one -- is not the
