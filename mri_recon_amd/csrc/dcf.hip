@@ -779,21 +779,35 @@ __global__ void k_dcf_unsort(const uint32_t *__restrict__ perm, const float *__r
 
 int64_t nblocks(int64_t n, int b) { return (n + b - 1) / b; }
 
-// Device memory of one call, freed with it.
+// Device memory of one call, freed with it: arrays wanted together are one
+// allocation (a hipMalloc and hipFree of some MB take 40 us between them).
 struct Scratch {
-  void *p[20];
-  int n = 0;
+  struct Want {
+    void **q;
+    size_t at;
+  };
+  void *p[3];
+  Want w[16];
+  int n = 0, nw = 0;
+  size_t bytes = 0;
   hipStream_t st;
   explicit Scratch(hipStream_t s) : st(s) {}
   Scratch(const Scratch &) = delete;
   template <class T>
-  hipError_t get(T *&q, int64_t count) {
+  void want(T *&q, int64_t count) {
     q = nullptr;
-    if (n == (int)(sizeof(p) / sizeof(p[0]))) return hipErrorInvalidValue;
+    w[nw++] = Want{(void **)&q, bytes};
+    bytes += (sizeof(T) * (size_t)(count > 0 ? count : 1) + 255) & ~(size_t)255;
+  }
+  hipError_t take() {  // the arrays wanted since the last one
     void *v = nullptr;
-    const hipError_t e = dev_malloc(&v, sizeof(T) * (size_t)(count > 0 ? count : 1));
-    if (e == hipSuccess) p[n++] = v;
-    q = (T *)v;
+    const hipError_t e = dev_malloc(&v, bytes);
+    if (e == hipSuccess) {
+      p[n++] = v;
+      for (int i = 0; i < nw; i++) *w[i].q = (uint8_t *)v + w[i].at;
+    }
+    nw = 0;
+    bytes = 0;
     return e;
   }
   ~Scratch() {
@@ -841,10 +855,13 @@ bool dm_iters(int iters, int64_t M) { return iters >= 3 || iters * M >= (1 << 20
 // per iteration, general / one-width: 256^3, random samples 50000 253 / 288 us
 // (206193 items), 200000 507 / 662 (499762), 500000 905 / 896 (621276), 2 M 2850 /
 // 1268; 256^3 radial 200000 446 / 194 (108247); 384^3 random 50000 447 / 319
-// (235967), 500000 1179 / 1807 (1455385), 2 M 3283 / 3096 (2090240).
-bool dm_sparse(const DcfGeom &g, int64_t M, int64_t items) {
+// (235967), 200000 715 / 1016 (793909), 500000 1179 / 1807 (1455385), 2 M 3283 / 3096
+// (2090240).  By now the lists are built and the general form starts from its
+// own sort: the iterations have to save 600 us.
+bool dm_sparse(const DcfGeom &g, int64_t M, int64_t items, int iters) {
   const int64_t cells = (int64_t)g.S[0] * g.S[1] * g.S[2];
-  return items > M * 6 / 7 + cells / 2000 + 50000;
+  const int64_t over = items - (M + cells / 1740 + 60000);  // at 1.2 ns
+  return over * iters > 500000;
 }
 
 // A status that is none of the interface's: the call goes on in the general form.
@@ -871,29 +888,30 @@ int dm_calc(const mrn_dcf_params *p, const DcfGeom &g, const DmGeom &m, int64_t 
   int *nheavy_d;
   double *dsum, *part;
   uint8_t *tmp;
-  DM_MEM(mem.get(tab, g.len));
-  DM_MEM(mem.get(dsum, p->iters));
-  DM_MEM(mem.get(coords, M));
-  DM_MEM(mem.get(keys, 2 * M));
-  DM_MEM(mem.get(perm, 2 * M));
-  DM_MEM(mem.get(start, (int64_t)nbins + 1));
-  DM_MEM(mem.get(items, (int64_t)ntiles + 1));
-  DM_MEM(mem.get(ofs, (int64_t)ntiles + 1));
-  DM_MEM(mem.get(slots, (int64_t)ntiles + 1));
-  DM_MEM(mem.get(slot0, (int64_t)ntiles + 1));
-  DM_MEM(mem.get(nheavy_d, 1));
+  mem.want(tab, g.len);
+  mem.want(dsum, p->iters);
+  mem.want(coords, M);
+  mem.want(keys, 2 * M);
+  mem.want(perm, 2 * M);
+  mem.want(start, (int64_t)nbins + 1);
+  mem.want(items, (int64_t)ntiles + 1);
+  mem.want(ofs, (int64_t)ntiles + 1);
+  mem.want(slots, (int64_t)ntiles + 1);
+  mem.want(slot0, (int64_t)ntiles + 1);
+  mem.want(nheavy_d, 1);
+  int bits = 1;
+  while ((1ll << bits) <= nbins) bits++;  // keys 0 .. nbins
+  size_t tb = 0, sb = 0;
+  DCF_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, keys, keys, perm, perm, (int)M, 0, bits, st));
+  DCF_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, sb, items, ofs, ntiles + 1, st));
+  tb = tb > sb ? tb : sb;
+  mem.want(tmp, (int64_t)tb);
+  DM_MEM(mem.take());
   DCF_HIP(hipMemcpyAsync(tab, tab_h, sizeof(float) * g.len, hipMemcpyHostToDevice, st));
   const size_t lds = sizeof(float) * g.len;
   const dim3 gs((unsigned)nblocks(M, 256));
   hipLaunchKernelGGL(k_dm_keys, gs, dim3(256), 0, st, kx, ky, kz, M, g, m, keys, perm);
   DCF_HIP(hipGetLastError());
-  int bits = 1;
-  while ((1ll << bits) <= nbins) bits++;  // keys 0 .. nbins
-  size_t tb = 0, sb = 0;
-  DCF_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, keys, keys + M, perm, perm + M, (int)M, 0, bits, st));
-  DCF_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, sb, items, ofs, ntiles + 1, st));
-  tb = tb > sb ? tb : sb;
-  DM_MEM(mem.get(tmp, (int64_t)tb));
   DCF_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, keys, keys + M, perm, perm + M, (int)M, 0, bits, st));
   const uint32_t *order = perm + M;
   hipLaunchKernelGGL(k_dm_coords, gs, dim3(256), 0, st, order, kx, ky, kz, M, g, coords);
@@ -907,11 +925,12 @@ int dm_calc(const mrn_dcf_params *p, const DcfGeom &g, const DmGeom &m, int64_t 
   DCF_HIP(hipMemcpyAsync(&nitems, ofs + ntiles, sizeof(int32_t), hipMemcpyDeviceToHost, st));
   DCF_HIP(hipMemcpyAsync(&nslots, slot0 + ntiles, sizeof(int32_t), hipMemcpyDeviceToHost, st));
   DCF_HIP(hipStreamSynchronize(st));
-  if (dm_sparse(g, M, nitems)) return DM_GENERAL;
-  DM_MEM(mem.get(X, (int64_t)g.S[0] * g.S[1] * g.S[2]));
-  DM_MEM(mem.get(list, nitems));
-  DM_MEM(mem.get(heavy, nslots));  // at least two slots per split tile
-  DM_MEM(mem.get(part, (int64_t)nslots * DM_CELLS));
+  if (dm_sparse(g, M, nitems, p->iters)) return DM_GENERAL;
+  mem.want(X, (int64_t)g.S[0] * g.S[1] * g.S[2]);
+  mem.want(list, nitems);
+  mem.want(heavy, nslots);  // at least two slots per split tile
+  mem.want(part, (int64_t)nslots * DM_CELLS);
+  DM_MEM(mem.take());
   hipLaunchKernelGGL(k_dm_items, dim3((unsigned)nblocks(ntiles, 256)), dim3(256), 0, st, items, ofs, slot0, ntiles, list);
   hipLaunchKernelGGL(k_dcf_fill, dim3(1), dim3(1), 0, st, reinterpret_cast<float *>(nheavy_d), (int64_t)1, 0.0f);
   int nheavy = 0;

@@ -181,7 +181,8 @@ def test_dcf_item_lengths_match_oracle(M):
 @pytest.mark.parametrize("N,M,kind,iters,tiles", [
     (24, 5000, "radial", 0, False), (24, 5000, "radial", 2, False), (24, 5000, "radial", 3, True),
     (24, 524288, "radial", 1, False), (24, 524288, "radial", 2, True),   # iters * M at 2^20
-    (256, 200000, "random", 3, False), (256, 200000, "radial", 3, True), (128, 200000, "random", 3, True)])
+    (256, 200000, "random", 5, False), (256, 200000, "random", 3, True), (256, 200000, "radial", 20, True),
+    (128, 200000, "random", 20, True)])
 def test_dcf_form_rule(N, M, kind, iters, tiles):
     """Which calls go by tiles: from 3 iterations or 2^20 sample visits on, and
     not with samples so scattered that the tiles' items are nearly empty.  Both
