@@ -54,7 +54,7 @@ def cpu_fft_setup(o32):
 # device kernel behind each stage of GridFFT.stage_times (as rocprofv3 names it)
 KERNEL_NAMES = {
     "pre_z": "k_fft_pre_z", "fft_y": "k_fft_lines (y)", "fft_x": "k_fft_lines (x)",
-    "gather": "k_gather", "scatter_zero": "k_sum_tiles", "scatter": "k_scatter_mm",
+    "gather": "k_gather", "scatter_zero": "(empty)", "scatter": "k_scatter_mm",
     "ifft_x": "k_fft_lines (x, inverse)", "ifft_y": "k_fft_lines (y, inverse)", "post_z": "k_fft_post_z",
 }
 

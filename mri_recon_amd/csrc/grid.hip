@@ -2330,9 +2330,9 @@ static bool group_items(const mrn_op *op, int64_t Mv, int64_t n, int64_t total) 
 // Cost of a group: the list's total over 4 rounds of the chip's 4096 scatter
 // wavefronts, from two items' fixed part to one whole item of MRN_AUTO_MAXV
 // visits (longer groups only lengthen the launch's tail).  Scatter at a cost of
-// 64 / 256 / 1056 / 2112 / this rule: 32^3 x 4 coils 25 / 43 / 124 / 227 / 25 us;
-// 128^3 x 8 165 / 145 / 178 / 248 / 144; 160^3 x 24 1235 / 935 / 827 / 890 / 845;
-// 256^3 x 32 6454 / 4836 / 3774 / 3715 / 3755.
+// 64 / 256 / 1056 / 2112 / this rule: 128^3 x 8 coils, 262144 samples 165 / 140 /
+// 161 / 215 / 141 us; 160^3 x 24, 768000 1137 / 840 / 746 / 782 / 763; 256^3 x 32,
+// 5.12 M 6299 / 4679 / 3697 / 3680 / 3704.
 static int64_t group_cost(int64_t total) {
   return std::min<int64_t>(std::max<int64_t>(total / (4 * 4096), 64), MRN_AUTO_MAXV + 32);
 }
@@ -2344,10 +2344,10 @@ static int64_t group_cost(int64_t total) {
 // at least 64 (below it the split tiles' partial sums cost more than the shorter
 // walks save) and at most 1024 (more gains nothing at 41 M visits).
 // Scatter at 64 / 256 / 1024 / 4096 visits per item: 32^3 x 8 coils, 8192
-// samples 23 / 33 / 74 / 86 us; 128^3 x 8, 262144 samples 180 / 169 / 179 /
-// 338; 100 x 84 x 92 x 8, 303101 samples 211 / 165 / 186 / 346; 160^3 x 24,
-// 768000 samples 1268 / 1028 / 1007 / 1119; 256^3 x 16, 5.12 M samples
-// 4280 / 2217 / 2036 / 2066.
+// samples 22 / 31 / 73 / 102 us; 128^3 x 8, 262144 samples 164 / 142 / 156 /
+// 333; 100 x 84 x 92 x 8, 303101 samples 139 / 127 / 151 / 324; 160^3 x 24,
+// 768000 samples 892 / 796 / 762 / 938; 256^3 x 16, 5.12 M samples 2128 / 2137 /
+// 1890 / 2059.
 #define MIN_PART (8ll << 20)  // partial sums always allowed: 8 M values, 64 MB
 static int visits_per_item(const Tiles &t, int64_t Mv) {
   const double per = (t.NTb + t.T - 1) / (double)t.T;  // tiles a sample reaches, per axis

@@ -1,9 +1,9 @@
 """Pipe DCF on the GPU (mrn_dcf_calc) against the oracle's restatement of
 RECON::dcf_calc (recon_lib.cpp:854-917) and DCFgridFFT (DCFgridFFT.cpp).
 
-The GPU scatter adds with float atomics, so the order of the additions into a
-grid cell differs from the oracle's sample order: results agree to FP32
-rounding of those sums, carried through the ratio iteration.  Bars: relative
+The GPU's general form adds with float atomics, its tile form along matrix
+products, so the order of the additions into a grid cell differs from the
+oracle's sample order: results agree to FP32 rounding of those sums, carried through the ratio iteration.  Bars: relative
 L2 <= 1e-5 after one iteration, <= 1e-4 after 20 (the default), against the
 FP32 oracle; the FP64 oracle within 1e-4.  The gather, the update, the table
 and scale_kw have no ordering freedom.

@@ -5,7 +5,7 @@ over a per-frame table on the device) against the same op frame by frame
 the power method over frames of uneven sample counts, coil blocks of 4, 8 and
 16 (24 coils: three blocks of 8), k-space support pruning on and off.  The
 per-frame kernels are the same, so the results agree to FP32 summation order
-of the split tiles' atomics (<= 1e-6); the fused FISTA+LLR also matches the
+of the window-edge samples' atomics (<= 1e-6); the fused FISTA+LLR also matches the
 composed oracle loop."""
 import numpy as np
 import pytest

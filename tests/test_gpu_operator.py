@@ -313,7 +313,7 @@ def test_matrix_core_scatter_matches_valu_and_oracle(C, dwin, max_visits):
     """The matrix-core scatter (16-coil blocks) sums the same products as the
     VALU scatter in another order: Aᴴ agrees with it to FP32 rounding and with
     the oracle to the usual bar.  max_visits=64 splits the dense tiles over
-    several work items, whose partial sums are added with atomics."""
+    several work items, whose partial sums are added in order."""
     N = 32
     traj, X, smaps, d = radial_problem(N, C, 900, 40, seed=43)
     out = []

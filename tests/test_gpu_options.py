@@ -190,8 +190,8 @@ def test_xcd_block_order_same_bits():
 def test_xcd_slab_scatter(C, kw):
     """xcd_run = -1: the scatter's work list is cut into 8 contiguous ranges
     of equal cost and workgroup b takes its items from range b % 8.  Every
-    item must run exactly once: A^H as with the hardware order (split tiles'
-    atomics aside, the same bits) and as the oracle, for the matrix-core and
+    item must run exactly once: A^H as with the hardware order (the
+    window-edge samples' atomics aside, the same bits) and as the oracle, for the matrix-core and
     vector-ALU forms, split tiles, accumulation and three fused frames of
     different sizes."""
     N = 32
