@@ -146,11 +146,13 @@ static void make_window(mrn_op *op, int a) {
 }
 
 // Coils per grid cell where the caller gave none.  8- and 16-coil blocks take
-// the four-step FFT passes, the k-space support and the matrix-core scatter;
-// blocks of 1, 2 and 4 take none of them, so that even mostly empty 8-coil
-// blocks are faster: the coils are padded to whole blocks (zero maps), of 16
-// when that pads no more than blocks of 8 would.  3 coils go as 4.  Pair of A
-// and A^H at 160^3, 800000 samples, the largest block that divides C / 8 / 16:
+// the matrix-core scatter, the k-space support and, on edges that have them, the
+// four-step FFT passes; blocks of 1, 2 and 4 take none of them, so that even
+// mostly empty 8-coil blocks are faster, also on edges without the four-step
+// passes (16, 32, 48, 400, 432, 480: 1.1 to 8 times): the coils are padded to
+// whole blocks (zero maps), of 16 when that pads no more than blocks of 8 would.
+// 3 coils go as 4.  Pair of A and A^H at 160^3, 800000 samples, the largest block
+// that divides C / 8 / 16:
 // 3 coils 2.20 ms (4: 1.65) / 1.82 / 3.17; 5: 3.52 / 1.85 / 3.20; 6: 2.86 /
 // 1.87 / 3.20; 12: 4.55 / 3.40 / 3.23; 18: 7.94 / 5.19 / 6.30; 20: 7.49 /
 // 5.23 / 6.30; 28: 10.4 / 6.78 / 6.35.  1, 2 and 4 coils stay as they are:
